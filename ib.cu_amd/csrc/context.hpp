@@ -43,6 +43,7 @@ enum scratch_slot {
     SLOT_FLAGS,
     SLOT_REDUCE,        // reduction partials of the solvers (REDUCE_PARTS + 8 doubles)
     SLOT_RBF_X,         // packed data-site coordinates of an RBF evaluation
+    SLOT_RBF_WORK,      // residues of an RBF evaluation's tiles (rbf_residue.hip)
     SLOT_TILES,         // fixed-point tiles of the tile spread (3 x 12^3 per brick)
     SLOT_TILE_FLAGS,    // per-brick "has markers" flags and the tile scale
     SLOT_BOX_OFF,       // marker offsets of the boxes of a batched spread / interpolation
@@ -77,6 +78,10 @@ struct prof_scope {
 ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* const* ops, const int* N,
                           const double* const* X, double* const* Y, int j0, int j1, bool do_pack,
                           unsigned char** packed);
+
+// The scratch that rbf_eval_range on `ctx` without packing needs, allocated
+// ahead (a call under graph capture cannot allocate).
+ibm_status rbf_reserve(ibm_ctx* ctx, int count, ibm_rbf* const* ops, const int* N, int j0, int j1);
 
 // Membrane force passes (forces.hip) on `stream`.
 ibm_status membrane_table(ibm_ctx* ctx, hipStream_t stream, int ns, const double* geo, const double* w, double* table);

@@ -14,7 +14,9 @@
 // each is packed once into "rows x Kp" tiles (k fastest, zero padded):
 // the operator at creation, X per call.  One launch covers every
 // (cell type, operator) pair.  Precisions:
-//   64  v_mfma_f64_16x16x4 on FP64 operands (the plain path);
+//   64  v_mfma_f64_16x16x4 on FP64 operands (evaluations of fewer than
+//       RES_MIN_N columns); wider ones through residues on the INT8 matrix
+//       cores (rbf_residue.hip);
 //   32  v_mfma_f32_16x16x4 on FP32 operands, FP32 accumulation;
 //   16  split BF16: a = a_hi + a_lo with a_hi = bf16(a), a_lo = bf16(a -
 //       a_hi); a b ~ a_hi b_hi + a_hi b_lo + a_lo b_hi with
@@ -33,6 +35,7 @@
 #include <utility>
 #include <vector>
 #include "context.hpp"
+#include "rbf_residue.hpp"
 
 namespace ibm {
 namespace {
@@ -342,6 +345,8 @@ __global__ __launch_bounds__(256) void geometry_kernel(int ns, int nc, const dou
     }
 }
 
+__global__ void clear_flag_kernel(int* flag) { *flag = 0; }
+
 int mode_of(int precision)
 {
     return precision == 64 ? MODE_F64 : precision == 32 ? MODE_F32 : precision == 16 ? MODE_BF16X3 : -1;
@@ -376,6 +381,8 @@ struct ibm_rbf {
     int mode, M, K, Kp, rows_pad, nops;
     size_t plane_bytes;                  // bytes of one operator plane
     unsigned char* mem;                  // nops x planes(mode) planes
+    unsigned char* res;                  // FP64: nops x res_bytes of residue planes, or null
+    size_t res_bytes;
     const unsigned char* plane(int op, int p) const { return mem + (size_t) (op * planes(mode) + p) * plane_bytes; }
 };
 
@@ -444,6 +451,66 @@ int f64_variant(ibm_ctx* ctx, hipStream_t stream, const gemm_groups& G, int bloc
     return pick;
 }
 
+// Whether N columns of `op` are evaluated through residues (rbf_residue.hip)
+// rather than on the FP64 matrix cores: from RES_MIN_N columns on.  Measured
+// with 65 columns (FP64 / residues, us): 3 operators 8832 x 2210 295 / 236,
+// 2843 x 935 129 / 54, 715 x 503 71 / 28; with 600: 1349 / 651, 241 / 143,
+// 77 / 46.
+constexpr int RES_MIN_N = 65;
+bool by_residues(const ibm_rbf* op, int N) { return op->res && N >= RES_MIN_N; }
+
+// Offset of entry b's packed columns in the evaluation's packed operand and,
+// at b = count, its total; entries with the same columns share a packing
+// (first: the entry that owns it).
+size_t packed_offset(int count, ibm_rbf* const* ops, const int* N, const double* const* X, int b, int* first)
+{
+    size_t at = 0;
+    for (int i = 0; i < count; ++i) {
+        const ibm_rbf& op = *ops[i];
+        const bool res = by_residues(&op, N[i]);
+        int owner = i;
+        for (int j = 0; j < i && owner == i; ++j)
+            if (X[j] == X[i] && N[j] == N[i] && ops[j]->K == op.K && by_residues(ops[j], N[j]) == res) owner = j;
+        if (i == b) {
+            if (first) *first = owner;
+            return owner == i ? at : packed_offset(count, ops, N, X, owner, nullptr);
+        }
+        if (owner != i) continue;
+        at += res ? (res_columns_bytes(N[i], op.K) + 255) / 256 * 256
+                  : (size_t) round_up(std::max(N[i], 1), TILE) * op.Kp * elem_bytes(op.mode) * planes(op.mode);
+    }
+    return at;
+}
+
+// The residue path's products of operators [j0, j1) (operands and outputs
+// unset without X / Y: for sizes only).
+int residue_products(int count, ibm_rbf* const* ops, const int* N, const double* const* X, double* const* Y, int j0,
+                     int j1, unsigned char* packed, res_product* out)
+{
+    int n = 0;
+    for (int b = 0; b < count; ++b) {
+        const ibm_rbf& op = *ops[b];
+        if (N[b] == 0 || !by_residues(&op, N[b])) continue;
+        for (int j = j0; j < std::min(j1, op.nops); ++j)
+            out[n++] = res_product{op.res + (size_t) j * op.res_bytes,
+                                   X ? packed + packed_offset(count, ops, N, X, b, nullptr) : nullptr,
+                                   (const double*) op.plane(j, 0), X ? X[b] : nullptr,
+                                   Y ? Y[b] + (size_t) j * op.M * N[b] : nullptr, op.M, N[b], op.K, op.Kp};
+    }
+    return n;
+}
+
+ibm_status rbf_reserve(ibm_ctx* ctx, int count, ibm_rbf* const* ops, const int* N, int j0, int j1)
+{
+    res_product products[MAX_GROUPS];
+    int groups = 0;
+    for (int b = 0; b < count; ++b) groups += std::max(0, std::min(j1, ops[b]->nops) - j0);
+    if (groups > MAX_GROUPS) return IBM_OK;          // refused by the evaluation itself
+    const int n = residue_products(count, ops, N, nullptr, nullptr, j0, j1, nullptr, products);
+    void* mem;
+    return n ? scratch(ctx, SLOT_RBF_WORK, res_work_bytes(n, products), &mem) : IBM_OK;
+}
+
 ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* const* ops, const int* N,
                           const double* const* X, double* const* Y, int j0, int j1, bool do_pack,
                           unsigned char** packed)
@@ -452,35 +519,42 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
     if (count <= 0 || !ops || !N || !X || !Y) return fail(ctx, IBM_ERR_ARG, "empty or null batch");
     int mode = ops[0] ? ops[0]->mode : -1;
     int groups = 0;
-    size_t xbytes = 0;
     for (int b = 0; b < count; ++b) {
         if (!ops[b] || !X[b] || !Y[b] || N[b] < 0) return fail(ctx, IBM_ERR_ARG, "bad batch entry %d", b);
         if (ops[b]->mode != mode) return fail(ctx, IBM_ERR_ARG, "batch mixes precisions");
         if (ops[b]->device != ctx->device) return fail(ctx, IBM_ERR_ARG, "operator %d lives on another device", b);
         groups += std::max(0, std::min(j1, ops[b]->nops) - j0);
-        xbytes += (size_t) round_up(std::max(N[b], 1), TILE) * ops[b]->Kp * elem_bytes(mode) * planes(mode);
     }
     if (groups > MAX_GROUPS) return fail(ctx, IBM_ERR_SIZE, "at most %d operator blocks per launch", MAX_GROUPS);
     if (do_pack) {
         void* scratch_mem;
-        IBM_TRY(scratch(ctx, SLOT_RBF_X, xbytes, &scratch_mem));
+        IBM_TRY(scratch(ctx, SLOT_RBF_X, packed_offset(count, ops, N, X, count, nullptr), &scratch_mem));
         *packed = (unsigned char*) scratch_mem;
     } else if (!*packed) {
         return fail(ctx, IBM_ERR_ARG, "no packed operand");
     }
-    unsigned char* xp = *packed;
 
     gemm_groups G{};
-    int tiles = 0;
+    int tiles = 0, ncols = 0;
+    res_columns cols[RES_MAX_COLUMNS];
     for (int b = 0; b < count; ++b) {
         const ibm_rbf& op = *ops[b];
-        int cols_pad = round_up(std::max(N[b], 1), TILE);
-        size_t plane = (size_t) cols_pad * op.Kp * elem_bytes(mode);
-        unsigned char* hi = xp;
-        unsigned char* lo = planes(mode) > 1 ? xp + plane : nullptr;
-        xp += plane * planes(mode);
         if (N[b] == 0) continue;
-        if (do_pack) pack(mode, stream, X[b], op.K, N[b], op.K, cols_pad, op.Kp, hi, lo);
+        int owner = b;
+        unsigned char* hi = *packed + packed_offset(count, ops, N, X, b, &owner);
+        if (by_residues(&op, N[b])) {
+            if (do_pack && owner == b) {
+                cols[ncols++] = res_columns{X[b], hi, N[b], op.K};
+                if (ncols == RES_MAX_COLUMNS) {
+                    res_pack_columns(stream, ncols, cols);
+                    ncols = 0;
+                }
+            }
+            continue;
+        }
+        int cols_pad = round_up(N[b], TILE);
+        unsigned char* lo = planes(mode) > 1 ? hi + (size_t) cols_pad * op.Kp * elem_bytes(mode) : nullptr;
+        if (do_pack && owner == b) pack(mode, stream, X[b], op.K, N[b], op.K, cols_pad, op.Kp, hi, lo);
         for (int j = j0; j < std::min(j1, op.nops); ++j) {
             gemm_group& g = G.g[G.count++];
             g.E[0] = op.plane(j, 0);
@@ -496,33 +570,43 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
             tiles += (op.rows_pad / TILE) * g.tiles_n;
         }
     }
+    if (ncols) res_pack_columns(stream, ncols, cols);
     IBM_LAUNCH_CHECK(ctx);
-    if (!tiles) return IBM_OK;
-    // Longest contraction first: each XCD takes its share of the groups in
-    // group order, so the short tiles come last and fill the tail.
-    std::stable_sort(G.g, G.g + G.count, [](const gemm_group& a, const gemm_group& b) { return a.Kp > b.Kp; });
-    tiles = 0;
-    for (int q = 0; q < G.count; ++q) {
-        G.g[q].first_tile = tiles;
-        tiles += (round_up(G.g[q].M, TILE) / TILE) * G.g[q].tiles_n;
-    }
-    G.total_tiles = tiles;
-    // blocks: 8 x the most tiles any XCD takes (its share of every group)
-    int per_xcd = 0;
-    for (int x = 0; x < 8; ++x) {
-        int n = 0;
-        for (int q = 0; q < G.count; ++q) {
-            const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : tiles) - G.g[q].first_tile;
-            n += (x + 1) * tq / 8 - x * tq / 8;
-        }
-        per_xcd = std::max(per_xcd, n);
-    }
-    const int blocks = 8 * per_xcd;
+    res_product products[MAX_GROUPS];
+    const int nres = residue_products(count, ops, N, X, Y, j0, j1, *packed, products);
     double flops = 0;
     for (int b = 0; b < count; ++b)
         flops += 2.0 * ops[b]->M * (double) N[b] * ops[b]->K * std::max(0, std::min(j1, ops[b]->nops) - j0);
-    const int wn = mode == MODE_F64 ? f64_variant(ctx, stream, G, blocks) : 2;
+    void* work = nullptr;
+    if (nres) IBM_TRY(scratch(ctx, SLOT_RBF_WORK, res_work_bytes(nres, products), &work));
+    int blocks = 0;
+    if (tiles) {
+        // Longest contraction first: each XCD takes its share of the groups
+        // in group order, so the short tiles come last and fill the tail.
+        std::stable_sort(G.g, G.g + G.count, [](const gemm_group& a, const gemm_group& b) { return a.Kp > b.Kp; });
+        tiles = 0;
+        for (int q = 0; q < G.count; ++q) {
+            G.g[q].first_tile = tiles;
+            tiles += (round_up(G.g[q].M, TILE) / TILE) * G.g[q].tiles_n;
+        }
+        G.total_tiles = tiles;
+        // blocks: 8 x the most tiles any XCD takes (its share of every group)
+        int per_xcd = 0;
+        for (int x = 0; x < 8; ++x) {
+            int n = 0;
+            for (int q = 0; q < G.count; ++q) {
+                const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : tiles) - G.g[q].first_tile;
+                n += (x + 1) * tq / 8 - x * tq / 8;
+            }
+            per_xcd = std::max(per_xcd, n);
+        }
+        blocks = 8 * per_xcd;
+    }
+    if (!tiles && !nres) return IBM_OK;
+    const int wn = mode == MODE_F64 && tiles ? f64_variant(ctx, stream, G, blocks) : 2;
     prof_scope prof(ctx, "rbf_gemm", flops);
+    if (nres) IBM_TRY(res_products(ctx, stream, nres, products, (unsigned char*) work));
+    if (!tiles) return IBM_OK;
     if (mode == MODE_F64) {
         launch_f64(wn, G, blocks, stream);
     } else if (mode == MODE_F32) {
@@ -563,13 +647,37 @@ ibm_status ibm_rbf_create(ibm_ctx* ctx, int precision, int M, int K, int nops, c
         delete op;
         return fail(ctx, IBM_ERR_HIP, "out of device memory for a %zu-byte operator", bytes);
     }
+    // FP64 operators also keep their residue planes (fifteen bytes per
+    // element beside the eight); without the memory for them, or with
+    // elements they cannot represent, every product runs on the FP64 matrix
+    // cores.
+    int* flag = nullptr;
+    if (mode == MODE_F64 && res_fits(K)) {
+        op->res_bytes = (res_operator_bytes(M, K) + 255) / 256 * 256;
+        if (hipMalloc(&op->res, op->res_bytes * nops + sizeof(int)) != hipSuccess) {
+            (void) hipGetLastError();
+            op->res = nullptr;
+        } else {
+            flag = (int*) (op->res + op->res_bytes * nops);
+            clear_flag_kernel<<<1, 1, 0, ctx->stream>>>(flag);
+            for (int j = 0; j < nops; ++j) res_pack_operator(ctx->stream, E[j], lde, M, K, op->res + op->res_bytes * j, flag);
+        }
+    }
     for (int j = 0; j < nops; ++j)
         pack(mode, ctx->stream, E[j], lde, M, K, op->rows_pad, op->Kp, (unsigned char*) op->plane(j, 0),
              planes(mode) > 1 ? (unsigned char*) op->plane(j, 1) : nullptr);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess) {
+    int unfit = 0;
+    if (hipGetLastError() != hipSuccess ||
+        (flag && hipMemcpyAsync(&unfit, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess) ||
+        hipStreamSynchronize(ctx->stream) != hipSuccess) {
         hipFree(op->mem);
+        hipFree(op->res);
         delete op;
         return fail(ctx, IBM_ERR_HIP, "operator packing failed");
+    }
+    if (unfit) {
+        hipFree(op->res);
+        op->res = nullptr;
     }
     *out = op;
     return IBM_OK;
@@ -586,6 +694,7 @@ ibm_status ibm_rbf_destroy(ibm_rbf* op)
 {
     if (!op) return IBM_OK;
     hipFree(op->mem);
+    hipFree(op->res);
     delete op;
     return IBM_OK;
 }

@@ -776,6 +776,20 @@ ibm_status ibm_solver_create(ibm_ctx* ctx, const ibm_dimension* domain, int ndim
         }
         s->types.push_back(T);
     }
+    // Fixed-count steps without membrane models evaluate the tangents on the
+    // first auxiliary context, which a captured step cannot allocate for.
+    if (st == IBM_OK) {
+        ibm_rbf* ops[MAX_TYPES];
+        int N[MAX_TYPES], count = 0;
+        bool any_membrane = false;
+        for (auto& T : s->types)
+            if (T.nc) {
+                any_membrane = any_membrane || T.membrane;
+                ops[count] = T.ops;
+                N[count++] = 3 * T.nc;
+            }
+        if (!any_membrane) st = step_status(ctx, s->aux[0], rbf_reserve(s->aux[0], count, ops, N, 1, 8));
+    }
     if (st == IBM_OK && hipStreamSynchronize(ctx->stream) != hipSuccess) st = fail(ctx, IBM_ERR_HIP, "solver setup");
     if (st != IBM_OK) {
         release(s);

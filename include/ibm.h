@@ -389,13 +389,15 @@ ibm_status ibm_rbf_destroy(ibm_rbf* op);
 ibm_status ibm_rbf_eval(ibm_ctx* ctx, int count, ibm_rbf* const* ops, const int* N, const double* const* X,
                         double* const* Y);
 
-/* Kernel variant of the FP64 evaluation (no counterpart in the reference,
- * whose products go to cuBLAS): waves_n = 2 runs four 64 x 64-output waves
- * per 128 x 128 tile, 4 runs eight 64 x 32-output waves (half the
- * registers, twice the waves per SIMD) over two LDS buffers (one barrier
- * per contraction chunk), 0 (the default) times both on the
- * first eager launch of each shape and keeps the faster for the process.
- * Both variants give bitwise the same results.  Process-wide. */
+/* Kernel variant of the FP64 evaluation on the FP64 matrix cores (no
+ * counterpart in the reference, whose products go to cuBLAS): waves_n = 2
+ * runs four 64 x 64-output waves per 128 x 128 tile, 4 runs eight
+ * 64 x 32-output waves (half the registers, twice the waves per SIMD) over
+ * two LDS buffers (one barrier per contraction chunk), 0 (the default) times
+ * both on the first eager launch of each shape and keeps the faster for the
+ * process.  Evaluations of 65 columns or more run on the INT8 matrix cores
+ * instead (as accurate as the FP64 ones: see rbf_residue.hip), whatever the
+ * variant.  Every setting gives bitwise the same results.  Process-wide. */
 ibm_status ibm_rbf_gemm_variant(int waves_n);
 
 /* Operator construction on the device (bases/operators.h:145-190,
