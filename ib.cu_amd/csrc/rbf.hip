@@ -14,9 +14,9 @@
 // each is packed once into "rows x Kp" tiles (k fastest, zero padded):
 // the operator at creation, X per call.  One launch covers every
 // (cell type, operator) pair.  Precisions:
-//   64  v_mfma_f64_16x16x4 on FP64 operands (evaluations of fewer than
-//       RES_MIN_N columns); wider ones through residues on the INT8 matrix
-//       cores (rbf_residue.hip);
+//   64  few columns on v_mfma_f64_16x16x4 (rbf_thin_kernel); more through
+//       residues on the INT8 matrix cores (rbf_residue.hip), or, where an
+//       operator has no residue planes, on FP64 128 x 128 tiles;
 //   32  v_mfma_f32_16x16x4 on FP32 operands, FP32 accumulation;
 //   16  split BF16: a = a_hi + a_lo with a_hi = bf16(a), a_lo = bf16(a -
 //       a_hi); a b ~ a_hi b_hi + a_hi b_lo + a_lo b_hi with
@@ -296,6 +296,100 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
         }
 }
 
+// FP64 products of few columns, in column tiles of at most 64: bound by
+// reading the operator (once; its matrix-core time is 0.3 NB of that).  A
+// wave owns 16 samples and the tile's columns, so that operator rows go
+// straight from memory to the wave that multiplies them, THIN_AHEAD chunks
+// ahead (4 KB each: the 1656 waves of three 8832 x 2210 operators keep 20 MB
+// in flight), and only the columns are shared, through two LDS buffers.  The
+// multiply sequence of every output is rbf_gemm_kernel's.  Measured against
+// its 128-column tiles (us): three operators 8832 x 2210, 3 / 24 / 64 columns
+// 294 / 303 / 295 -> 110 / 135 / 203 (the operators alone take 97 at the
+// copy rate); 715 x 503, 24 columns 70 -> 15.
+constexpr int THIN_ROWS = 32, THIN_RB = 256, THIN_RS = THIN_RB + 16, THIN_AHEAD = 3, THIN_THREADS = 128;
+
+template <int NB>
+__global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
+{
+    constexpr int XLOADS = NB * 16 * THIN_RB / 16 / THIN_THREADS;    // 16-byte staging loads per thread
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2][NB * 16 * THIN_RS];
+    int gi = 0;
+    while (gi + 1 < G.count && (int) blockIdx.x >= G.g[gi + 1].first_tile) ++gi;
+    const gemm_group g = G.g[gi];
+    const int tile = (int) blockIdx.x - g.first_tile, row_tile = tile / g.tiles_n, col0 = (tile - row_tile * g.tiles_n) * (16 * NB);
+    const int row0 = row_tile * THIN_ROWS + (threadIdx.x >> 6) * 16;
+    const long row_bytes = (long) g.Kp * 8;
+    const int nchunks = (int) (row_bytes / THIN_RB);
+    const int lane = threadIdx.x & 63, frow = lane & 15, fgrp = lane >> 4;
+    const unsigned char* e = g.E[0] + (long) (row0 + frow) * row_bytes + fgrp * 16;
+    const unsigned char* x[XLOADS];
+    int xo[XLOADS];
+#pragma unroll
+    for (int i = 0; i < XLOADS; ++i) {
+        const int idx = threadIdx.x + THIN_THREADS * i, r = idx / (THIN_RB / 16), q = idx % (THIN_RB / 16);
+        x[i] = g.X[0] + (long) (col0 + r) * row_bytes + q * 16;
+        xo[i] = r * THIN_RS + q * 16;
+    }
+    u4 pe[THIN_AHEAD][4], px[XLOADS];
+    d4 acc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] = d4{};
+    // Loads past the last chunk repeat it (not used).
+    auto load_e = [&](int c, u4 (&to)[4]) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) to[s] = *(const u4*) (e + (long) min(c, nchunks - 1) * THIN_RB + s * 64);
+    };
+    auto load_x = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < XLOADS; ++i) px[i] = *(const u4*) (x[i] + (long) min(c, nchunks - 1) * THIN_RB);
+    };
+    auto store_x = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < XLOADS; ++i) *(u4*) (&lds[buf][xo[i]]) = px[i];
+    };
+#pragma unroll
+    for (int a = 0; a < THIN_AHEAD; ++a) load_e(a, pe[a]);
+    load_x(0);
+    store_x(0);
+    load_x(1);
+    __syncthreads();
+    auto chunk = [&](int c, u4 (&ce)[4]) {
+        const int buf = c & 1;
+        u4 ef[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) ef[s] = ce[s];
+        store_x(buf ^ 1);                       // chunk c + 1, read after the barrier below
+        load_x(c + 2);
+        load_e(c + THIN_AHEAD, ce);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const u4 xf = *(const u4*) (&lds[buf][(b * 16 + frow) * THIN_RS + s * 64 + fgrp * 16]);
+                mfma_step<MODE_F64>(xf, ef[s], xf, ef[s], acc[b]);
+            }
+        __syncthreads();
+    };
+    int c = 0;
+    for (; c + THIN_AHEAD <= nchunks; c += THIN_AHEAD) {
+#pragma unroll
+        for (int a = 0; a < THIN_AHEAD; ++a) chunk(c + a, pe[a]);
+    }
+#pragma unroll
+    for (int a = 0; a < THIN_AHEAD; ++a)
+        if (c + a < nchunks) chunk(c + a, pe[a]);
+    const int m = row0 + frow;
+    if (m >= g.M) return;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int n = col0 + b * 16 + fgrp + 4 * r;
+            if (n < g.N) g.Y[m + (long) g.M * n] = acc[b][r];
+        }
+}
+
 // Surface geometry of one cell per block from the evaluated position and
 // the two tangent blocks (each ns x 3nc, column comp*nc + cell).
 __global__ __launch_bounds__(256) void geometry_kernel(int ns, int nc, const double* __restrict__ y,
@@ -411,6 +505,16 @@ void launch_f64(int wn, const gemm_groups& G, int blocks, hipStream_t stream)
     else rbf_gemm_kernel<MODE_F64, 2><<<blocks, NTHREADS, 0, stream>>>(G);
 }
 
+constexpr int THIN_COLUMNS = 64;       // columns of a full tile of rbf_thin_kernel
+
+void launch_thin(int k, const gemm_groups& T, hipStream_t stream)
+{
+    if (k == 0) rbf_thin_kernel<1><<<T.total_tiles, THIN_THREADS, 0, stream>>>(T);
+    else if (k == 1) rbf_thin_kernel<2><<<T.total_tiles, THIN_THREADS, 0, stream>>>(T);
+    else if (k == 2) rbf_thin_kernel<3><<<T.total_tiles, THIN_THREADS, 0, stream>>>(T);
+    else rbf_thin_kernel<4><<<T.total_tiles, THIN_THREADS, 0, stream>>>(T);
+}
+
 int f64_variant(ibm_ctx* ctx, hipStream_t stream, const gemm_groups& G, int blocks)
 {
     (void) ctx;
@@ -451,13 +555,24 @@ int f64_variant(ibm_ctx* ctx, hipStream_t stream, const gemm_groups& G, int bloc
     return pick;
 }
 
-// Whether N columns of `op` are evaluated through residues (rbf_residue.hip)
-// rather than on the FP64 matrix cores: from RES_MIN_N columns on.  Measured
-// with 65 columns (FP64 / residues, us): 3 operators 8832 x 2210 295 / 236,
-// 2843 x 935 129 / 54, 715 x 503 71 / 28; with 600: 1349 / 651, 241 / 143,
-// 77 / 46.
-constexpr int RES_MIN_N = 65;
-bool by_residues(const ibm_rbf* op, int N) { return op->res && N >= RES_MIN_N; }
+// Whether an FP64 evaluation of N columns runs in rbf_thin_kernel: up to 64
+// columns, where reading the operator bounds it, and further on while the
+// contraction is short and the product small, where the residue path's four
+// launches take longer than the thin kernel's one.  Otherwise it goes through
+// residues (rbf_residue.hip) if the operator has them.  Measured (us, thin /
+// residues): one operator 584 x 311, 128 columns 17 / 24, 600 columns 19 / 29;
+// six of 715 x 503, 192 columns 29 / 42, 256 columns 50 / 43; six of
+// 1552 x 605, 66 columns 60 / 47; three of 2843 x 935, 66 columns 81 / 54.
+// The rule looks at one operator's shape only: an entry's path (and so every
+// bit of its result) does not depend on what it is batched with.
+constexpr int THIN_K = 550;
+constexpr double THIN_WORK = 9e7;
+bool by_thin_kernel(const ibm_rbf* op, int N)
+{
+    return op->mode == MODE_F64 &&
+           (N <= THIN_COLUMNS || (op->K <= THIN_K && (double) op->M * op->K * N < THIN_WORK));
+}
+bool by_residues(const ibm_rbf* op, int N) { return op->res && !by_thin_kernel(op, N); }
 
 // Offset of entry b's packed columns in the evaluation's packed operand and,
 // at b = count, its total; entries with the same columns share a packing
@@ -534,7 +649,7 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
         return fail(ctx, IBM_ERR_ARG, "no packed operand");
     }
 
-    gemm_groups G{};
+    gemm_groups G{}, thin[4]{};        // thin[k]: rbf_thin_kernel's entries with tiles of 16 (k + 1) columns
     int tiles = 0, ncols = 0;
     res_columns cols[RES_MAX_COLUMNS];
     for (int b = 0; b < count; ++b) {
@@ -555,8 +670,10 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
         int cols_pad = round_up(N[b], TILE);
         unsigned char* lo = planes(mode) > 1 ? hi + (size_t) cols_pad * op.Kp * elem_bytes(mode) : nullptr;
         if (do_pack && owner == b) pack(mode, stream, X[b], op.K, N[b], op.K, cols_pad, op.Kp, hi, lo);
+        const bool is_thin = by_thin_kernel(&op, N[b]);
         for (int j = j0; j < std::min(j1, op.nops); ++j) {
-            gemm_group& g = G.g[G.count++];
+            gemm_groups& to = is_thin ? thin[std::min(N[b] - 1, THIN_COLUMNS - 1) / 16] : G;
+            gemm_group& g = to.g[to.count++];
             g.E[0] = op.plane(j, 0);
             g.E[1] = planes(mode) > 1 ? op.plane(j, 1) : g.E[0];
             g.X[0] = hi;
@@ -565,9 +682,9 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
             g.M = op.M;
             g.N = N[b];
             g.Kp = op.Kp;
-            g.tiles_n = cols_pad / TILE;
+            g.tiles_n = is_thin ? (N[b] + THIN_COLUMNS - 1) / THIN_COLUMNS : cols_pad / TILE;
             g.first_tile = tiles;
-            tiles += (op.rows_pad / TILE) * g.tiles_n;
+            if (!is_thin) tiles += (op.rows_pad / TILE) * g.tiles_n;
         }
     }
     if (ncols) res_pack_columns(stream, ncols, cols);
@@ -602,10 +719,20 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
         }
         blocks = 8 * per_xcd;
     }
-    if (!tiles && !nres) return IBM_OK;
     const int wn = mode == MODE_F64 && tiles ? f64_variant(ctx, stream, G, blocks) : 2;
     prof_scope prof(ctx, "rbf_gemm", flops);
     if (nres) IBM_TRY(res_products(ctx, stream, nres, products, (unsigned char*) work));
+    for (int k = 0; k < 4; ++k) {
+        gemm_groups& T = thin[k];
+        if (!T.count) continue;
+        std::stable_sort(T.g, T.g + T.count, [](const gemm_group& a, const gemm_group& b) { return a.Kp > b.Kp; });
+        for (int q = 0; q < T.count; ++q) {
+            T.g[q].first_tile = T.total_tiles;
+            T.total_tiles += (T.g[q].M + THIN_ROWS - 1) / THIN_ROWS * T.g[q].tiles_n;
+        }
+        launch_thin(k, T, stream);
+    }
+    IBM_LAUNCH_CHECK(ctx);
     if (!tiles) return IBM_OK;
     if (mode == MODE_F64) {
         launch_f64(wn, G, blocks, stream);

@@ -1,5 +1,6 @@
 """FP64 RBF evaluation through residues on the INT8 matrix cores
-(csrc/rbf_residue.hip; taken from 65 columns on) against long-double products.
+(csrc/rbf_residue.hip) and in the few-column kernel (rbf_thin_kernel) against
+long-double products.
 
 Bar, elementwise: the operands are rounded to 2^-62 of the row's 1-norm and
 2^-54 of the column's maximum (half a unit each, the scales being powers of
@@ -27,9 +28,14 @@ def _bar(E, x):
     return (np.abs(x).max(1)[:, None] * np.abs(E).sum(1)[None, :]) * (K * 2.0 ** -62 + 2.0 ** -54 + 2.0 ** -53) * (1 + 2.0 ** -20)
 
 
-# (M, K, N): tiles of 256 x 128, 64-element chunks, three LDS buffers
-SHAPES = [(1, 1, 65), (255, 63, 65), (256, 64, 127), (257, 65, 128), (300, 129, 129), (513, 192, 200), (40, 257, 256),
-          (700, 320, 385)]
+# (M, K, N): tiles of 256 x 128, 64-element chunks, three LDS buffers;
+# contractions of more than 550 elements take the residue path
+SHAPES = [(1, 551, 65), (255, 575, 65), (256, 576, 127), (257, 577, 128), (300, 640, 129), (513, 641, 200), (40, 705, 256),
+          (700, 768, 385), (2000, 320, 400)]
+# 32-row blocks of 16-row waves, column tiles of 16 to 64, 32-element chunks
+# loaded three ahead; the last is past the work limit of the few-column kernel
+THIN = [(1, 1, 1), (15, 31, 3), (31, 32, 16), (33, 33, 17), (129, 95, 48), (64, 97, 49), (300, 129, 64), (257, 550, 65),
+        (90, 200, 129), (700, 321, 300)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
@@ -49,13 +55,29 @@ def test_residue_products_at_tile_edges(ibm, ctx, shape):
     op.close()
 
 
+@pytest.mark.parametrize("shape", THIN, ids=lambda s: "x".join(map(str, s)))
+def test_thin_products_at_tile_edges(ibm, ctx, shape):
+    """Bar: a chain of K fused multiply-adds, K 2^-53 of sum |E||X|."""
+    M, K, N = shape
+    rng = np.random.default_rng(M * K + N)
+    mats = [rng.standard_normal((M, K + 1)) for _ in range(2)]
+    x = rng.standard_normal((N, K))
+    op = ibm.RbfOperator(ctx, "f64", [_t(m) for m in mats], K)
+    (Y,) = ibm.rbf_eval(ctx, [op], [_t(x)])
+    Y = Y.cpu().numpy()
+    for j in range(2):
+        scale = np.abs(x) @ np.abs(mats[j][:, :K]).T
+        assert (np.abs(Y[j] - O.evaluate(mats[j], K, x)) <= (K + 1) * 2.0 ** -53 * scale).all()
+    op.close()
+
+
 @pytest.mark.parametrize("scale", [1e-300, 1e-160, 1e150, 1e300])
 def test_residue_products_at_extreme_scales(ibm, ctx, scale):
     rng = np.random.default_rng(7)
-    E, x = rng.standard_normal((200, 100)), rng.standard_normal((70, 100)) * scale
-    op = ibm.RbfOperator(ctx, "f64", [_t(E)], 100)
+    E, x = rng.standard_normal((200, 600)), rng.standard_normal((70, 600)) * scale
+    op = ibm.RbfOperator(ctx, "f64", [_t(E)], 600)
     (Y,) = ibm.rbf_eval(ctx, [op], [_t(x)])
-    err = np.abs(Y.cpu().numpy()[0] / scale - O.evaluate(E, 100, x / scale))
+    err = np.abs(Y.cpu().numpy()[0] / scale - O.evaluate(E, 600, x / scale))
     assert (err <= _bar(E, x / scale) + 2.0 ** -52 * np.abs(E).sum(1).max() * 6).all()
     op.close()
 
@@ -89,18 +111,18 @@ def test_residue_error_no_larger_than_a_fused_chain(ibm, ctx):
 
 def test_residue_products_carry_nan_and_infinity(ibm, ctx):
     rng = np.random.default_rng(5)
-    E, x = np.abs(rng.standard_normal((300, 90))) + 0.1, rng.standard_normal((80, 90))
-    x[3, 4], x[66, 0], x[79, 89] = np.nan, np.inf, -np.inf
-    op = ibm.RbfOperator(ctx, "f64", [_t(E)], 90)
+    E, x = np.abs(rng.standard_normal((300, 590))) + 0.1, rng.standard_normal((80, 590))
+    x[3, 4], x[66, 0], x[79, 589] = np.nan, np.inf, -np.inf
+    op = ibm.RbfOperator(ctx, "f64", [_t(E)], 590)
     (Y,) = ibm.rbf_eval(ctx, [op], [_t(x)])
     Y = Y.cpu().numpy()[0]
     assert np.isnan(Y[3]).all() and (Y[66] == np.inf).all() and (Y[79] == -np.inf).all()
     fine = [n for n in range(80) if n not in (3, 66, 79)]
-    assert (np.abs(Y[fine] - O.evaluate(E, 90, x[fine])) <= _bar(E, x[fine])).all()
+    assert (np.abs(Y[fine] - O.evaluate(E, 590, x[fine])) <= _bar(E, x[fine])).all()
     op.close()
     # an operator with a NaN stays on the FP64 matrix cores
     E[10, 10] = np.nan
-    op = ibm.RbfOperator(ctx, "f64", [_t(E)], 90)
+    op = ibm.RbfOperator(ctx, "f64", [_t(E)], 590)
     (Y,) = ibm.rbf_eval(ctx, [op], [_t(x[fine])])
     Y = Y.cpu().numpy()[0]
     assert np.isnan(Y[:, 10]).all() and np.isfinite(np.delete(Y, 10, axis=1)).all()
@@ -108,12 +130,12 @@ def test_residue_products_carry_nan_and_infinity(ibm, ctx):
 
 
 def test_batches_mix_both_paths_and_share_columns(ibm, ctx):
-    """Entries below and above the column threshold, and two operators on one
+    """Entries of both kernels, and two operators on one
     set of columns, give the values of separate calls."""
     rng = np.random.default_rng(6)
-    a = ibm.RbfOperator(ctx, "f64", [_t(rng.standard_normal((300, 150))) for _ in range(2)], 150)
-    b = ibm.RbfOperator(ctx, "f64", [_t(rng.standard_normal((90, 150)))], 150)
-    wide, thin = _t(rng.standard_normal((100, 150))), _t(rng.standard_normal((12, 150)))
+    a = ibm.RbfOperator(ctx, "f64", [_t(rng.standard_normal((300, 600))) for _ in range(2)], 600)
+    b = ibm.RbfOperator(ctx, "f64", [_t(rng.standard_normal((90, 600)))], 600)
+    wide, thin = _t(rng.standard_normal((100, 600))), _t(rng.standard_normal((12, 600)))
     got = ibm.rbf_eval(ctx, [a, b, a, b], [wide, wide, thin, thin])
     for y, op, x in zip(got, (a, b, a, b), (wide, wide, thin, thin)):
         (alone,) = ibm.rbf_eval(ctx, [op], [x])
@@ -127,7 +149,7 @@ def test_captured_tether_step_with_many_cells(ibm, ctx):
     (24 cells: 72 columns) equal those of the eager step, replay after replay."""
     import torch
     S, I = load_surfaces(), load_inputs()
-    ct = S.CellType(I.rbc_shape, 120, 300, 5, I.bauer_params)
+    ct = S.CellType(I.rbc_shape, 560, 700, 5, I.bauer_params)
     rng = np.random.default_rng(8)
     ref = 0.3 * ct.data_reference()
     x0 = np.stack([ref + 0.4 + 0.8 * rng.random(3)[:, None] for _ in range(24)], axis=1).reshape(-1)
