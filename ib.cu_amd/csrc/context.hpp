@@ -56,8 +56,8 @@ ibm_status hip_fail(ibm_ctx* ctx, hipError_t e, const char* what);
 // Returns a device buffer of at least `bytes` for `slot`, reallocating when
 // the request grows.  Contents are not preserved across growth.
 ibm_status scratch(ibm_ctx* ctx, int slot, size_t bytes, void** out);
-// Looks up, once per device, the device address of the fixed workspace of
-// ibm_spread_sets_noalloc; `device` must be current.
+// Allocates, once per device, the fixed workspace of ibm_spread_sets_noalloc;
+// `device` must be current.
 ibm_status static_scratch_init(ibm_ctx* ctx, int device);
 
 // Brackets a kernel launch with timing events when profiling is on.
@@ -108,10 +108,8 @@ ibm_status mg_solve_fixed_multi(int count, ibm_ctx* const* ctxs, ibm_mg* const* 
 bool fft_usable(const ibm_grid& g);
 ibm_status fft_solve(ibm_ctx* ctx, ibm_fft* p, double sigma, double tau, const double* b, double* x);
 
-// Whether the tile spread takes these MAC grids, and the timestep's spread
-// of nsets marker sets by the tile (tiles = true) or the brick kernel.
-bool tiles_usable(ibm_ctx* ctx, const ibm_grid* grids);
-ibm_status spread_sets_step(ibm_ctx* ctx, const ibm_grid* grids, int delta, bool tiles, int nsets, const int* n,
+// The timestep's spread of nsets marker sets.
+ibm_status spread_sets_step(ibm_ctx* ctx, const ibm_grid* grids, int delta, int nsets, const int* n,
                             const double* const* x, const double* const* f, double* const* fe);
 
 } // namespace ibm

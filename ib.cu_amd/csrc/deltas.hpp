@@ -55,13 +55,19 @@ IBM_HD void delta_cosine4(double d, double w[4])
     w[3] = 0.25 * (1 - c);
 }
 
-// Peskin's 4-point kernel (ib/peskin.h:6-14), evaluated as written.
-IBM_HD double delta_peskin(double r)
+// Peskin's 4-point kernel (ib/peskin.h:6-14) at the four offsets.  With
+// s = -d in [0, 1) all four distances 1 + s, s, 1 - s, 2 - s have the same
+// square root q = sqrt(1 + 4 s - 4 s^2) (substitute them into 1 + 4 r - 4 r^2
+// for r < 1 and -7 + 12 r - 4 r^2 beyond), so
+//   phi(d-1) = (3 - 2s - q)/8, phi(d) = (3 - 2s + q)/8,
+//   phi(d+1) = (1 + 2s + q)/8, phi(d+2) = (1 + 2s - q)/8.
+IBM_HD void delta_peskin4(double d, double w[4])
 {
-#pragma clang fp contract(off)
-    double s = r < 0 ? -r : r;
-    return s < 1 ? (3 - 2 * s + sqrt(1 + 4 * s - 4 * s * s)) / 8
-                 : (5 - 2 * s - sqrt(-7 + 12 * s - 4 * s * s)) / 8;
+    const double s = -d, q = sqrt(fma(4 * s, 1 - s, 1.0)), a = 3 - 2 * s, b = 1 + 2 * s;
+    w[0] = 0.125 * (a - q);
+    w[1] = 0.125 * (a + q);
+    w[2] = 0.125 * (b + q);
+    w[3] = 0.125 * (b - q);
 }
 
 // Cardinal B-spline by the reference's recursion (ib/bspline.h:13-27):
@@ -85,8 +91,7 @@ IBM_HD void delta4(int kind, double d, double w[4])
     if (kind == IBM_DELTA_COSINE) {
         delta_cosine4(d, w);
     } else if (kind == IBM_DELTA_PESKIN) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) w[s] = delta_peskin(d + (s - 1));
+        delta_peskin4(d, w);
     } else {
 #pragma unroll
         for (int s = 0; s < 4; ++s) w[s] = delta_bspline<3>(d + (s - 1));

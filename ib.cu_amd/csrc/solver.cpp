@@ -129,7 +129,6 @@ struct ibm_solver {
     };
     std::vector<type_t> types;
     double *F[3]{}, *H[3]{}, *rhs[3]{}, *du[3]{}, *div = nullptr;
-    bool tile_spread = false;          // spread by tiles (the grids allow it) or by the brick kernel
     double *du_prev[3]{}, *p_prev = nullptr;   // the solutions one step further back
     int* warm_hist = nullptr;          // device: solutions known at step size history_dt (0, 1, 2)
     // Fixed-count steps run the three Helmholtz solves concurrently: the
@@ -423,7 +422,7 @@ ibm_status step_impl(ibm_ctx* ctx, ibm_solver* s, ibm_state* st, const double* c
             xs[t] = s->types[t].Y;
             fs[t] = s->types[t].f;
         }
-        IBM_TRY(spread_sets_step(ctx, s->g, P.delta, s->tile_spread, nt, counts, xs, fs, s->F));
+        IBM_TRY(spread_sets_step(ctx, s->g, P.delta, nt, counts, xs, fs, s->F));
     }
     // 4. advection (on an auxiliary stream beside the geometry it was starved
     // of compute units by the matrix-core blocks: 0.47 ms per component
@@ -628,9 +627,6 @@ ibm_status ibm_solver_create(ibm_ctx* ctx, const ibm_dimension* domain, int ndim
         s->nu[i] = (size_t) ibm_grid_size(&s->g[i]);
         s->Bw[i] = make_ins_boundary(s->g[i], i, 2);
     }
-    // The tile spread visits every marker once (the brick kernel about 2.6
-    // times at C4 density); it needs periodic axes of whole bricks.
-    s->tile_spread = ndims == 3 && tiles_usable(ctx, s->g);
     s->np = (size_t) ibm_grid_size(&s->gp);
     s->dt = P.timestep;
     // Channel grids (periodic x and z of power-of-two sizes, walls in y) are

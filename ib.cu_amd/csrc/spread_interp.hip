@@ -9,15 +9,15 @@
 // with the reference's index conventions (geometry.hpp).
 //
 // MI355X design:
-//   * markers are counting-sorted once into grid bins (shared by the three
-//     components), canonically ordered inside a bin, so every later pass is
-//     independent of scheduling;
-//   * spreading is owner-computes: one workgroup per 8x8x8 brick of grid
-//     points gathers the markers of the bins whose stencils reach the brick,
-//     evaluates their separable weights once per chunk into LDS, and one
-//     wavefront per component adds each marker's 4x4x4 = 64 stencil values
-//     with one lane per stencil point.  The brick is written once with plain
-//     stores: no zero fill, no global atomics, bitwise reproducible.
+//   * markers are counting-sorted into bins of 4 x 4 x 4 cells, and one
+//     workgroup per brick of 8 x 8 x 8 cells adds its markers' stencils, each
+//     visited once, to a tile of 64-bit fixed-point integers in LDS; a merge
+//     pass sums the tiles.  Integer sums do not depend on scheduling: bitwise
+//     reproducible without global atomics or an order inside a bin;
+//   * grids whose tiles would not fit the fixed workspace although their bins
+//     do are spread owner-computes: one workgroup per 8x8x8 brick of grid
+//     points gathers the (canonically ordered) markers of the bins whose
+//     stencils reach the brick into an LDS tile of the same integers;
 //   * interpolation is one lane per marker with the separable sum
 //     sum_z wz sum_y wy sum_x wx u.
 #include <hip/hip_runtime.h>
@@ -29,30 +29,39 @@
 
 
 // ----------------------------------------------------------------------
-// Fixed workspace of ibm_spread_sets_noalloc: the buffers of one binning
-// pass for at most STATIC_MAX_MARKERS markers and STATIC_MAX_BINS bins
-// (a 128 x 129 x 128 cell grid), 36.6 MB per device, held from module load
-// until the process ends.  Host code never passes `scratch` itself to a
-// kernel: its device address (one per GPU) comes from hipGetSymbolAddress.
+// Fixed workspace of ibm_spread_sets_noalloc: the buffers of one spread of at
+// most STATIC_MAX_MARKERS markers onto grids of at most STATIC_MAX_BINS bins
+// (a 128 x 129 x 128 cell grid), 184 MB per device, held from the first
+// ibm_create until the process ends: the tiles of STATIC_MAX_BRICKS bricks (as many as
+// such a grid has, unless an axis is so short that its bricks are mostly
+// empty: those grids take the brick kernel, which needs 36.6 MB) or that
+// kernel's bins.
 // ----------------------------------------------------------------------
 namespace ibm_fixed {
 constexpr size_t STATIC_MAX_MARKERS = size_t(1) << 18;
 constexpr size_t STATIC_MAX_BINS = size_t(128) * 129 * 128;
+constexpr size_t STATIC_MAX_BRICKS = size_t(16) * 17 * 16;
 constexpr size_t STATIC_SCAN_BYTES = size_t(1) << 20;
 constexpr size_t STATIC_STATS_BYTES = 4096;
+constexpr size_t TILE_BYTES = sizeof(long long) * 3 * 12 * 12 * 12;      // one brick's tiles
 
 constexpr size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 constexpr size_t STATIC_BIN_WORDS = align256(sizeof(int) * (STATIC_MAX_BINS + 1));
 constexpr size_t STATIC_INT_ARRAY = align256(sizeof(int) * STATIC_MAX_MARKERS);
-constexpr size_t STATIC_SCRATCH_BYTES =
+constexpr size_t STATIC_BRICK_KERNEL_BYTES =
     2 * STATIC_BIN_WORDS +                                   // count, start
     4 * STATIC_INT_ARRAY +                                   // key, rank, perm, code
     align256(sizeof(long long) * STATIC_MAX_MARKERS) +       // tmp
     align256(sizeof(double) * 6 * STATIC_MAX_MARKERS) +      // sorted positions and forces
     STATIC_STATS_BYTES + STATIC_SCAN_BYTES;
+constexpr size_t STATIC_TILE_KERNEL_BYTES =
+    2 * align256(sizeof(int) * (8 * STATIC_MAX_BRICKS + 1)) +    // count, start
+    3 * STATIC_INT_ARRAY +                                   // key, rank, perm
+    STATIC_STATS_BYTES + 256 + align256(sizeof(int) * STATIC_MAX_BRICKS) +   // statistics, quantum, flags
+    TILE_BYTES * STATIC_MAX_BRICKS;
+constexpr size_t STATIC_SCRATCH_BYTES =
+    STATIC_TILE_KERNEL_BYTES > STATIC_BRICK_KERNEL_BYTES ? STATIC_TILE_KERNEL_BYTES : STATIC_BRICK_KERNEL_BYTES;
 } // namespace ibm_fixed
-
-static __device__ __align__(256) unsigned char scratch[ibm_fixed::STATIC_SCRATCH_BYTES];
 
 namespace ibm {
 namespace {
@@ -977,9 +986,7 @@ constexpr int STATIC_MAX_DEVICES = 64;
 std::mutex static_scratch_mutex;
 void* static_scratch_ptr[STATIC_MAX_DEVICES] = {};
 
-// Carves the binning buffers out of the fixed workspace at `base` (a device
-// address of `scratch`).
-ibm_status static_bin_work(ibm_ctx* ctx, unsigned char* base, int total, int nbins, bin_work* w)
+ibm_status static_limits(ibm_ctx* ctx, int total, int nbins)
 {
     if ((size_t) total > STATIC_MAX_MARKERS)
         return fail(ctx, IBM_ERR_SIZE, "ibm_spread_sets_noalloc takes at most %zu markers (got %d)",
@@ -987,6 +994,13 @@ ibm_status static_bin_work(ibm_ctx* ctx, unsigned char* base, int total, int nbi
     if ((size_t) nbins > STATIC_MAX_BINS)
         return fail(ctx, IBM_ERR_SIZE, "ibm_spread_sets_noalloc takes grids of at most %zu bins (got %d)",
                     STATIC_MAX_BINS, nbins);
+    return IBM_OK;
+}
+
+// Carves the binning buffers of the brick kernel out of the fixed workspace
+// at `base` (a device address of `scratch`).
+ibm_status static_bin_work(ibm_ctx* ctx, unsigned char* base, int nbins, bin_work* w)
+{
     size_t off = 0;
     auto take = [&](size_t bytes) { unsigned char* p = base + off; off += align256(bytes); return p; };
     w->count = (int*) take(STATIC_BIN_WORDS);
@@ -1013,23 +1027,27 @@ ibm_status static_bin_work(ibm_ctx* ctx, unsigned char* base, int total, int nbi
 //
 // The markers of nboxes independent boxes (one set of component grids,
 // repeated; the C4 channel is one box, the small periodic boxes of a batch
-// are many) are counting-sorted into bins of 8 x 8 x 8 face-aligned cells
-// ("bricks"), brick-major.  One workgroup per brick adds each of its
-// markers' 64 stencil values per component into a 12 x 12 x 12 tile of
-// 64-bit fixed-point integers in LDS (the brick's points plus the reach of
-// its stencils), and stores the tile once.  A merge pass then forms every
-// grid point from the (at most eight) tiles that cover it.  Integer addition
-// is associative, so the result does not depend on scheduling: no
-// floating-point atomics, no global atomics, bitwise reproducible.
+// are many) are counting-sorted into bins of 4 x 4 x 4 face-aligned cells,
+// eight to a "brick" of 8 x 8 x 8, brick-major.  One workgroup per brick adds
+// each of its markers' 64 stencil values per component into a 12 x 12 x 12
+// tile of 64-bit fixed-point integers in LDS (the brick's points plus the
+// reach of its stencils), and stores the tile once.  A merge pass then forms
+// every grid point from the tiles that cover it.  Integer addition is
+// associative, so the result does not depend on scheduling nor on the order
+// inside a bin: no floating-point atomics, no global atomics on the grid,
+// bitwise reproducible.
 //
 // Tile geometry along axis j: brick b covers bins q in [8 b, 8 b + 8) (bin
-// coordinates relative to qmin); a marker of bin q has base cell
-// base_c = q + qmin + d_c for component c with d_c in [lo_j, hi_j]
-// (hi_j - lo_j <= 1), and touches points base_c - 1 .. base_c + 2, so the
-// tile starts at point T0 = 8 b + qmin + lo - 1 and a marker's stencil
-// origin lies at tile index (q - 8 b) + (d_c - lo) in [0, 8].
+// coordinates relative to qmin; the last brick of an axis may be partial); a
+// marker of bin q has base cell base_c = q + qmin + d_c for component c with
+// d_c in [lo_j, hi_j] (hi_j - lo_j <= 1), and touches points base_c - 1 ..
+// base_c + 2, so the tile starts at point T0 = 8 b + qmin + lo - 1 and a
+// marker's stencil origin lies at tile index (q - 8 b) + (d_c - lo) in
+// [0, 8].  On a periodic axis the tile index of a point is its distance from
+// T0 modulo the cells, plus any multiple of them that stays in the tile.
 // ----------------------------------------------------------------------
-constexpr int TB = 8;                       // brick edge in bins
+constexpr int TB = 8;                       // brick edge in cells
+constexpr int SUB = 8;                      // bins (of 4 x 4 x 4 cells) per brick
 constexpr int TT = 12;                      // tile edge in points
 constexpr int TILE_PTS = TT * TT * TT;
 constexpr int TILE_THREADS = 256;
@@ -1038,7 +1056,7 @@ struct tile_desc {
     int nbr[3];         // bricks per axis
     int bricks;         // bricks per box
     int nboxes;
-    int keys;           // nboxes * bricks * 512
+    int keys;           // nboxes * bricks * SUB
     int box_points[3];  // points of one box's component grid
 };
 
@@ -1053,270 +1071,537 @@ __device__ inline int box_of(const int* __restrict__ off, int nboxes, int m)
     return lo;
 }
 
-__global__ void tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td,
-                                  const int* __restrict__ box_off, int* __restrict__ key, int* __restrict__ rank,
-                                  int* __restrict__ count, bin_stats* __restrict__ stats)
+// Global load through a pointer that comes out of an indexed table (which
+// would otherwise compile to a flat load).
+__device__ inline double gload(const double* p, size_t i)
 {
-    int m = blockIdx.x * blockDim.x + threadIdx.x;
+    return ((const __attribute__((address_space(1))) double*) p)[i];
+}
+
+__device__ inline void load_marker(const marker_sets& sets, int m, double (&p)[3])
+{
+    const int k = set_of(sets, m), l = m - sets.offset[k];
+    const size_t n = (size_t) (sets.offset[k + 1] - sets.offset[k]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) p[j] = gload(sets.x[k], j * n + l);
+}
+
+__device__ inline void load_force(const marker_sets& sets, int m, double (&f)[3])
+{
+    const int k = set_of(sets, m), l = m - sets.offset[k];
+    const size_t n = (size_t) (sets.offset[k + 1] - sets.offset[k]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) f[j] = gload(sets.f[k], j * n + l);
+}
+
+__device__ inline double load_force(const marker_sets& sets, int m, int c)
+{
+    const int k = set_of(sets, m), l = m - sets.offset[k];
+    return gload(sets.f[k], (size_t) c * (sets.offset[k + 1] - sets.offset[k]) + l);
+}
+
+// Clears the bin counts and the statistics of a tile spread.
+__global__ void __launch_bounds__(256) tile_clear_kernel(int* __restrict__ count, int keys, bin_stats* __restrict__ stats)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < keys + 1) count[i] = 0;
+    if (blockIdx.x == 0)
+        for (int w = threadIdx.x; w < (int) (sizeof(bin_stats) / 4); w += 256) ((unsigned*) stats)[w] = 0u;
+}
+
+// Bin of every marker, its rank inside the bin and the force maximum.  Bound
+// by latency (positions and forces, then the returning atomics): a thread
+// takes COUNT_ITEMS markers, 64 apart, so that their loads and atomics are in
+// flight together.  Consecutive markers mostly share a bin, so a wavefront
+// finds its few distinct bins by ballots and takes each one's ranks with one
+// atomic.  2.39 M markers: 134 us with single-cell bins (a wavefront meets
+// twenty or more), 102 with 4 x 4 x 4-cell bins, 58 with four markers a
+// thread.
+constexpr int COUNT_ITEMS = 4;
+
+__global__ void __launch_bounds__(256)
+tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const int* __restrict__ box_off,
+                  int* __restrict__ key, int* __restrict__ rank, int* __restrict__ count, bin_stats* __restrict__ stats)
+{
+    const int lane = threadIdx.x & 63;
+    const int m0 = (blockIdx.x * 4 + (int) (threadIdx.x >> 6)) * (64 * COUNT_ITEMS) + lane;
+    double p[COUNT_ITEMS][3], f[COUNT_ITEMS][3];
+#pragma unroll
+    for (int i = 0; i < COUNT_ITEMS; ++i) {
+        const int m = min(m0 + 64 * i, sets.total - 1);
+        load_marker(sets, m, p[i]);
+        load_force(sets, m, f[i]);
+    }
     unsigned long long fbits = 0;
-    const bool valid = m < sets.total;
-    int bin = -1;
-    if (valid) {
-        int k = set_of(sets, m);
-        int l = m - sets.offset[k];
-        int n = sets.offset[k + 1] - sets.offset[k];
-        const double* x = sets.x[k];
-        double p[3] = {x[l], x[n + l], x[2 * n + l]};
-        int q[3], br[3], lb[3];
+    int bin[COUNT_ITEMS], leader[COUNT_ITEMS], before[COUNT_ITEMS], base[COUNT_ITEMS];
+#pragma unroll
+    for (int i = 0; i < COUNT_ITEMS; ++i) {
+        const int m = m0 + 64 * i;
+        const bool valid = m < sets.total;
+        int br[3], sub = 0;
+#pragma unroll
         for (int j = 0; j < 3; ++j) {
-            stencil_axis st = kstencil(g.a[bd.fc[j]][j], p[j]);
-            q[j] = st.base + bd.fs[j];
-            int qb = q[j] - bd.qmin[j];
+            stencil_axis st = kstencil(g.a[bd.fc[j]][j], p[i][j]);
+            int qb = st.base + bd.fs[j] - bd.qmin[j];
             qb = qb < 0 ? 0 : (qb >= bd.nb[j] ? bd.nb[j] - 1 : qb);
             br[j] = qb / TB;
-            lb[j] = qb - br[j] * TB;
+            sub |= ((qb >> 2) & 1) << j;
         }
-        const int box = box_of(box_off, td.nboxes, m);
-        const int brick = ((box * td.nbr[2] + br[2]) * td.nbr[1] + br[1]) * td.nbr[0] + br[0];
-        bin = brick * (TB * TB * TB) + lb[0] + TB * (lb[1] + TB * lb[2]);
-        key[m] = bin;
-        const double* f = sets.f[k];
-        const double f0 = fabs(f[l]), f1 = fabs(f[n + l]), f2 = fabs(f[2 * n + l]);
+        const int box = td.nboxes > 1 && valid ? box_of(box_off, td.nboxes, m) : 0;
+        bin[i] = (((box * td.nbr[2] + br[2]) * td.nbr[1] + br[1]) * td.nbr[0] + br[0]) * SUB + sub;
+        const double f0 = fabs(f[i][0]), f1 = fabs(f[i][1]), f2 = fabs(f[i][2]);
         double a = f0 > f1 ? f0 : f1;
         a = a > f2 ? a : f2;
+        // A non-finite force is recorded as the canonical NaN, whose bit
+        // pattern exceeds every finite and infinite one, so it survives the
+        // integer maxima and poisons the spread result.
         if (!(isfinite(f0) && isfinite(f1) && isfinite(f2))) a = __longlong_as_double(0x7ff8000000000000ll);
-        fbits = (unsigned long long) __double_as_longlong(a);
-    }
-    {
+        if (valid) {
+            key[m] = bin[i];
+            const unsigned long long bits = (unsigned long long) __double_as_longlong(a);
+            fbits = bits > fbits ? bits : fbits;
+        }
         // ranks inside a bin, one atomic per group of lanes sharing a bin
-        const int lane = threadIdx.x & 63;
         const unsigned long long lt = (1ull << lane) - 1;
         unsigned long long todo = __ballot(valid);
-        int leader = lane, before = 0, size = 0;
+        int size = 0;
+        leader[i] = lane;
+        before[i] = 0;
         while (todo) {
             const int l = __ffsll((long long) todo) - 1;
-            const int lbin = __shfl(bin, l, 64);
-            const unsigned long long grp = __ballot(valid && bin == lbin) & todo;
+            const int lbin = __shfl(bin[i], l, 64);
+            const unsigned long long grp = __ballot(valid && bin[i] == lbin) & todo;
             if ((grp >> lane) & 1) {
-                leader = l;
-                before = __popcll(grp & lt);
+                leader[i] = l;
+                before[i] = __popcll(grp & lt);
             }
             if (lane == l) size = __popcll(grp);
             todo &= ~grp;
         }
-        int base = 0;
-        if (valid && leader == lane) base = atomicAdd(&count[bin], size);
-        base = __shfl(base, leader, 64);
-        if (valid) rank[m] = base + before;
+        base[i] = 0;
+        if (valid && leader[i] == lane) base[i] = atomicAdd(&count[bin[i]], size);
+    }
+#pragma unroll
+    for (int i = 0; i < COUNT_ITEMS; ++i) {
+        const int r = __shfl(base[i], leader[i], 64) + before[i];
+        if (m0 + 64 * i < sets.total) rank[m0 + 64 * i] = r;
     }
     fbits = wave_max(fbits);
-    if ((threadIdx.x & 63) == 0 && fbits) atomicMax(&stats->max_abs_f[blockIdx.x % STAT_SLOTS], fbits);
+    if (lane == 0 && fbits) atomicMax(&stats->max_abs_f[blockIdx.x % STAT_SLOTS], fbits);
 }
 
-// Marker m to slot start[key[m]] + rank[m] of its bin, positions and forces
-// gathered into `sorted` (six consecutive doubles per slot: x, y, z, fx, fy,
-// fz, one 48-byte store); the largest bin count into the stats.  The order inside a bin is that of tile_count_kernel's atomics and
-// varies from run to run: the tiles sum integers, so it does not matter.
-__global__ void tile_scatter_kernel(marker_sets sets, const int* __restrict__ key, const int* __restrict__ rank,
-                                    const int* __restrict__ start, double* __restrict__ sorted,
-                                    bin_stats* __restrict__ stats)
+// The marker indices in bin order (start[key] + rank).
+__global__ void __launch_bounds__(256)
+tile_place_kernel(int total, const int* __restrict__ key, const int* __restrict__ rank, const int* __restrict__ start,
+                  int* __restrict__ perm)
 {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const int total = sets.total;
-    unsigned long long cnt = 0;
-    if (m < total) {
-        const int b = key[m];
-        const int s0 = start[b];
-        const int dst = s0 + rank[m];
-        cnt = (unsigned long long) (start[b + 1] - s0);
-        const int k = set_of(sets, m);
-        const int l = m - sets.offset[k];
-        const int n = sets.offset[k + 1] - sets.offset[k];
-        const double* x = sets.x[k];
-        const double* f = sets.f[k];
-        double2* o = (double2*) (sorted + (size_t) 6 * dst);
-        o[0] = make_double2(x[l], x[(size_t) n + l]);
-        o[1] = make_double2(x[(size_t) 2 * n + l], f[l]);
-        o[2] = make_double2(f[(size_t) n + l], f[(size_t) 2 * n + l]);
-    }
-    cnt = wave_max(cnt);
-    if ((threadIdx.x & 63) == 0 && cnt) atomicMax(&stats->max_count[blockIdx.x % STAT_SLOTS], cnt);
+    if (m < total) perm[start[key[m]] + rank[m]] = m;
 }
 
-// The quantum of the fixed-point tiles: q = 2^(e - 62) with e the exponent
-// of the bound 64 * max_count * max|f| * max_c res3_c * 0.3 on any point's
-// sum; a non-finite bound marks the result as poisoned (all NaN).
+// The fixed-point quantum q = 2^(e - 62), e the exponent of a bound on any
+// point's sum: the base cells whose stencils reach a point lie in five
+// consecutive face-aligned cells per axis, so in `reach` bins (two per axis,
+// three where the last bin of a periodic axis is partial), and |sum| <= reach
+// max_count max|f| max_c res3_c phi^3, phi the delta kernel's maximum.  A
+// non-finite bound marks the result as poisoned (all NaN).
 struct tile_scale {
     double inv_q, q;
     int poisoned, pad;
 };
 
-__global__ void tile_scale_kernel(kgrids g, const bin_stats* __restrict__ stats, tile_scale* __restrict__ out)
+__device__ inline void make_scale(const kgrids& g, int delta, int reach, unsigned long long max_f, unsigned long long max_count,
+                                  tile_scale* out)
+{
+    const double phi3 = delta == IBM_DELTA_BSPLINE3 ? 0.3 : 0.126;     // (2/3)^3, (1/2)^3 with room for rounding
+    const double res3 = fmax(g.res3[0], fmax(g.res3[1], g.res3[2]));
+    const double one = __longlong_as_double((long long) max_f) * res3 * phi3;
+    const double bound = (double) reach * (double) max_count * one;
+    tile_scale s;
+    s.poisoned = !(bound <= 1.7976931348623157e308);
+    int e2 = 0;
+    if (!s.poisoned && bound > 0) frexp(bound, &e2);
+    s.inv_q = ldexp(1.0, 62 - e2);
+    s.q = s.poisoned ? __longlong_as_double(0x7ff8000000000000ll) : ldexp(1.0, e2 - 62);
+    s.pad = 0;
+    *out = s;
+}
+
+__global__ void tile_scale_kernel(kgrids g, int delta, int reach, const bin_stats* __restrict__ stats, tile_scale* __restrict__ out)
 {
     const int tid = threadIdx.x;      // one wavefront
     unsigned long long fb = wave_max(stats->max_abs_f[tid]);
     unsigned long long cm = wave_max(stats->max_count[tid]);
-    if (tid == 0) {
-        double res3 = fmax(g.res3[0], fmax(g.res3[1], g.res3[2]));
-        double bound = 64.0 * (double) cm * __longlong_as_double((long long) fb) * res3 * 0.3;
-        tile_scale s;
-        s.poisoned = !(bound <= 1.7976931348623157e308);
-        int e2 = 0;
-        if (!s.poisoned && bound > 0) frexp(bound, &e2);
-        s.inv_q = ldexp(1.0, 62 - e2);
-        s.q = s.poisoned ? __longlong_as_double(0x7ff8000000000000ll) : ldexp(1.0, e2 - 62);
-        s.pad = 0;
-        *out = s;
+    if (tid == 0) make_scale(g, delta, reach, fb, cm, out);
+}
+
+__global__ void __launch_bounds__(256) tile_max_kernel(const int* __restrict__ count, int keys, bin_stats* __restrict__ stats)
+{
+    unsigned long long m = 0;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < keys; i += gridDim.x * 256)
+        m = (unsigned long long) count[i] > m ? (unsigned long long) count[i] : m;
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0 && m) atomicMax(&stats->max_count[blockIdx.x % STAT_SLOTS], m);
+}
+
+// Bin starts (keys + 1), the largest bin and the quantum, in one workgroup:
+// up to SCAN_MAX bins this is one launch instead of the two of a device-wide
+// scan and the quantum's own.  Wave w takes the w-th sixteenth of the bins, in
+// steps of 256: once for its sum, once for the starts (67,584 bins of the C4
+// channel: 8 us; 32 with a thread on 66 consecutive bins).
+constexpr int SCAN_THREADS = 1024, SCAN_WAVES = SCAN_THREADS / 64, SCAN_MAX = 1 << 17;
+
+__device__ inline int4 load_counts(const int* __restrict__ count, int i, int end)
+{
+    if (i + 4 <= end) return *(const int4*) (count + i);
+    return make_int4(i < end ? count[i] : 0, i + 1 < end ? count[i + 1] : 0, i + 2 < end ? count[i + 2] : 0, 0);
+}
+
+__global__ void __launch_bounds__(SCAN_THREADS)
+tile_scan_kernel(kgrids g, int delta, int reach, const int* __restrict__ count, int keys, const bin_stats* __restrict__ stats,
+                 int* __restrict__ start, tile_scale* __restrict__ out)
+{
+    __shared__ int wave_sum[SCAN_WAVES];
+    __shared__ int wave_top[SCAN_WAVES];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per = (keys + SCAN_WAVES * 256 - 1) / (SCAN_WAVES * 256) * 256;
+    const int i0 = wave * per + lane * 4, end = min(wave * per + per, keys);
+    int sum = 0, top = 0;
+#pragma unroll 4
+    for (int i = i0; i < end; i += 256) {
+        const int4 v = load_counts(count, i, end);
+        sum += v.x + v.y + v.z + v.w;
+        top = max(max(top, max(v.x, v.y)), max(v.z, v.w));
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        sum += __shfl_xor(sum, off, 64);
+        top = max(top, __shfl_xor(top, off, 64));
+    }
+    if (lane == 0) {
+        wave_sum[wave] = sum;
+        wave_top[wave] = top;
+    }
+    __syncthreads();
+    int run = 0;
+    for (int w = 0; w < wave; ++w) run += wave_sum[w];
+    int4 next = load_counts(count, i0, end);
+    for (int step = 0; step < per; step += 256) {
+        const int i = i0 + step;
+        const int4 v = next;
+        next = load_counts(count, i + 256, end);
+        const int own = v.x + v.y + v.z + v.w;
+        int incl = own;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += y;
+        }
+        const int s0 = run + incl - own, s1 = s0 + v.x, s2 = s1 + v.y, s3 = s2 + v.z;
+        if (i + 4 <= end) {
+            *(int4*) (start + i) = make_int4(s0, s1, s2, s3);
+        } else {
+            if (i < end) start[i] = s0;
+            if (i + 1 < end) start[i + 1] = s1;
+            if (i + 2 < end) start[i + 2] = s2;
+        }
+        run += __shfl(incl, 63, 64);
+    }
+    if (wave == SCAN_WAVES - 1 && lane == 0) start[keys] = run;          // the last wave ends at the total
+    if (wave == 0) {
+        const unsigned long long fb = wave_max(stats->max_abs_f[lane]);
+        const unsigned long long cm = wave_max((unsigned long long) (lane < SCAN_WAVES ? wave_top[lane] : 0));
+        if (lane == 0) make_scale(g, delta, reach, fb, cm, out);
     }
 }
 
-// One workgroup per brick: lanes are markers, each adds its 3 x 64 stencil
-// values to the LDS tile; the tile is then stored (flags[brick] = 0 for a
-// brick without markers, whose tile is not written).
-__global__ void __launch_bounds__(TILE_THREADS)
-tile_spread_kernel(kgrids g, bin_desc bd, tile_desc td, int delta, int total, const int* __restrict__ start,
-                   const double* __restrict__ sorted, const tile_scale* __restrict__ scale,
-                   unsigned long long* __restrict__ tiles, int* __restrict__ flags)
+// Adds the integer nearest to w v (in quanta) to a tile entry.  FAST: the
+// integer is below 2^51, so one fused multiply-add with 1.5 * 2^52 leaves it
+// in the low bits (the constant's own bits are the high word's).  Otherwise
+// the same in two parts: the multiple of 2^12 nearest to w v, taken with a
+// constant whose mantissa bits, shifted up by 12, cancel those that the exact
+// remainder's constant brings along (the mantissa field holds 2^52 - 0x4338
+// 2^36 plus an integer below 2^50 in magnitude: no carry leaves it).  A plain
+// conversion to a 64-bit integer is about ten instructions, several of them
+// at a fraction of the rate.
+template <bool FAST>
+__device__ inline void add_value(unsigned long long* at, double w, double v)
 {
-    __shared__ unsigned long long acc[3][TILE_PTS];
-    const int brick = blockIdx.x;
-    const int s0 = start[(size_t) brick * (TB * TB * TB)];
-    const int s1 = start[(size_t) (brick + 1) * (TB * TB * TB)];
-    const int tid = threadIdx.x;
+    constexpr double ROUND = 0x1.8p52;                        // bits 0x4338 << 48
+    if (FAST) {
+        const double t = fma(w, v, ROUND);
+        atomicAdd(at, (unsigned long long) __double_as_longlong(t) - 0x4338000000000000ull);
+    } else {
+        constexpr double C = ((double) (1ull << 52) + (double) ((1ull << 52) - (0x4338ull << 36))) * 0x1p12;
+        const double t = fma(w, v, C);
+        const double rest = fma(w, v, C - t) + ROUND;
+        atomicAdd(at, ((unsigned long long) __double_as_longlong(t) << 12) + (unsigned long long) __double_as_longlong(rest));
+    }
+}
+
+// The 64 values of one component of a marker, plane by plane.
+template <bool FAST>
+__device__ inline void add_stencil(unsigned long long* t, const double (&wx)[4], const double (&wy)[4],
+                                   const double (&wz)[4], double fq)
+{
+    double z0 = wz[0], z1 = wz[1], z2 = wz[2], z3 = wz[3];
+#pragma unroll 1
+    for (int sz = 0; sz < 4; ++sz) {
+#pragma unroll
+        for (int sy = 0; sy < 4; ++sy) {
+            const double wyz = z0 * (wy[sy] * fq);
+#pragma unroll
+            for (int sx = 0; sx < 4; ++sx) add_value<FAST>(t + sx + TT * sy, wx[sx], wyz);
+        }
+        t += TT * TT;
+        z0 = z1;
+        z1 = z2;
+        z2 = z3;
+    }
+}
+
+// One workgroup per brick and component: its markers' stencils into the
+// component's tile in LDS, which is then stored (flags[brick] = 0 for a brick
+// without markers, whose tiles are not written).  Bound by the LDS atomics
+// (52 % of the cycles at C4, two thirds of them bank conflicts), the vector
+// ALU that feeds them (47 %) and the loads' latency.  Lanes of one atomic
+// that hit one address serialise, so each chunk of markers is first listed by
+// its rank among the markers of one stencil origin: 64 consecutive entries
+// then nearly always have 64 different origins.  What a marker needs (its
+// three offsets inside a cell, its scaled force) waits in LDS meanwhile, so
+// that memory is read once, in the bin order.  One component per block gives
+// three times the blocks where bricks are few, and four blocks per CU where
+// they are many; the short code (the planes of the stencil in a loop) matters
+// where a block runs once, since most of 35 us on a 32^3 grid with 2562
+// markers went into fetching straight-line code for three components and both
+// conversions.  Measured in us, C4 channel with 2.39 M markers / that sphere /
+// 64 boxes of 32^3 with 0.26 M markers: three components per block in bin order
+// 398 / 28 / 188; listed by rank and origin, per component 458 / 20 / 133; by
+// rank alone 384 to 399 / 17.5 / 94.
+constexpr int CHUNK_MARKERS = 512, ORIGINS = 9 * 9 * 9, THREAD_MARKERS = CHUNK_MARKERS / TILE_THREADS;
+
+__global__ void __launch_bounds__(TILE_THREADS, 4)
+tile_spread_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, int delta, const int* __restrict__ start,
+                   const int* __restrict__ perm, const tile_scale* __restrict__ scale,
+                   unsigned long long* __restrict__ tiles, int* __restrict__ flags, int blocks, int chunk)
+{
+    __shared__ __attribute__((aligned(16))) unsigned long long acc[TILE_PTS];
+    __shared__ __attribute__((aligned(16))) double2 offsets01[CHUNK_MARKERS], offset2_force[CHUNK_MARKERS];
+    __shared__ int count[ORIGINS];
+    __shared__ int level[64];                                // markers of rank r (63: and beyond)
+    __shared__ unsigned short order[CHUNK_MARKERS];
+    __shared__ unsigned short corner[CHUNK_MARKERS];         // tile index of a marker's stencil origin
+    // XCD x takes the x-th eighth: a brick's components share its L2's markers
+    const int block = (int) (blockIdx.x & 7) * chunk + (int) (blockIdx.x >> 3);
+    if ((int) (blockIdx.x >> 3) >= chunk || block >= blocks) return;
+    const int brick = block / 3, c = block - 3 * brick;
+    const int s0 = start[(size_t) brick * SUB];
+    const int s1 = start[(size_t) (brick + 1) * SUB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (s1 == s0) {
-        if (tid == 0) flags[brick] = 0;
+        if (tid == 0 && c == 0) flags[brick] = 0;
         return;                                      // whole block
     }
-    for (int i = tid; i < 3 * TILE_PTS; i += TILE_THREADS) (&acc[0][0])[i] = 0ull;
-    int r = brick % td.bricks;
-    int b0 = r % td.nbr[0];
-    int b1 = (r / td.nbr[0]) % td.nbr[1];
-    int b2 = r / (td.nbr[0] * td.nbr[1]);
+    for (int i = tid; i < TILE_PTS; i += TILE_THREADS) acc[i] = 0ull;
+    const int r = brick % td.bricks;
+    const int b0 = r % td.nbr[0];
+    const int b1 = (r / td.nbr[0]) % td.nbr[1];
+    const int b2 = r / (td.nbr[0] * td.nbr[1]);
     const int bq[3] = {b0 * TB, b1 * TB, b2 * TB};
+    // The quantum's inverse is a power of two: applied to the force first, it
+    // scales every product exactly as it would scale the finished one (a
+    // product that ends at 1/2 or more has no subnormal factor on the way).
     const double inv_q = scale->inv_q;
-    __syncthreads();
-    // Markers are sorted by bin, so neighbours in the sorted order often
-    // share a stencil origin, and lanes of one LDS atomic that hit the same
-    // address serialise.  Lane l of every wave therefore walks its own
-    // segment [l seg, (l + 1) seg) of the brick's markers (the waves
-    // interleaved in it): the lanes of one instruction are seg markers apart.
-    const int nm = s1 - s0, seg = (nm + 63) / 64, lane = tid & 63;
-    for (int r = tid >> 6; r < seg; r += TILE_THREADS / 64) {
-        const int li = lane * seg + r;
-        if (li >= nm) continue;
-        const int i = s0 + li;
-        const double2* rec = (const double2*) (sorted + (size_t) 6 * i);
-        const double2 r0 = rec[0], r1 = rec[1], r2 = rec[2];
-        const double p[3] = {r0.x, r0.y, r1.x}, fv[3] = {r1.y, r2.x, r2.y};
-        // bin coordinates of the marker (relative to its brick), as binned
-        int lq[3];
+    // values of a force below this (in quanta) stay below 2^51: see make_scale
+    const double fast_below = 0x1p51 / (delta == IBM_DELTA_BSPLINE3 ? 0.3 : 0.126);
+    const double force_scale = g.res3[c] * inv_q;
+#pragma unroll 1
+    for (int c0 = s0; c0 < s1; c0 += CHUNK_MARKERS) {
+        const int n = min(s1 - c0, CHUNK_MARKERS);
+        double p[THREAD_MARKERS][3], f[THREAD_MARKERS];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            stencil_axis st = kstencil(g.a[bd.fc[j]][j], p[j]);
-            int qb = st.base + bd.fs[j] - bd.qmin[j];
-            qb = qb < 0 ? 0 : (qb >= bd.nb[j] ? bd.nb[j] - 1 : qb);
-            lq[j] = qb - bq[j];
+        for (int k = 0; k < THREAD_MARKERS; ++k) {
+            const int m = perm[c0 + min(tid + k * TILE_THREADS, n - 1)];
+            load_marker(sets, m, p[k]);
+            f[k] = load_force(sets, m, c);
         }
+        for (int i = tid; i < ORIGINS; i += TILE_THREADS) count[i] = 0;
+        if (tid < 64) level[tid] = 0;
+        __syncthreads();
+        int at[THREAD_MARKERS];                              // rank and place among its markers, or -1
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            double w[3][4];
+        for (int k = 0; k < THREAD_MARKERS; ++k) {
+            const int i = tid + k * TILE_THREADS;
             int o[3];
+            double d[3];
+            bool on = i < n;
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const kaxis& a = g.a[c][j];
-                stencil_axis st = kstencil(a, p[j]);
-                delta4(delta, st.d, w[j]);
+                const int q = kstencil(g.a[bd.fc[j]][j], p[k][j]).base + bd.fs[j];
+                int qb = q - bd.qmin[j];
+                qb = qb < 0 ? 0 : (qb >= bd.nb[j] ? bd.nb[j] - 1 : qb);
+                const stencil_axis st = kstencil(a, p[k][j]);
                 // base_c - q, unwrapped across a periodic seam
-                stencil_axis fq = kstencil(g.a[bd.fc[j]][j], p[j]);
-                int d = st.base - (fq.base + bd.fs[j]);
+                int s = st.base - q;
                 if (!a.solid) {
-                    if (d > 2) d -= a.cells;
-                    else if (d < -3) d += a.cells;
+                    if (s > 2) s -= a.cells;
+                    else if (s < -3) s += a.cells;
                 }
-                o[j] = lq[j] + d - bd.lo[j];
+                o[j] = qb - bq[j] + s - bd.lo[j];
+                d[j] = st.d;
+                // A marker outside a walled axis's range (clamped by the
+                // index policy) can have an origin off the tile: its points
+                // lie outside the grid, which drops them, so it is skipped.
+                on = on && o[j] >= 0 && o[j] <= TT - 4;
             }
-            // A marker outside a walled axis's range (clamped by the index
-            // policy) can have an origin off the tile: its points lie outside
-            // the grid, which drops them, so it is skipped.
-            if (o[0] < 0 || o[0] > TT - 4 || o[1] < 0 || o[1] > TT - 4 || o[2] < 0 || o[2] > TT - 4) continue;
-            // The quantum's inverse is a power of two: applied to the force
-            // first, it scales every product exactly as it would scale the
-            // finished one (a product that ends at 1/2 or more has no
-            // subnormal factor on the way), one multiplication fewer per value.
-            const double fcq = fv[c] * g.res3[c] * inv_q;
-            unsigned long long* t = acc[c];
-#pragma unroll
-            for (int sz = 0; sz < 4; ++sz) {
-#pragma unroll
-                for (int sy = 0; sy < 4; ++sy) {
-                    const double wyz = w[2][sz] * (w[1][sy] * fcq);
-                    const int row = o[0] + TT * ((o[1] + sy) + TT * (o[2] + sz));
-#pragma unroll
-                    for (int sx = 0; sx < 4; ++sx)
-                        atomicAdd(&t[row + sx], (unsigned long long) __double2ll_rn(w[0][sx] * wyz));
-                }
+            at[k] = -1;
+            if (on) {
+                const int rank = min(atomicAdd(&count[o[0] + 9 * (o[1] + 9 * o[2])], 1), 63);
+                at[k] = rank << 16 | atomicAdd(&level[rank], 1);
+                offsets01[i] = make_double2(d[0], d[1]);
+                offset2_force[i] = make_double2(d[2], f[k] * force_scale);
+                corner[i] = (unsigned short) (o[0] + TT * (o[1] + TT * o[2]));
             }
         }
+        __syncthreads();
+        // list of the markers by rank
+        const int members = level[lane];
+        int incl = members;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += y;
+        }
+        const int listed = __shfl(incl, 63, 64);
+#pragma unroll
+        for (int k = 0; k < THREAD_MARKERS; ++k) {
+            const int to = __shfl(incl - members, at[k] >= 0 ? at[k] >> 16 : 0, 64) + (at[k] & 0xffff);
+            if (at[k] >= 0) order[to] = (unsigned short) (tid + k * TILE_THREADS);
+        }
+        __syncthreads();
+        for (int i0 = wave * 64; i0 < listed; i0 += TILE_THREADS) {
+            if (i0 + lane >= listed) continue;
+            const int i = order[i0 + lane];
+            const double2 d01 = offsets01[i], d2f = offset2_force[i];
+            double wx[4], wy[4], wz[4];
+            delta4(delta, d01.x, wx);
+            delta4(delta, d01.y, wy);
+            delta4(delta, d2f.x, wz);
+            unsigned long long* t = acc + corner[i];
+            if (fabs(d2f.y) < fast_below) add_stencil<true>(t, wx, wy, wz, d2f.y);
+            else add_stencil<false>(t, wx, wy, wz, d2f.y);
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    unsigned long long* dst = tiles + (size_t) brick * 3 * TILE_PTS;
-    for (int i = tid; i < 3 * TILE_PTS; i += TILE_THREADS) dst[i] = (&acc[0][0])[i];
-    if (tid == 0) flags[brick] = 1;
+    ulonglong2* dst = (ulonglong2*) (tiles + ((size_t) brick * 3 + c) * TILE_PTS);
+    for (int i = tid; i < TILE_PTS / 2; i += TILE_THREADS) dst[i] = ((const ulonglong2*) acc)[i];
+    if (tid == 0 && c == 0) flags[brick] = 1;
 }
 
 // Every grid point of every box and component: the sum of the tile entries
-// that cover it, times the quantum.  Block (row, x chunk, box * 3 + c) takes
-// MERGE_THREADS points of one x-row (row = y + points_y z) of component c's
-// grid, so the y and z coverage is the same for the whole block.
-constexpr int MERGE_THREADS = 128;
+// that cover it, times the quantum.  HBM-bound in its traffic (3.4 entries a
+// point), latency-bound if the entries are loaded one after another: all of a
+// thread's flags are loaded first, then all its entries, absent ones from the
+// first entry's address.  A thread takes one point of one component
+// (consecutive threads consecutive points, whatever the row length: a block
+// per grid row left 96 of its 128 threads idle on boxes of 32 cells), XCD x
+// the x-th eighth of them, so that rows that share tiles share an L2.
+//
+// Per axis a point is covered by the tiles b with 8 b + t = v, t < 12, v its
+// distance from the first tile's start: on walled axes one v, on periodic
+// ones every v = rel + k cells up to the last tile's end.  Walls and whole
+// bricks (WHOLE) leave at most two tiles: b = v / 8 and, for the first four
+// points of a brick, the one before it (the last one before the first).
+// Other periodic axes have up to six: those grids loop over them.
+constexpr int MERGE_THREADS = 256;
 
-__global__ void __launch_bounds__(MERGE_THREADS)
-tile_merge_kernel(kgrids g, bin_desc bd, tile_desc td, int box0, const unsigned long long* __restrict__ tiles,
-                  const int* __restrict__ flags, const tile_scale* __restrict__ scale, double* __restrict__ fe0,
-                  double* __restrict__ fe1, double* __restrict__ fe2)
+struct cover {
+    int rel, cells, nbr, solid;
+};
+
+template <typename F>
+__device__ inline void visit(const cover& a, F&& f)
 {
-    const int bz = blockIdx.z / 3, c = blockIdx.z - 3 * bz, box = box0 + bz;
-    const int* pt = g.points[c];
-    const int row = blockIdx.x;
-    const int x = blockIdx.y * MERGE_THREADS + threadIdx.x;
-    if (row >= pt[1] * pt[2] || x >= pt[0]) return;
-    const int pp[3] = {x, row % pt[1], row / pt[1]};
-    // per axis: up to two (brick, tile index) pairs covering the point
-    int nb_c[3], bb[3][2], tt[3][2];
+    for (int v = a.rel; v < (a.nbr - 1) * TB + TT; v += a.cells) {
+        if (v >= 0) {
+            const int b = v / TB, t = v - b * TB;
+            if (b < a.nbr) f(b, t);
+            if (b > 0 && b - 1 < a.nbr && t + TB < TT) f(b - 1, t + TB);
+        }
+        if (a.solid) break;
+    }
+}
+
+template <bool WHOLE>
+__global__ void __launch_bounds__(MERGE_THREADS)
+tile_merge_kernel(kgrids g, bin_desc bd, tile_desc td, int box0, unsigned chunk,
+                  const unsigned long long* __restrict__ tiles, const int* __restrict__ flags,
+                  const tile_scale* __restrict__ scale, double* __restrict__ fe0, double* __restrict__ fe1,
+                  double* __restrict__ fe2)
+{
+    const int bz = blockIdx.y / 3, c = blockIdx.y - 3 * bz, box = box0 + bz;
+    const unsigned block = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
+    const unsigned at = block * MERGE_THREADS + threadIdx.x;
+    if (at >= (unsigned) td.box_points[c]) return;
+    const unsigned n0 = g.points[c][0], n1 = g.points[c][1];
+    const unsigned row = at / n0, z = row / n1;
+    const int pp[3] = {(int) (at - row * n0), (int) (row - z * n1), (int) z};
+    cover cv[3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         const kaxis& a = g.a[c][j];
-        const int t0 = bd.qmin[j] + bd.lo[j] - 1;        // first tile point of brick 0
-        int rel = pp[j] - t0;
-        int cnt = 0;
-        if (!a.solid) {
-            // periodic: cells is a multiple of the brick edge here
-            rel %= a.cells;
-            if (rel < 0) rel += a.cells;
-            const int b = rel / TB, t = rel - b * TB;
-            bb[j][cnt] = b; tt[j][cnt] = t; ++cnt;
-            if (t + TB < TT) {
-                bb[j][cnt] = b - 1 < 0 ? td.nbr[j] - 1 : b - 1; tt[j][cnt] = t + TB; ++cnt;
-            }
-        } else {
-            const int b = rel >= 0 ? rel / TB : -1;
-            const int t = rel - b * TB;
-            if (b >= 0 && b < td.nbr[j]) { bb[j][cnt] = b; tt[j][cnt] = t; ++cnt; }
-            if (b - 1 >= 0 && b - 1 < td.nbr[j] && t + TB < TT) { bb[j][cnt] = b - 1; tt[j][cnt] = t + TB; ++cnt; }
-        }
-        nb_c[j] = cnt;
+        int rel = pp[j] - (bd.qmin[j] + bd.lo[j] - 1);       // from the first tile point of brick 0
+        if (!a.solid) rel = rel < 0 ? rel + a.cells : (rel >= a.cells ? rel - a.cells : rel);
+        cv[j] = cover{rel, a.cells, td.nbr[j], a.solid};
     }
     long long sum = 0;
-    for (int iz = 0; iz < nb_c[2]; ++iz)
-        for (int iy = 0; iy < nb_c[1]; ++iy)
-            for (int ix = 0; ix < nb_c[0]; ++ix) {
-                const int brick = ((box * td.nbr[2] + bb[2][iz]) * td.nbr[1] + bb[1][iy]) * td.nbr[0] + bb[0][ix];
-                if (!flags[brick]) continue;
-                const size_t at = ((size_t) brick * 3 + c) * TILE_PTS + tt[0][ix] + TT * (tt[1][iy] + TT * tt[2][iz]);
-                sum += (long long) tiles[at];
-            }
+    if (WHOLE) {
+        int b[3][2], t[3][2];
+        bool ok[3][2];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int v = cv[j].rel < 0 ? 0 : cv[j].rel, b0 = v / TB, t0 = v - b0 * TB;
+            b[j][0] = b0;
+            t[j][0] = t0;
+            ok[j][0] = cv[j].rel >= 0 && b0 < cv[j].nbr;
+            b[j][1] = b0 > 0 ? b0 - 1 : (cv[j].solid ? 0 : cv[j].nbr - 1);
+            t[j][1] = t0 + TB;
+            ok[j][1] = cv[j].rel >= 0 && t0 + TB < TT && b[j][1] < cv[j].nbr && (b0 > 0 || !cv[j].solid);
+        }
+        unsigned brick[8];
+        bool has[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int x = k & 1, y = k >> 1 & 1, w = k >> 2;
+            has[k] = ok[0][x] && ok[1][y] && ok[2][w];
+            brick[k] = ((unsigned) (box * td.nbr[2] + b[2][w]) * td.nbr[1] + b[1][y]) * td.nbr[0] + b[0][x];
+            brick[k] = has[k] ? brick[k] : 0u;
+        }
+        int fl[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) fl[k] = flags[brick[k]];
+        unsigned long long e[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int x = k & 1, y = k >> 1 & 1, w = k >> 2;
+            has[k] = has[k] && fl[k];
+            const size_t i = ((size_t) brick[k] * 3 + c) * TILE_PTS + t[0][x] + TT * (t[1][y] + TT * t[2][w]);
+            e[k] = tiles[has[k] ? i : (size_t) 0];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum += has[k] ? (long long) e[k] : 0ll;
+    } else {
+        visit(cv[2], [&](int b2, int t2) {
+            visit(cv[1], [&](int b1, int t1) {
+                const unsigned brick_row = ((unsigned) (box * td.nbr[2] + b2) * td.nbr[1] + b1) * td.nbr[0];
+                const unsigned tile_row = TT * (t1 + TT * t2);
+                visit(cv[0], [&](int b0, int t0) {
+                    const unsigned brick = brick_row + b0;
+                    if (flags[brick]) sum += (long long) tiles[((size_t) brick * 3 + c) * TILE_PTS + tile_row + t0];
+                });
+            });
+        });
+    }
     double* fe = c == 0 ? fe0 : (c == 1 ? fe1 : fe2);
-    fe[(size_t) box * td.box_points[c] + (size_t) pt[0] * row + x] = (double) sum * scale->q;
+    fe[(size_t) box * td.box_points[c] + at] = (double) sum * scale->q;
 }
 
 // Interpolation over boxes: one lane per marker, grid vectors of box b at
@@ -1368,39 +1653,80 @@ interp_boxes_kernel(marker_sets sets, kgrids g, int delta, const int* __restrict
 
 } // namespace
 
-// Resolves the device address of `scratch` on `device` (made current by the
-// caller) once per device; ibm_create calls it.
+// Allocates the fixed workspace of `device` (made current by the caller) once
+// per device; ibm_create calls it.  (As a __device__ array the loader fills it
+// from the host, 73 ms in the first ibm_create of a process instead of 1.)
 ibm_status static_scratch_init(ibm_ctx* ctx, int device)
 {
     if (device < 0 || device >= STATIC_MAX_DEVICES)
         return fail(ctx, IBM_ERR_ARG, "device %d beyond the fixed-workspace table", device);
     std::lock_guard<std::mutex> lock(static_scratch_mutex);
-    if (static_scratch_ptr[device]) return IBM_OK;
-    void* p = nullptr;
-    IBM_HIP(ctx, hipGetSymbolAddress(&p, HIP_SYMBOL(::scratch)));
-    if (!p) return fail(ctx, IBM_ERR_HIP, "hipGetSymbolAddress returned a null workspace address");
-    static_scratch_ptr[device] = p;
+    if (!static_scratch_ptr[device]) IBM_HIP(ctx, hipMalloc(&static_scratch_ptr[device], STATIC_SCRATCH_BYTES));
     return IBM_OK;
 }
 
-ibm_status spread_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const marker_sets& sets,
-                       double* const* fe, unsigned char* fixed_workspace = nullptr)
+// Checked inputs of a spread and its bins.
+ibm_status spread_setup(ibm_ctx* ctx, const ibm_grid* grids, int delta, double* const* fe, kgrids* kg, bin_desc* bd)
 {
-    kgrids kg;
-    IBM_TRY(make_kgrids(ctx, grids, &kg));
+    IBM_TRY(make_kgrids(ctx, grids, kg));
     IBM_TRY(check_delta(ctx, delta));
     if (!fe || !fe[0] || !fe[1] || !fe[2]) return fail(ctx, IBM_ERR_ARG, "null output grid");
     for (int c = 0; c < 3; ++c)
         for (int j = 0; j < 3; ++j)
-            if (!kg.a[c][j].solid && kg.a[c][j].cells < 4)
+            if (!kg->a[c][j].solid && kg->a[c][j].cells < 4)
                 return fail(ctx, IBM_ERR_BAD_GRID, "periodic dimension needs at least 4 cells for a 4-point stencil");
-    bin_desc bd = make_bins(grids);
-    if (bd.nbins <= 0) return fail(ctx, IBM_ERR_SIZE, "too many grid bins");
+    *bd = make_bins(grids);
+    if (bd->nbins <= 0) return fail(ctx, IBM_ERR_SIZE, "too many grid bins");
     for (int j = 0; j < 3; ++j)
-        if (bd.hi[j] - bd.lo[j] > 1 || bd.hi[j] < bd.lo[j])
+        if (bd->hi[j] - bd->lo[j] > 1 || bd->hi[j] < bd->lo[j])
             return fail(ctx, IBM_ERR_BAD_GRID, "component grids are not a staggering of one cell grid");
+    return IBM_OK;
+}
+
+// Component j alone differs along axis j.
+bool mac_shaped(const kgrids& kg)
+{
+    for (int c = 0; c < 3; ++c)
+        for (int j = 0; j < 3; ++j)
+            if (kg.sel[c][j] != (c == j ? 1 : 0) || kg.cand[1][j] != j || kg.cand[0][j] == j) return false;
+    return true;
+}
+
+// Every periodic axis long enough for the brick kernel's division-free wrap.
+bool wide_axes(const kgrids& kg)
+{
+    for (int c = 0; c < 3; ++c)
+        for (int j = 0; j < 3; ++j)
+            if (!kg.a[c][j].solid && kg.a[c][j].cells < MIN_FAST_CELLS) return false;
+    return true;
+}
+
+// The general wrap of the brick kernel packs point indices into 10 bits; the
+// entry points refuse such grids whichever path takes the call.
+ibm_status narrow_axes_limit(ibm_ctx* ctx, const kgrids& kg)
+{
+    if (wide_axes(kg)) return IBM_OK;
+    for (int c = 0; c < 3; ++c)
+        for (int j = 0; j < 3; ++j)
+            if (kg.a[c][j].points > 1022)
+                return fail(ctx, IBM_ERR_SIZE, "small periodic axes with more than 1022 points on another axis");
+    return IBM_OK;
+}
+
+bool whole_bricks(const kgrids& kg)
+{
+    for (int c = 0; c < 3; ++c)
+        for (int j = 0; j < 3; ++j)
+            if (!kg.a[c][j].solid && kg.a[c][j].cells % TB != 0) return false;
+    return true;
+}
+
+// The brick kernel's spread.
+ibm_status spread_bricks(ibm_ctx* ctx, const kgrids& kg, const bin_desc& bd, int delta, const marker_sets& sets,
+                         double* const* fe, unsigned char* fixed_workspace)
+{
     bin_work w;
-    if (fixed_workspace) IBM_TRY(static_bin_work(ctx, fixed_workspace, sets.total, bd.nbins, &w));
+    if (fixed_workspace) IBM_TRY(static_bin_work(ctx, fixed_workspace, bd.nbins, &w));
     else IBM_TRY(ctx_bin_work(ctx, sets.total, bd.nbins, &w));
     IBM_TRY(bin_markers(ctx, sets, kg, bd, 1, w, fixed_workspace == nullptr));
     int maxp[3] = {0, 0, 0};
@@ -1410,17 +1736,7 @@ ibm_status spread_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const mar
     long long nbricks = (long long) bx * by * bz;
     if (nbricks > 0x7fffffff) return fail(ctx, IBM_ERR_SIZE, "grid too large");
     int xcd_chunk = (nbricks % 8 == 0) ? (int) (nbricks / 8) : 0;
-    bool mac = true, fast = true;
-    for (int c = 0; c < 3; ++c)
-        for (int j = 0; j < 3; ++j) {
-            if (kg.sel[c][j] != (c == j ? 1 : 0) || kg.cand[1][j] != j || kg.cand[0][j] == j) mac = false;
-            if (!kg.a[c][j].solid && kg.a[c][j].cells < MIN_FAST_CELLS) fast = false;
-        }
-    if (!fast)
-        for (int c = 0; c < 3; ++c)
-            for (int j = 0; j < 3; ++j)
-                if (kg.a[c][j].points > 1022)
-                    return fail(ctx, IBM_ERR_SIZE, "small periodic axes with more than 1022 points on another axis");
+    const bool mac = mac_shaped(kg), fast = wide_axes(kg);
     double grid_points = 0;
     for (int c = 0; c < 3; ++c) grid_points += (double) kg.points[c][0] * kg.points[c][1] * kg.points[c][2];
     // positions + forces read once, three grids written once
@@ -1438,6 +1754,190 @@ ibm_status spread_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const mar
     return IBM_OK;
 }
 
+// Bricks of one box, and whether every brick's tiles of nboxes boxes may be
+// held (16 GiB) and numbered.
+long long bricks_of(const bin_desc& bd)
+{
+    long long n = 1;
+    for (int j = 0; j < 3; ++j) n *= (bd.nb[j] + TB - 1) / TB;
+    return n;
+}
+
+constexpr long long TILE_MAX_BYTES = 1ll << 34;
+bool tiles_fit(const bin_desc& bd, int nboxes)
+{
+    const long long bricks = bricks_of(bd);
+    return bricks <= TILE_MAX_BYTES / (long long) TILE_BYTES / nboxes && bricks * nboxes * SUB <= INT_MAX - 1;
+}
+
+// Spread of the markers of nboxes boxes (box b: markers [off[b], off[b+1])
+// of the sets' concatenation, off on the device) into nboxes consecutive
+// copies of each component grid, by bricks and tiles.
+ibm_status spread_tiles(ibm_ctx* ctx, const kgrids& kg, const bin_desc& bd, int delta, const marker_sets& sets, int nboxes,
+                        const int* box_off, double* const* fe, unsigned char* fixed_workspace)
+{
+    tile_desc td{};
+    int reach = 1;
+    for (int j = 0; j < 3; ++j) {
+        const kaxis& a = kg.a[bd.fc[j]][j];
+        td.nbr[j] = (bd.nb[j] + TB - 1) / TB;
+        reach *= !a.solid && a.cells % 4 != 0 ? 3 : 2;
+    }
+    td.bricks = (int) bricks_of(bd);
+    td.nboxes = nboxes;
+    td.keys = td.bricks * nboxes * SUB;
+    double grid_points = 0;
+    unsigned most = 0;
+    for (int c = 0; c < 3; ++c) {
+        td.box_points[c] = kg.points[c][0] * kg.points[c][1] * kg.points[c][2];
+        most = std::max(most, (unsigned) td.box_points[c]);
+        grid_points += (double) td.box_points[c] * nboxes;
+    }
+    const size_t nbricks = (size_t) td.bricks * nboxes, total = (size_t) sets.total;
+    const size_t key_words = sizeof(int) * ((size_t) td.keys + 1);
+    int *count, *start, *key, *rank, *perm, *flags;
+    bin_stats* stats;
+    tile_scale* sc;
+    unsigned long long* tiles;
+    void *p, *scan_tmp = nullptr;
+    size_t scan_bytes = 0;
+    if (fixed_workspace) {
+        size_t off = 0;
+        auto take = [&](size_t bytes) { unsigned char* q = fixed_workspace + off; off += align256(bytes); return q; };
+        count = (int*) take(key_words);
+        start = (int*) take(key_words);
+        key = (int*) take(sizeof(int) * total);
+        rank = (int*) take(sizeof(int) * total);
+        perm = (int*) take(sizeof(int) * total);
+        stats = (bin_stats*) take(STATIC_STATS_BYTES);
+        sc = (tile_scale*) take(sizeof(tile_scale));
+        flags = (int*) take(sizeof(int) * nbricks);
+        tiles = (unsigned long long*) take(TILE_BYTES * nbricks);
+    } else {
+        IBM_TRY(scratch(ctx, SLOT_BIN_COUNT, key_words, &p)); count = (int*) p;
+        IBM_TRY(scratch(ctx, SLOT_BIN_START, key_words, &p)); start = (int*) p;
+        IBM_TRY(scratch(ctx, SLOT_KEY, sizeof(int) * total, &p)); key = (int*) p;
+        IBM_TRY(scratch(ctx, SLOT_RANK, sizeof(int) * total, &p)); rank = (int*) p;
+        IBM_TRY(scratch(ctx, SLOT_PERM, sizeof(int) * total, &p)); perm = (int*) p;
+        IBM_TRY(scratch(ctx, SLOT_FLAGS, sizeof(bin_stats), &p)); stats = (bin_stats*) p;
+        IBM_TRY(scratch(ctx, SLOT_TILES, TILE_BYTES * nbricks, &p)); tiles = (unsigned long long*) p;
+        IBM_TRY(scratch(ctx, SLOT_TILE_FLAGS, align256(sizeof(tile_scale)) + sizeof(int) * nbricks, &p));
+        sc = (tile_scale*) p;
+        flags = (int*) ((unsigned char*) p + align256(sizeof(tile_scale)));
+        if (td.keys > SCAN_MAX) {
+            IBM_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, count, start, td.keys + 1, ctx->stream));
+            IBM_TRY(scratch(ctx, SLOT_SCAN_TMP, scan_bytes, &scan_tmp));
+        }
+    }
+    const bool timed = fixed_workspace == nullptr;
+    {
+        prof_scope prof(ctx, timed ? "bin" : nullptr);
+        tile_clear_kernel<<<blocks_for((long long) td.keys + 1, 256), 256, 0, ctx->stream>>>(count, td.keys, stats);
+        IBM_LAUNCH_CHECK(ctx);
+        if (total > 0) {
+            tile_count_kernel<<<blocks_for(sets.total, 256 * COUNT_ITEMS), 256, 0, ctx->stream>>>(
+                sets, kg, bd, td, box_off, key, rank, count, stats);
+            IBM_LAUNCH_CHECK(ctx);
+        }
+        if (td.keys <= SCAN_MAX) {
+            tile_scan_kernel<<<1, SCAN_THREADS, 0, ctx->stream>>>(kg, delta, reach, count, td.keys, stats, start, sc);
+            IBM_LAUNCH_CHECK(ctx);
+        } else {
+            IBM_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(scan_tmp, scan_bytes, count, start, td.keys + 1, ctx->stream));
+            tile_max_kernel<<<std::min(blocks_for(td.keys, 256), 1024), 256, 0, ctx->stream>>>(count, td.keys, stats);
+            IBM_LAUNCH_CHECK(ctx);
+            tile_scale_kernel<<<1, 64, 0, ctx->stream>>>(kg, delta, reach, stats, sc);
+            IBM_LAUNCH_CHECK(ctx);
+        }
+        if (total > 0) {
+            tile_place_kernel<<<blocks_for(sets.total, 256), 256, 0, ctx->stream>>>(sets.total, key, rank, start, perm);
+            IBM_LAUNCH_CHECK(ctx);
+        }
+    }
+    {
+        prof_scope prof(ctx, timed ? "spread_tile" : nullptr, 48.0 * sets.total);
+        const int blocks = (int) nbricks * 3, chunk = (blocks + 7) / 8;
+        tile_spread_kernel<<<(unsigned) (8 * chunk), TILE_THREADS, 0, ctx->stream>>>(sets, kg, bd, td, delta, start, perm, sc,
+                                                                                     tiles, flags, blocks, chunk);
+        IBM_LAUNCH_CHECK(ctx);
+    }
+    {
+        prof_scope prof(ctx, timed ? "spread_merge" : nullptr, 8.0 * grid_points);
+        bool whole = true;
+        for (int c = 0; c < 3; ++c)
+            for (int j = 0; j < 3; ++j) whole = whole && (kg.a[c][j].solid || kg.a[c][j].cells % TB == 0);
+        const unsigned blocks = (most + MERGE_THREADS - 1) / MERGE_THREADS, chunk = (blocks + 7) / 8;
+        constexpr int BOXES_PER_LAUNCH = 65535 / 3;
+        for (int b0 = 0; most > 0 && b0 < nboxes; b0 += BOXES_PER_LAUNCH) {
+            const int nb = std::min(BOXES_PER_LAUNCH, nboxes - b0);
+            const dim3 grid(8 * chunk, (unsigned) (3 * nb));
+            if (whole)
+                tile_merge_kernel<true><<<grid, MERGE_THREADS, 0, ctx->stream>>>(kg, bd, td, b0, chunk, tiles, flags, sc,
+                                                                                 fe[0], fe[1], fe[2]);
+            else
+                tile_merge_kernel<false><<<grid, MERGE_THREADS, 0, ctx->stream>>>(kg, bd, td, b0, chunk, tiles, flags, sc,
+                                                                                  fe[0], fe[1], fe[2]);
+            IBM_LAUNCH_CHECK(ctx);
+        }
+    }
+    return IBM_OK;
+}
+
+// The public spread.  ibm_spread_sets and ibm_spread_sets_noalloc give the
+// same bits, so the path depends on the markers and grids alone: tiles where
+// a brick's tiles for the whole grid fit the fixed workspace, or where the
+// input is beyond what the fixed workspace takes at all; else (grids of few
+// bins and many mostly empty bricks) the brick kernel.  Measured (us, brick
+// kernel / tiles, binning included): C4 channel with 2.39 M markers 1802 /
+// 580, 100^3 periodic with 176,000 markers 268 / 120, one sphere of 2562
+// markers on 32^3 89 / 41.
+ibm_status spread_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const marker_sets& sets,
+                       double* const* fe, unsigned char* fixed_workspace = nullptr)
+{
+    kgrids kg;
+    bin_desc bd;
+    IBM_TRY(spread_setup(ctx, grids, delta, fe, &kg, &bd));
+    if (fixed_workspace) IBM_TRY(static_limits(ctx, sets.total, bd.nbins));
+    IBM_TRY(narrow_axes_limit(ctx, kg));
+    const bool beyond = (size_t) sets.total > STATIC_MAX_MARKERS || (size_t) bd.nbins > STATIC_MAX_BINS;
+    if (bricks_of(bd) <= (long long) STATIC_MAX_BRICKS || (beyond && tiles_fit(bd, 1)))
+        return spread_tiles(ctx, kg, bd, delta, sets, 1, nullptr, fe, fixed_workspace);
+    return spread_bricks(ctx, kg, bd, delta, sets, fe, fixed_workspace);
+}
+
+// The timestep's spread of several marker sets: by tiles wherever they fit.
+ibm_status spread_sets_step(ibm_ctx* ctx, const ibm_grid* grids, int delta, int nsets, const int* n,
+                            const double* const* x, const double* const* f, double* const* fe)
+{
+    marker_sets s;
+    IBM_TRY(make_sets(ctx, nsets, n, x, f, nullptr, &s));
+    kgrids kg;
+    bin_desc bd;
+    IBM_TRY(spread_setup(ctx, grids, delta, fe, &kg, &bd));
+    const bool fit = tiles_fit(bd, 1);
+    if (!fit || !whole_bricks(kg)) IBM_TRY(narrow_axes_limit(ctx, kg));
+    if (fit) return spread_tiles(ctx, kg, bd, delta, s, 1, nullptr, fe, nullptr);
+    return spread_bricks(ctx, kg, bd, delta, s, fe, nullptr);
+}
+
+// ibm_spread_boxes' grids: every periodic axis a multiple of the brick edge.
+ibm_status spread_boxes(ibm_ctx* ctx, const ibm_grid* grids, int delta, const marker_sets& sets, int nboxes,
+                        const int* box_off, double* const* fe)
+{
+    kgrids kg;
+    bin_desc bd;
+    IBM_TRY(make_kgrids(ctx, grids, &kg));
+    if (!whole_bricks(kg))
+        return fail(ctx, IBM_ERR_BAD_GRID, "batched spreading needs periodic axes of a multiple of %d cells", TB);
+    IBM_TRY(spread_setup(ctx, grids, delta, fe, &kg, &bd));
+    for (int c = 0; c < 3; ++c)
+        if (kg.points[c][0] > 65535 * 128)
+            return fail(ctx, IBM_ERR_SIZE, "grid rows of %d points too long for the tile spread", kg.points[c][0]);
+    if (bricks_of(bd) * nboxes > (INT_MAX - 1) / SUB)
+        return fail(ctx, IBM_ERR_SIZE, "too many boxes or bins for one batched spread");
+    return spread_tiles(ctx, kg, bd, delta, sets, nboxes, box_off, fe, nullptr);
+}
+
 ibm_status interp_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const marker_sets& sets,
                        const double* const* ue)
 {
@@ -1452,133 +1952,6 @@ ibm_status interp_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const mar
     return IBM_OK;
 }
 
-
-// Whether the tile spread takes these grids: 3-dimensional, every periodic
-// axis a multiple of the brick edge (so bricks tile it exactly).
-bool tiles_fit(const kgrids& kg)
-{
-    for (int c = 0; c < 3; ++c)
-        for (int j = 0; j < 3; ++j)
-            if (!kg.a[c][j].solid && kg.a[c][j].cells % TB != 0) return false;
-    return true;
-}
-
-// Spread of the markers of nboxes boxes (box b: markers [off[b], off[b+1])
-// of the sets' concatenation, off on the device) into nboxes consecutive
-// copies of each component grid, by bricks and tiles.
-ibm_status spread_tiles(ibm_ctx* ctx, const ibm_grid* grids, int delta, const marker_sets& sets, int nboxes,
-                        const int* box_off, double* const* fe, bool timed)
-{
-    kgrids kg;
-    IBM_TRY(make_kgrids(ctx, grids, &kg));
-    IBM_TRY(check_delta(ctx, delta));
-    if (!fe || !fe[0] || !fe[1] || !fe[2]) return fail(ctx, IBM_ERR_ARG, "null output grid");
-    if (nboxes < 1) return fail(ctx, IBM_ERR_ARG, "at least one box");
-    if (!tiles_fit(kg))
-        return fail(ctx, IBM_ERR_BAD_GRID, "batched spreading needs periodic axes of a multiple of %d cells", TB);
-    bin_desc bd = make_bins(grids);
-    if (bd.nbins <= 0) return fail(ctx, IBM_ERR_SIZE, "too many grid bins");
-    for (int j = 0; j < 3; ++j)
-        if (bd.hi[j] - bd.lo[j] > 1 || bd.hi[j] < bd.lo[j])
-            return fail(ctx, IBM_ERR_BAD_GRID, "component grids are not a staggering of one cell grid");
-    tile_desc td{};
-    long long bricks = 1;
-    for (int j = 0; j < 3; ++j) {
-        td.nbr[j] = (bd.nb[j] + TB - 1) / TB;
-        bricks *= td.nbr[j];
-    }
-    long long keys = bricks * nboxes * (TB * TB * TB);
-    if (keys > INT_MAX - 1) return fail(ctx, IBM_ERR_SIZE, "too many boxes or bins for one batched spread");
-    td.bricks = (int) bricks;
-    td.nboxes = nboxes;
-    td.keys = (int) keys;
-    double grid_points = 0;
-    for (int c = 0; c < 3; ++c) {
-        td.box_points[c] = kg.points[c][0] * kg.points[c][1] * kg.points[c][2];
-        grid_points += (double) td.box_points[c] * nboxes;
-    }
-    bin_work w;
-    IBM_TRY(ctx_bin_work(ctx, sets.total, td.keys, &w));
-    void* p;
-    const size_t nbricks = (size_t) bricks * nboxes;
-    IBM_TRY(scratch(ctx, SLOT_TILES, sizeof(unsigned long long) * 3 * TILE_PTS * nbricks, &p));
-    unsigned long long* tiles = (unsigned long long*) p;
-    IBM_TRY(scratch(ctx, SLOT_TILE_FLAGS, sizeof(int) * nbricks + 256 + sizeof(tile_scale), &p));
-    int* flags = (int*) p;
-    tile_scale* sc = (tile_scale*) ((unsigned char*) p + ((sizeof(int) * nbricks + 255) / 256) * 256);
-    {
-        prof_scope prof(ctx, timed ? "bin" : nullptr);
-        size_t words = (size_t) td.keys + 1;
-        zero_words_kernel<<<blocks_for((long) std::min<size_t>(words, 1u << 22), 256), 256, 0, ctx->stream>>>(
-            (unsigned int*) w.count, words);
-        IBM_LAUNCH_CHECK(ctx);
-        zero_words_kernel<<<1, 256, 0, ctx->stream>>>((unsigned int*) w.stats, sizeof(bin_stats) / 4);
-        IBM_LAUNCH_CHECK(ctx);
-        if (sets.total > 0) {
-            tile_count_kernel<<<blocks_for(sets.total, 256), 256, 0, ctx->stream>>>(sets, kg, bd, td, box_off, w.key,
-                                                                                     w.rank, w.count, w.stats);
-            IBM_LAUNCH_CHECK(ctx);
-        }
-        size_t tbytes = w.scan_bytes;
-        IBM_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(w.scan_tmp, tbytes, w.count, w.start, td.keys + 1, ctx->stream));
-        if (sets.total > 0) {
-            tile_scatter_kernel<<<blocks_for(sets.total, 256), 256, 0, ctx->stream>>>(sets, w.key, w.rank, w.start,
-                                                                                       w.sorted, w.stats);
-            IBM_LAUNCH_CHECK(ctx);
-        }
-        tile_scale_kernel<<<1, 64, 0, ctx->stream>>>(kg, w.stats, sc);
-        IBM_LAUNCH_CHECK(ctx);
-    }
-    {
-        prof_scope prof(ctx, timed ? "spread_tile" : nullptr, 48.0 * sets.total);
-        tile_spread_kernel<<<(int) nbricks, TILE_THREADS, 0, ctx->stream>>>(kg, bd, td, delta, sets.total, w.start,
-                                                                            w.sorted, sc, tiles, flags);
-        IBM_LAUNCH_CHECK(ctx);
-    }
-    {
-        prof_scope prof(ctx, timed ? "spread_merge" : nullptr, 8.0 * grid_points);
-        int rows = 0, xs = 0;
-        for (int c = 0; c < 3; ++c) {
-            rows = std::max(rows, kg.points[c][1] * kg.points[c][2]);
-            xs = std::max(xs, kg.points[c][0]);
-        }
-        const int xchunks = (xs + MERGE_THREADS - 1) / MERGE_THREADS;
-        if (xchunks > 65535) return fail(ctx, IBM_ERR_SIZE, "grid rows of %d points too long for the tile spread", xs);
-        constexpr int BOXES_PER_LAUNCH = 65535 / 3;
-        for (int b0 = 0; rows > 0 && b0 < td.nboxes; b0 += BOXES_PER_LAUNCH) {
-            const int nb = std::min(BOXES_PER_LAUNCH, td.nboxes - b0);
-            const dim3 mgrid((unsigned) rows, (unsigned) xchunks, (unsigned) (3 * nb));
-            tile_merge_kernel<<<mgrid, MERGE_THREADS, 0, ctx->stream>>>(kg, bd, td, b0, tiles, flags, sc, fe[0], fe[1],
-                                                                         fe[2]);
-            IBM_LAUNCH_CHECK(ctx);
-        }
-    }
-    return IBM_OK;
-}
-
-// The timestep's spread of several marker sets: the tile spread where the
-// grids allow it (every periodic axis a multiple of the brick edge), else
-// the brick spread.  Both are deterministic; they differ in the last bits
-// (their fixed-point scales differ), so one solver always uses one of them.
-bool tiles_usable(ibm_ctx* ctx, const ibm_grid* grids)
-{
-    kgrids kg;
-    if (make_kgrids(ctx, grids, &kg) != IBM_OK || !tiles_fit(kg)) return false;
-    bin_desc bd = make_bins(grids);
-    if (bd.nbins <= 0) return false;
-    long long keys = TB * TB * TB;
-    for (int j = 0; j < 3; ++j) keys *= (bd.nb[j] + TB - 1) / TB;
-    return keys <= INT_MAX - 1;
-}
-
-ibm_status spread_sets_step(ibm_ctx* ctx, const ibm_grid* grids, int delta, bool tiles, int nsets, const int* n,
-                            const double* const* x, const double* const* f, double* const* fe)
-{
-    marker_sets s;
-    IBM_TRY(make_sets(ctx, nsets, n, x, f, nullptr, &s));
-    if (tiles) return spread_tiles(ctx, grids, delta, s, 1, nullptr, fe, true);   // one box: no offsets read
-    return spread_sets(ctx, grids, delta, s, fe);
-}
 
 // The box offsets (host, nboxes + 1) in the context's scratch.
 ibm_status upload_box_offsets(ibm_ctx* ctx, int nboxes, const int* offsets, int total, const int** dev)
@@ -1673,7 +2046,7 @@ ibm_status ibm_spread_boxes(ibm_ctx* ctx, const ibm_grid* grids, ibm_delta delta
     IBM_TRY(ibm::make_sets(ctx, 1, &n, &x, &f, nullptr, &s));
     const int* dev_off = nullptr;
     IBM_TRY(ibm::upload_box_offsets(ctx, nboxes, offsets, s.total, &dev_off));
-    return ibm::spread_tiles(ctx, grids, (int) delta, s, nboxes, dev_off, fe, true);
+    return ibm::spread_boxes(ctx, grids, (int) delta, s, nboxes, dev_off, fe);
 }
 
 ibm_status ibm_interpolate_boxes(ibm_ctx* ctx, const ibm_grid* grids, ibm_delta delta, int nboxes, const int* offsets,

@@ -176,7 +176,7 @@ ibm_status ibm_spread_sets(ibm_ctx* ctx, const ibm_grid* grids, ibm_delta delta,
  * reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * binning buffers live in a fixed per-device workspace of the library
- * (36.6 MB, held until the process ends) instead of the context's scratch,
+ * (184 MB, held until the process ends) instead of the context's scratch,
  * so at most 262,144 markers in total and grids of at most 2,113,536 bins
  * (one bin per face-aligned cell; a 128 x 129 x 128 cell grid) are taken;
  * larger inputs return IBM_ERR_SIZE before any work is queued.  Every call
