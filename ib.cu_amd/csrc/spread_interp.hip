@@ -18,8 +18,8 @@
 //     do are spread owner-computes: one workgroup per 8x8x8 brick of grid
 //     points gathers the (canonically ordered) markers of the bins whose
 //     stencils reach the brick into an LDS tile of the same integers;
-//   * interpolation is one lane per marker with the separable sum
-//     sum_z wz sum_y wy sum_x wx u.
+//   * interpolation is two lanes per marker and component, each with half of
+//     every row of the separable sum sum_z wz sum_y wy sum_x wx u.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <climits>
@@ -714,70 +714,6 @@ spread_brick_kernel(kgrids g, bin_desc bd, int delta, int total,
 }
 
 // ----------------------------------------------------------------------
-// Interpolation: one lane per marker.
-// ----------------------------------------------------------------------
-// Four doubles at 8-byte alignment (global loads need only dword alignment).
-typedef double d4u8 __attribute__((ext_vector_type(4), aligned(8)));
-
-__global__ void __launch_bounds__(256)
-interp_kernel(marker_sets sets, kgrids g, int delta,
-              const double* __restrict__ u0, const double* __restrict__ u1,
-              const double* __restrict__ u2)
-{
-    int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= sets.total) return;
-    int k = set_of(sets, m);
-    int l = m - sets.offset[k];
-    int n = sets.offset[k + 1] - sets.offset[k];
-    const double* x = sets.x[k];
-    double p[3] = {x[l], x[n + l], x[2 * n + l]};
-    for (int c = 0; c < 3; ++c) {
-        double w[3][4];
-        size_t ix[4], oy[4], oz[4];
-        const int* pt = g.points[c];
-        for (int j = 0; j < 3; ++j) {
-            stencil_axis st = axis_stencil(g.a[c][j], p[j]);
-            delta4(delta, st.d, w[j]);
-            for (int o = 0; o < 4; ++o) {
-                size_t idx = (size_t) axis_interp_index(g.a[c][j], st.base + o - 1);
-                if (j == 0) ix[o] = idx;
-                else if (j == 1) oy[o] = idx * (size_t) pt[0];
-                else oz[o] = idx * (size_t) pt[0] * (size_t) pt[1];
-            }
-        }
-        const double* u = c == 0 ? u0 : (c == 1 ? u1 : u2);    // global loads (an indexed array would be flat)
-        // the four x points are adjacent except across a periodic seam or a
-        // clamped wall: then one 32-byte load per row instead of four
-        const bool adjacent = ix[1] == ix[0] + 1 && ix[2] == ix[0] + 2 && ix[3] == ix[0] + 3;
-        double acc = 0.0;
-        for (int a = 0; a < 4; ++a) {
-            double sy = 0.0;
-            for (int b = 0; b < 4; ++b) {
-                const double* row = u + oz[a] + oy[b];
-                double v[4];
-                if (adjacent) {
-                    const d4u8 q = *(const d4u8*) (row + ix[0]);
-                    v[0] = q.x;
-                    v[1] = q.y;
-                    v[2] = q.z;
-                    v[3] = q.w;
-                } else {
-#pragma unroll
-                    for (int o = 0; o < 4; ++o) v[o] = row[ix[o]];
-                }
-                double sx = w[0][0] * v[0];
-                sx = fma(w[0][1], v[1], sx);
-                sx = fma(w[0][2], v[2], sx);
-                sx = fma(w[0][3], v[3], sx);
-                sy = fma(w[1][b], sx, sy);
-            }
-            acc = fma(w[2][a], sy, acc);
-        }
-        sets.out[k][(size_t) c * n + l] = acc;
-    }
-}
-
-// ----------------------------------------------------------------------
 // Host side
 // ----------------------------------------------------------------------
 kaxis to_kaxis(const ibm_axis& a)
@@ -1060,13 +996,27 @@ struct tile_desc {
     int box_points[3];  // points of one box's component grid
 };
 
-// Box of marker m: offsets holds nboxes + 1 increasing marker indices.
+// Box of marker m: offsets holds nboxes + 1 increasing marker indices.  All 64
+// lanes call it together, the first with the smallest m, whose box is found by
+// comparing 64 offsets at a time (a wavefront's markers mostly lie in one box,
+// and a bisection per lane is log2(nboxes) dependent loads); lanes beyond that
+// box bisect the rest.
 __device__ inline int box_of(const int* __restrict__ off, int nboxes, int m)
 {
-    int lo = 0, hi = nboxes;
-    while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (off[mid] <= m) lo = mid; else hi = mid;
+    const int m0 = __builtin_amdgcn_readfirstlane(m), lane = threadIdx.x & 63;
+    int lo = 0, n = nboxes;
+    while (n > 1) {
+        const int step = (n + 63) / 64;
+        const int before = __popcll(__ballot(lane * step < n && off[lo + min(lane * step, n - 1)] <= m0));
+        lo += (before - 1) * step;
+        n = min(step, n - (before - 1) * step);
+    }
+    if (lo + 1 < nboxes && off[lo + 1] <= m) {
+        int hi = nboxes;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (off[mid] <= m) lo = mid; else hi = mid;
+        }
     }
     return lo;
 }
@@ -1147,7 +1097,7 @@ tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const i
             br[j] = qb / TB;
             sub |= ((qb >> 2) & 1) << j;
         }
-        const int box = td.nboxes > 1 && valid ? box_of(box_off, td.nboxes, m) : 0;
+        const int box = td.nboxes > 1 ? box_of(box_off, td.nboxes, min(m, sets.total - 1)) : 0;
         bin[i] = (((box * td.nbr[2] + br[2]) * td.nbr[1] + br[1]) * td.nbr[0] + br[0]) * SUB + sub;
         const double f0 = fabs(f[i][0]), f1 = fabs(f[i][1]), f2 = fabs(f[i][2]);
         double a = f0 > f1 ? f0 : f1;
@@ -1604,51 +1554,97 @@ tile_merge_kernel(kgrids g, bin_desc bd, tile_desc td, int box0, unsigned chunk,
     fe[(size_t) box * td.box_points[c] + at] = (double) sum * scale->q;
 }
 
-// Interpolation over boxes: one lane per marker, grid vectors of box b at
-// offset b * box_points[c] (ib/interpolate.h:49-76 per box).
-__global__ void __launch_bounds__(256)
-interp_boxes_kernel(marker_sets sets, kgrids g, int delta, const int* __restrict__ box_off, int nboxes,
-                    const double* __restrict__ u0, const double* __restrict__ u1, const double* __restrict__ u2)
+// Two doubles at 8-byte alignment (global loads need only dword alignment).
+typedef double d2u8 __attribute__((ext_vector_type(2), aligned(8)));
+
+// Grid index of stencil point p for interpolation (ib/interpolate.h:16-22):
+// axis_interp_index() for p in [-2, points + 1], its modulo by comparisons.
+__device__ inline int kinterp_index(const kaxis& a, int p)
 {
-    int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= sets.total) return;
-    int k = set_of(sets, m);
-    int l = m - sets.offset[k];
-    int n = sets.offset[k + 1] - sets.offset[k];
-    const int box = box_of(box_off, nboxes, m);
-    const double* x = sets.x[k];
-    double p[3] = {x[l], x[n + l], x[2 * n + l]};
-    const double* ue[3] = {u0, u1, u2};
-    for (int c = 0; c < 3; ++c) {
-        double w[3][4];
-        size_t ix[4], oy[4], oz[4];
-        const int* pt = g.points[c];
-        for (int j = 0; j < 3; ++j) {
-            stencil_axis st = axis_stencil(g.a[c][j], p[j]);
-            delta4(delta, st.d, w[j]);
-            for (int o = 0; o < 4; ++o) {
-                size_t idx = (size_t) axis_interp_index(g.a[c][j], st.base + o - 1);
-                if (j == 0) ix[o] = idx;
-                else if (j == 1) oy[o] = idx * (size_t) pt[0];
-                else oz[o] = idx * (size_t) pt[0] * (size_t) pt[1];
-            }
-        }
-        const double* u = ue[c] + (size_t) box * pt[0] * pt[1] * pt[2];
-        double acc = 0.0;
-        for (int a = 0; a < 4; ++a) {
-            double sy = 0.0;
-            for (int b = 0; b < 4; ++b) {
-                const double* row = u + oz[a] + oy[b];
-                double sx = w[0][0] * row[ix[0]];
-                sx = fma(w[0][1], row[ix[1]], sx);
-                sx = fma(w[0][2], row[ix[2]], sx);
-                sx = fma(w[0][3], row[ix[3]], sx);
-                sy = fma(w[1][b], sx, sy);
-            }
-            acc = fma(w[2][a], sy, acc);
-        }
-        sets.out[k][(size_t) c * n + l] = acc;
+    if (!a.solid) {
+        p = p < 0 ? p + a.cells : p;
+        p = p >= a.cells ? p - a.cells : p;
+        p = p >= a.cells ? p - a.cells : p;
     }
+    return p < 0 ? 0 : (p >= a.points ? a.points - 1 : p);
+}
+
+// Interpolation (ib/interpolate.h:49-76), two lanes per marker and component,
+// each with two points of the 16 stencil rows; with BOXES, box b's grids lie
+// at b * box_points.
+// Bound by the vector L1's handling of scattered rows and, at half its issue
+// rate, the vector ALU: lanes of a pair share a row's line, so a load has 32
+// rows to look up instead of 64, and all 16 rows of a component are on their
+// way at once (no branch between them, the weights computed meanwhile), which
+// also meets each line of neighbouring markers while it is in the cache (16.5
+// to 7.6 million L2 requests at the size below).  One lane for a marker's
+// three components, rows one after another / one lane per marker and
+// component / this, us: 2210 markers 19 / 7.6 / 6.8, 46,400 on 100^3
+// 25 / 19 / 15, 684,000 in the 128 x 256 x 128 channel 138 / 156 / 135, 64
+// boxes of 32^3 with 264,000 69 / 41 / 42.
+constexpr int INTERP_THREADS = 256, INTERP_MARKERS = INTERP_THREADS / 2;
+
+template <bool BOXES>
+__global__ void __launch_bounds__(INTERP_THREADS, 4)
+interp_kernel(marker_sets sets, kgrids g, int delta, const int* __restrict__ box_off, int nboxes, int blocks, int chunk,
+              const double* __restrict__ u0, const double* __restrict__ u1, const double* __restrict__ u2)
+{
+    // XCD x takes the x-th eighth: neighbouring markers share its L2's rows
+    const int nth = (int) (blockIdx.x >> 3), c = nth / chunk, block = (int) (blockIdx.x & 7) * chunk + nth % chunk;
+    if (block >= blocks) return;
+    const int half = threadIdx.x & 1, own = block * INTERP_MARKERS + (int) (threadIdx.x >> 1);
+    const int m = min(own, sets.total - 1);
+    double p[3];
+    load_marker(sets, m, p);
+    const kaxis* a = g.a[c];
+    double d[3];
+    int at[3][4];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const stencil_axis st = kstencil(a[j], p[j]);
+        d[j] = st.d;
+#pragma unroll
+        for (int o = 0; o < 4; ++o) at[j][o] = kinterp_index(a[j], st.base + o - 1);
+    }
+    const int x0 = half ? at[0][2] : at[0][0], x1 = half ? at[0][3] : at[0][1];
+    const int px = g.points[c][0], py = g.points[c][1];
+    const double* u = c == 0 ? u0 : (c == 1 ? u1 : u2);    // global loads (an indexed array would be flat)
+    if (BOXES) u += (size_t) box_of(box_off, nboxes, m) * px * py * g.points[c][2];
+    d2u8 v[4][4];
+    // the two points are adjacent except across a periodic seam or a clamped
+    // wall: then one 16-byte load per row instead of two
+    if (x1 == x0 + 1) {
+        u += x0;
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) v[z][y] = *(const d2u8*) (u + px * (at[1][y] + py * at[2][z]));
+    } else {
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                const double* row = u + px * (at[1][y] + py * at[2][z]);
+                v[z][y] = d2u8{row[x0], row[x1]};
+            }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the weights while the rows are on their way
+    double w[3][4], sum = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) delta4(delta, d[j], w[j]);
+    const double w0 = half ? w[0][2] : w[0][0], w1 = half ? w[0][3] : w[0][1];
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+        double sy = 0.0;
+#pragma unroll
+        for (int y = 0; y < 4; ++y) sy = fma(w[1][y], fma(w1, v[z][y].y, w0 * v[z][y].x), sy);
+        sum = fma(w[2][z], sy, sum);
+    }
+    sum += __shfl_xor(sum, 1, 64);
+    const int k = set_of(sets, m);
+    if (own < sets.total && half == 0)
+        sets.out[k][(size_t) c * (sets.offset[k + 1] - sets.offset[k]) + (m - sets.offset[k])] = sum;
 }
 
 } // namespace
@@ -1947,7 +1943,9 @@ ibm_status interp_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const mar
     if (!ue || !ue[0] || !ue[1] || !ue[2]) return fail(ctx, IBM_ERR_ARG, "null input grid");
     if (sets.total == 0) return IBM_OK;
     prof_scope prof(ctx, "interp");
-    interp_kernel<<<blocks_for(sets.total, 256), 256, 0, ctx->stream>>>(sets, kg, delta, ue[0], ue[1], ue[2]);
+    const int blocks = blocks_for(sets.total, INTERP_MARKERS), chunk = (blocks + 7) / 8;
+    interp_kernel<false><<<24 * chunk, INTERP_THREADS, 0, ctx->stream>>>(sets, kg, delta, nullptr, 1, blocks, chunk, ue[0],
+                                                                        ue[1], ue[2]);
     IBM_LAUNCH_CHECK(ctx);
     return IBM_OK;
 }
@@ -1979,8 +1977,9 @@ ibm_status interp_boxes(ibm_ctx* ctx, const ibm_grid* grids, int delta, const ma
     if (!ue || !ue[0] || !ue[1] || !ue[2]) return fail(ctx, IBM_ERR_ARG, "null input grid");
     if (sets.total == 0) return IBM_OK;
     prof_scope prof(ctx, "interp");
-    interp_boxes_kernel<<<blocks_for(sets.total, 256), 256, 0, ctx->stream>>>(sets, kg, delta, box_off, nboxes, ue[0],
-                                                                              ue[1], ue[2]);
+    const int blocks = blocks_for(sets.total, INTERP_MARKERS), chunk = (blocks + 7) / 8;
+    interp_kernel<true><<<24 * chunk, INTERP_THREADS, 0, ctx->stream>>>(sets, kg, delta, box_off, nboxes, blocks, chunk, ue[0],
+                                                                       ue[1], ue[2]);
     IBM_LAUNCH_CHECK(ctx);
     return IBM_OK;
 }
