@@ -12,10 +12,9 @@
 //   = B_j,   mu = lambda_x(kx) + lambda_z(kz),
 // with the wall rows' ghost coefficients in d_0, d_{n-1} (fd/discretization.h:
 // 94-108).  The solve is: real-to-half-complex FFT along x, complex FFT
-// along z, one tridiagonal solve per mode (parallel cyclic reduction in
-// LDS), and the inverse
-// transforms -- the exact solution of the same discrete system the multigrid
-// iterates on, in five memory passes.  The singular case (sigma = 0 with
+// along z, one tridiagonal solve per mode (chunks of rows in registers), and
+// the inverse transforms -- the exact solution of the same discrete system the
+// multigrid iterates on, in five memory passes.  The singular case (sigma = 0 with
 // Neumann walls: the pressure Poisson) solves the mean-free problem, as the
 // multigrid does: the (0, 0) mode's right-hand side loses its mean, its last
 // unknown is pinned and the solution's mean is removed.
@@ -38,11 +37,12 @@ constexpr int FFT_THREADS = 256;
 constexpr int ZT = 8;              // kx columns per z-transform block
 constexpr int MAX_FFT_POINTS = 512;
 constexpr int MAX_WALL_POINTS = 800;
+constexpr int LINE_THREADS = 256, LINE_MODES = 8, LINE_CHUNKS = LINE_THREADS / LINE_MODES;
 constexpr size_t MAX_DYNAMIC_LDS = 160 * 1024;
 
 // Row stride of the half-spectrum in coefficients: nh rounded up to 8 (rows
 // start on 128-byte boundaries, so the column tiles of the z transform and
-// the cyclic reduction read whole cache lines).
+// the line solves read whole cache lines).
 __host__ __device__ constexpr int spec_ld(int nh) { return (nh + 7) & ~7; }
 
 __device__ inline double2 cmul(double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
@@ -223,155 +223,152 @@ __device__ inline void tri_row(const wall_axis& y, double sigma, double tau, dou
     diag = id * (sigma + tau * mu) + ty * d;
 }
 
-// Every Fourier mode's tridiagonal system along y by parallel cyclic
-// reduction in LDS: block (kx tile of zt modes, kz) holds zt x np2 rows
-// (np2 = ny rounded up to a power of two; rows past ny are identity rows),
-// 256 threads update PCR_ITEMS rows each per step (row j combined with rows
-// j -+ 2^s) until P interleaved subsystems of np2 / P <= PCR_SPLIT rows are
-// left (P >= PCR_SPLIT where np2 allows), which one thread each solves by
-// the Thomas algorithm.  The singular mode's last
-// equation is replaced by x = 0 after its right-hand side loses its mean,
-// and its solution loses its mean.
-constexpr int PCR_THREADS = 256, PCR_ITEMS = 4, PCR_ROWS = PCR_THREADS * PCR_ITEMS, PCR_SPLIT = 16;
-
-__global__ void __launch_bounds__(PCR_THREADS) pcr_kernel(int nh, int zt, int np2, wall_axis y, double sigma,
-                                                          double tau, int singular, const double* __restrict__ lam_x,
-                                                          const double* __restrict__ lam_z, double2* __restrict__ s)
+// Sum over a workgroup's LINE_CHUNKS chunks of the lanes with t = 0.
+__device__ inline double2 line_sum(double2 v, double2* part)
 {
-    extern __shared__ double2 sh[];
-    double2* D = sh;
-    double* A = (double*) (sh + PCR_ROWS);
-    double* B = A + PCR_ROWS;
-    double* C = B + PCR_ROWS;
-    const int ny = y.n, kx0 = blockIdx.x * zt, kz = blockIdx.y;
+    __syncthreads();
+    if (threadIdx.x % LINE_MODES == 0) part[threadIdx.x / LINE_MODES] = v;
+    __syncthreads();
+    double2 m = make_double2(0.0, 0.0);
+    for (int i = 0; i < LINE_CHUNKS; ++i) {
+        m.x += part[i].x;
+        m.y += part[i].y;
+    }
+    return m;
+}
+
+// Every Fourier mode's tridiagonal system along y: block (tile of LINE_MODES
+// kx, kz), one thread per mode and chunk of M consecutive rows, which it keeps
+// in registers (rows past ny are identity rows).  A forward elimination leaves
+// row r as X_r = d_r - c_r X_{r+1} - a_r X_{-1}, with X_{-1} the last row of
+// the chunk before, and a backward one gives the first row by the chunk's and
+// the previous chunk's last; put into the previous chunk's last row that is
+// one equation per chunk, solved by cyclic reduction over the LINE_CHUNKS of
+// them, and a back substitution ends it.  The singular mode's last equation is
+// replaced by x = 0 after its right-hand side loses its mean, and its solution
+// loses its mean.  Bound by memory (16 bytes per row read and written, whole
+// 128-byte lines): cyclic reduction over all rows in LDS took two divisions
+// per row and step, eight in all, this one and a fraction.  65 x 256 x 128
+// coefficients: 48 us / 17.
+template <int M>
+__global__ void __launch_bounds__(LINE_THREADS) line_kernel(int nh, wall_axis y, double sigma, double tau, int singular,
+                                                            const double* __restrict__ lam_x,
+                                                            const double* __restrict__ lam_z, double2* __restrict__ s)
+{
+    __shared__ double2 D[2][LINE_THREADS];
+    __shared__ double2 AC[2][LINE_THREADS];
+    __shared__ double2 part[LINE_CHUNKS];
+    const int ny = y.n, t = threadIdx.x % LINE_MODES, q = threadIdx.x / LINE_MODES;
+    const int kx = blockIdx.x * LINE_MODES + t, kz = blockIdx.y, j0 = q * M;
     const int ld = spec_ld(nh);
-    const size_t plane = (size_t) ld * ny;
-    const bool pin_block = singular && kx0 == 0 && kz == 0;     // holds the singular mode (t = 0)
-    for (int e = threadIdx.x; e < PCR_ROWS; e += PCR_THREADS) {
-        const int t = e % zt, j = e / zt, kx = kx0 + t;
-        double a = 0.0, b = 1.0, c = 0.0;
-        double2 d = make_double2(0.0, 0.0);
-        if (kx < nh && j < ny) {
-            tri_row(y, sigma, tau, lam_x[kx] + lam_z[kz], j, a, c, b);
-            d = s[(size_t) kz * plane + (size_t) j * ld + kx];
-        }
-        A[e] = a;
-        B[e] = b;
-        C[e] = c;
-        D[e] = d;
-    }
-    __syncthreads();
-    if (pin_block && threadIdx.x == 0) {
-        double2 m = make_double2(0.0, 0.0);
-        for (int j = 0; j < ny; ++j) {
-            m.x += D[j * zt].x;
-            m.y += D[j * zt].y;
-        }
-        m.x /= ny;
-        m.y /= ny;
-        for (int j = 0; j < ny - 1; ++j) {
-            D[j * zt].x -= m.x;
-            D[j * zt].y -= m.y;
-        }
-        const int last = (ny - 1) * zt;
-        A[last] = 0.0;
-        B[last] = 1.0;
-        C[last] = 0.0;
-        D[last] = make_double2(0.0, 0.0);
-    }
-    __syncthreads();
-    // Reduction until the rows left coupled (j -+ P) form P interleaved
-    // subsystems of at most PCR_SPLIT rows, then one Thomas sweep per
-    // subsystem.
-    const int P = max(min(np2, PCR_SPLIT), np2 / PCR_SPLIT);
-    for (int sft = 1; sft < P; sft <<= 1) {
-        double na[PCR_ITEMS], nb[PCR_ITEMS], nc[PCR_ITEMS];
-        double2 nd[PCR_ITEMS];
+    const bool pin_block = singular && blockIdx.x == 0 && kz == 0;     // holds the singular mode (t = 0)
+    const bool pinned = pin_block && t == 0;
+    double2* col = s + (size_t) kz * ld * ny + kx;
+    double a[M], c[M];
+    double2 d[M];
 #pragma unroll
-        for (int i = 0; i < PCR_ITEMS; ++i) {
-            const int e = threadIdx.x + PCR_THREADS * i;
-            const int t = e % zt, j = e / zt;
-            double a = A[e], b = B[e], c = C[e];
-            double2 d = D[e];
-            if (j - sft >= 0) {
-                const int m = (j - sft) * zt + t;
-                const double al = -a / B[m];
-                b += al * C[m];
-                d.x += al * D[m].x;
-                d.y += al * D[m].y;
-                a = al * A[m];
-            } else {
-                a = 0.0;
-            }
-            if (j + sft < np2) {
-                const int p = (j + sft) * zt + t;
-                const double ga = -c / B[p];
-                b += ga * A[p];
-                d.x += ga * D[p].x;
-                d.y += ga * D[p].y;
-                c = ga * C[p];
-            } else {
-                c = 0.0;
-            }
-            na[i] = a;
-            nb[i] = b;
-            nc[i] = c;
-            nd[i] = d;
-        }
-        __syncthreads();
+    for (int r = 0; r < M; ++r) d[r] = kx < nh && j0 + r < ny ? col[(size_t) (j0 + r) * ld] : make_double2(0.0, 0.0);
+    const double mu = kx < nh ? lam_x[kx] + lam_z[kz] : 0.0;
+    if (pin_block) {
+        double2 own = make_double2(0.0, 0.0);
 #pragma unroll
-        for (int i = 0; i < PCR_ITEMS; ++i) {
-            const int e = threadIdx.x + PCR_THREADS * i;
-            A[e] = na[i];
-            B[e] = nb[i];
-            C[e] = nc[i];
-            D[e] = nd[i];
+        for (int r = 0; r < M; ++r) own = make_double2(own.x + d[r].x, own.y + d[r].y);
+        const double2 sum = line_sum(own, part);
+        if (pinned) {
+#pragma unroll
+            for (int r = 0; r < M; ++r)
+                if (j0 + r < ny) d[r] = make_double2(d[r].x - sum.x / ny, d[r].y - sum.y / ny);
         }
+    }
+#pragma unroll
+    for (int r = 0; r < M; ++r) {
+        const int j = j0 + r;
+        double lo = 0.0, hi = 0.0, diag = 1.0;
+        if (kx < nh && j < ny) tri_row(y, sigma, tau, mu, j, lo, hi, diag);
+        if (pinned && j == ny - 1) {
+            lo = hi = 0.0;
+            diag = 1.0;
+            d[r] = make_double2(0.0, 0.0);
+        }
+        if (r == 0) {
+            const double inv = 1.0 / diag;
+            a[r] = lo * inv;
+            c[r] = hi * inv;
+            d[r] = make_double2(d[r].x * inv, d[r].y * inv);
+        } else {
+            const double inv = 1.0 / (diag - lo * c[r - 1]);
+            a[r] = -lo * a[r - 1] * inv;
+            c[r] = hi * inv;
+            d[r] = make_double2((d[r].x - lo * d[r - 1].x) * inv, (d[r].y - lo * d[r - 1].y) * inv);
+        }
+    }
+    // the chunk's first row: X_0 = p - f X_{-1} - g X_{M-1}
+    double f = a[M - 2], g = c[M - 2];
+    double2 p = d[M - 2];
+#pragma unroll
+    for (int r = M - 3; r >= 0; --r) {
+        f = a[r] - c[r] * f;
+        p = make_double2(d[r].x - c[r] * p.x, d[r].y - c[r] * p.y);
+        g = -c[r] * g;
+    }
+    // the next chunk's first row in this one's last
+    const int id = threadIdx.x;
+    D[0][id] = p;
+    AC[0][id] = make_double2(f, g);
+    __syncthreads();
+    double ra = a[M - 1], rc = 0.0;
+    double2 rd = d[M - 1];
+    if (q + 1 < LINE_CHUNKS) {
+        const double2 np = D[0][id + LINE_MODES], nfg = AC[0][id + LINE_MODES];
+        const double inv = 1.0 / (1.0 - c[M - 1] * nfg.x);
+        ra *= inv;
+        rc = -c[M - 1] * nfg.y * inv;
+        rd = make_double2((rd.x - c[M - 1] * np.x) * inv, (rd.y - c[M - 1] * np.y) * inv);
+    }
+    if (q == 0) ra = 0.0;
+    // cyclic reduction of X_q + ra X_{q-1} + rc X_{q+1} = rd
+    int buf = 1;
+#pragma unroll
+    for (int sft = 1; sft < LINE_CHUNKS; sft <<= 1) {
+        D[buf][id] = rd;
+        AC[buf][id] = make_double2(ra, rc);
         __syncthreads();
-    }
-    const int L = np2 / P, step = P * zt;
-    for (int id = threadIdx.x; id < zt * P; id += PCR_THREADS) {
-        int e = id;                                  // row r = id / zt of mode t = id % zt
-        double inv = 1.0 / B[e];
-        double cp = C[e] * inv;
-        double2 dp = make_double2(D[e].x * inv, D[e].y * inv);
-        C[e] = cp;
-        D[e] = dp;
-        for (int m = 1; m < L; ++m) {
-            e += step;
-            const double a = A[e];
-            inv = 1.0 / (B[e] - a * cp);
-            cp = C[e] * inv;
-            dp = make_double2((D[e].x - a * dp.x) * inv, (D[e].y - a * dp.y) * inv);
-            C[e] = cp;
-            D[e] = dp;
+        double2 dm = make_double2(0.0, 0.0), dn = dm, am = dm, an = dm;
+        if (q >= sft) {
+            dm = D[buf][id - sft * LINE_MODES];
+            am = AC[buf][id - sft * LINE_MODES];
         }
-        double2 xv = dp;
-        for (int m = L - 2; m >= 0; --m) {
-            e -= step;
-            xv = make_double2(D[e].x - C[e] * xv.x, D[e].y - C[e] * xv.y);
-            D[e] = xv;
+        if (q + sft < LINE_CHUNKS) {
+            dn = D[buf][id + sft * LINE_MODES];
+            an = AC[buf][id + sft * LINE_MODES];
         }
+        const double inv = 1.0 / (1.0 - ra * am.y - rc * an.x);
+        rd = make_double2((rd.x - ra * dm.x - rc * dn.x) * inv, (rd.y - ra * dm.y - rc * dn.y) * inv);
+        ra = -ra * am.x * inv;
+        rc = -rc * an.y * inv;
+        buf ^= 1;
     }
+    D[buf][id] = rd;
     __syncthreads();
-    if (pin_block && threadIdx.x == 0) {
-        double2 m = make_double2(0.0, 0.0);
-        for (int j = 0; j < ny; ++j) {
-            m.x += D[j * zt].x;
-            m.y += D[j * zt].y;
-        }
-        m.x /= ny;
-        m.y /= ny;
-        for (int j = 0; j < ny; ++j) {
-            D[j * zt].x -= m.x;
-            D[j * zt].y -= m.y;
+    const double2 before = q > 0 ? D[buf][id - LINE_MODES] : make_double2(0.0, 0.0);
+    d[M - 1] = rd;
+#pragma unroll
+    for (int r = M - 2; r >= 0; --r)
+        d[r] = make_double2(d[r].x - c[r] * d[r + 1].x - a[r] * before.x, d[r].y - c[r] * d[r + 1].y - a[r] * before.y);
+    if (pin_block) {
+        double2 own = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int r = 0; r < M; ++r)
+            if (j0 + r < ny) own = make_double2(own.x + d[r].x, own.y + d[r].y);
+        const double2 sum = line_sum(own, part);
+        if (pinned) {
+#pragma unroll
+            for (int r = 0; r < M; ++r) d[r] = make_double2(d[r].x - sum.x / ny, d[r].y - sum.y / ny);
         }
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < PCR_ROWS; e += PCR_THREADS) {
-        const int t = e % zt, j = e / zt, kx = kx0 + t;
-        if (kx < nh && j < ny) s[(size_t) kz * plane + (size_t) j * ld + kx] = D[e];
-    }
+#pragma unroll
+    for (int r = 0; r < M; ++r)
+        if (kx < nh && j0 + r < ny) col[(size_t) (j0 + r) * ld] = d[r];
 }
 
 int log2_exact(int n)
@@ -450,8 +447,6 @@ static ibm_status fft_lds_attributes(ibm_ctx* ctx)
     if (done) return IBM_OK;
     IBM_HIP(ctx, hipFuncSetAttribute((const void*) zfft_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int) MAX_DYNAMIC_LDS));
-    IBM_HIP(ctx, hipFuncSetAttribute((const void*) pcr_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int) MAX_DYNAMIC_LDS));
     done = true;
     return IBM_OK;
 }
@@ -476,13 +471,15 @@ ibm_status fft_solve(ibm_ctx* ctx, ibm_fft* p, double sigma, double tau, const d
     zfft_kernel<<<zgrid, FFT_THREADS, zlds, ctx->stream>>>(p->nh, p->ny, p->nz, p->lz, p->spec, p->twz, 0);
     IBM_LAUNCH_CHECK(ctx);
     const int singular = sigma == 0.0 && p->neumann;
-    int np2 = 1;
-    while (np2 < p->ny) np2 <<= 1;
-    const int zt = PCR_ROWS / np2;
-    const dim3 tgrid((p->nh + zt - 1) / zt, p->nz);
-    const size_t tlds = (sizeof(double2) + 3 * sizeof(double)) * PCR_ROWS;
-    pcr_kernel<<<tgrid, PCR_THREADS, tlds, ctx->stream>>>(p->nh, zt, np2, p->y, sigma, tau, singular, p->lam_x, p->lam_z,
-                                                          p->spec);
+    const dim3 tgrid((p->nh + LINE_MODES - 1) / LINE_MODES, p->nz);
+    auto lines = [&](auto kernel) {
+        kernel<<<tgrid, LINE_THREADS, 0, ctx->stream>>>(p->nh, p->y, sigma, tau, singular, p->lam_x, p->lam_z, p->spec);
+    };
+    if (p->ny <= 2 * LINE_CHUNKS) lines(line_kernel<2>);
+    else if (p->ny <= 4 * LINE_CHUNKS) lines(line_kernel<4>);
+    else if (p->ny <= 8 * LINE_CHUNKS) lines(line_kernel<8>);
+    else if (p->ny <= 16 * LINE_CHUNKS) lines(line_kernel<16>);
+    else lines(line_kernel<(MAX_WALL_POINTS + LINE_CHUNKS - 1) / LINE_CHUNKS>);
     IBM_LAUNCH_CHECK(ctx);
     zfft_kernel<<<zgrid, FFT_THREADS, zlds, ctx->stream>>>(p->nh, p->ny, p->nz, p->lz, p->spec, p->twz, 1);
     IBM_LAUNCH_CHECK(ctx);

@@ -298,7 +298,7 @@ ibm_status ibm_mg_solve(ibm_ctx* ctx, ibm_mg* mg, const double* b, double* x, do
 /* Direct solves of A x = b, A = sigma I~ + tau L, on grids periodic in x
  * and z with power-of-two point counts (4 to 512) and walled in y (2 to
  * 800 points): FFTs in x and z diagonalise the periodic parts, leaving one
- * tridiagonal system along y per Fourier mode (Thomas elimination).  The
+ * tridiagonal system along y per Fourier mode.  The
  * exact solution of the system solvers::multigrid iterates on
  * (solvers/multigrid.h:176-212); no counterpart as an algorithm in the
  * reference.  sigma = 0 with Neumann walls is the singular Poisson case:
