@@ -258,7 +258,7 @@ PMC_KERNELS = {"chebyshev_f32": "cheb_march_kernel<float", "chebyshev_f64": "che
                "momentum_rhs": "momentum_rhs_kernel", "residual_update": "residual_update_kernel",
                "divergence": "divergence_kernel",
                "bin": ("tile_count_kernel", "tile_scatter_kernel"),
-               "fft_solve": ("xfft_forward_kernel", "zfft_kernel", "line_kernel", "xfft_inverse_kernel")}
+               "fft_solve": ("plane_forward_kernel", "line_kernel", "plane_inverse_kernel")}
 COPY_BYTES = 1 << 28     # the calibration copy: 256 MiB read, 256 MiB written
 
 

@@ -14,7 +14,8 @@
 // 94-108).  The solve is: real-to-half-complex FFT along x, complex FFT
 // along z, one tridiagonal solve per mode (chunks of rows in registers), and
 // the inverse transforms -- the exact solution of the same discrete system the
-// multigrid iterates on, in five memory passes.  The singular case (sigma = 0 with
+// multigrid iterates on.  The transforms of a y-plane are one memory pass where
+// the plane fits the LDS (three passes per solve) and two elsewhere (five).  The singular case (sigma = 0 with
 // Neumann walls: the pressure Poisson) solves the mean-free problem, as the
 // multigrid does: the (0, 0) mode's right-hand side loses its mean, its last
 // unknown is pinned and the solution's mean is removed.
@@ -195,6 +196,251 @@ __global__ void __launch_bounds__(FFT_THREADS) zfft_kernel(int nh, int ny, int n
     for (int e = threadIdx.x; e < ZT * nz; e += blockDim.x) {
         const int t = e % ZT, k = e / ZT, kx = kx0 + t;
         if (kx < nh) s[(size_t) k * plane + (size_t) j * ld + kx] = sh[e];
+    }
+}
+
+// ----------------------------------------------------------------------
+// Both transforms of one y-plane in LDS
+// ----------------------------------------------------------------------
+// DFT of R values in registers, natural order in and out.
+template <int R, bool INV>
+__device__ inline void dft(double2 (&v)[R])
+{
+    if constexpr (R == 2) {
+        const double2 u = v[0], w = v[1];
+        v[0] = make_double2(u.x + w.x, u.y + w.y);
+        v[1] = make_double2(u.x - w.x, u.y - w.y);
+    } else {
+        // cos(2 pi k / 16), k = 0..4
+        constexpr double C[5] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173, 0.0};
+        double2 e[R / 2], o[R / 2];
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k) {
+            e[k] = v[2 * k];
+            o[k] = v[2 * k + 1];
+        }
+        dft<R / 2, INV>(e);
+        dft<R / 2, INV>(o);
+#pragma unroll
+        for (int k = 0; k < R / 2; ++k) {
+            const int m = k * (16 / R);                       // exp(-+ 2 pi i m / 16), m < 8
+            double2 t = o[k];
+            if (m == 4) {
+                t = INV ? make_double2(-t.y, t.x) : make_double2(t.y, -t.x);
+            } else if (m > 0) {
+                const double c = m < 4 ? C[m] : -C[8 - m], sn = m < 4 ? C[4 - m] : C[m - 4];
+                t = cmul(t, make_double2(c, INV ? sn : -sn));
+            }
+            v[k] = make_double2(e[k].x + t.x, e[k].y + t.y);
+            v[k + R / 2] = make_double2(e[k].x - t.x, e[k].y - t.y);
+        }
+    }
+}
+
+__device__ inline double2 conj2(double2 a) { return make_double2(a.x, -a.y); }
+
+// LDS position of point n of a row: eight lanes with consecutive n, or with n
+// eight apart, lie in different banks.
+__device__ inline int swz(int n) { return n ^ ((n >> 3) & 7); }
+
+// Sizes of a plane transform: nx x nz points with nx = 2^LX, nz = 2^LZ.  A row
+// of nx reals is transformed as H = nx / 2 complex points, 8 x SX; a column of
+// nz as 8 x SZ.
+template <int LX, int LZ>
+struct plane_size {
+    static constexpr int NX = 1 << LX, NZ = 1 << LZ, H = NX / 2, SX = H / 8, SZ = NZ / 8, LD = H + 1;
+    static constexpr int THREADS = NX * NZ / 32 < 256 ? 256 : NX * NZ / 32;
+    static constexpr size_t LDS = sizeof(double2) * (NZ * LD + NX + NZ);
+};
+
+// Tables exp(-2 pi i e / n) for all e < n, from the first halves.
+template <class P>
+__device__ inline void plane_tables(double2* wx, double2* wz, const double2* __restrict__ twx, const double2* __restrict__ twz)
+{
+    for (int e = threadIdx.x; e < P::NX; e += P::THREADS) {
+        const double2 w = twx[e % (P::NX / 2)];
+        wx[e] = e < P::NX / 2 ? w : make_double2(-w.x, -w.y);
+    }
+    for (int e = threadIdx.x; e < P::NZ; e += P::THREADS) {
+        const double2 w = twz[e % (P::NZ / 2)];
+        wz[e] = e < P::NZ / 2 ? w : make_double2(-w.x, -w.y);
+    }
+}
+
+// Two doubles at 8-byte alignment (the caller's vector).
+typedef double d2u8 __attribute__((ext_vector_type(2), aligned(8)));
+
+// Forward transforms along x and z of plane j = blockIdx.x, the same values as
+// xfft_forward_kernel and zfft_kernel: the half-spectrum stays in LDS between
+// them, and every stage takes 8 or 16 points at a time in registers.
+// A row's reals are taken as half as many complex points.  Bound by the phases
+// of a block, which cannot overlap where one plane fills a CU's LDS (load, four
+// LDS round trips, store); two passes wrote and read the half-spectrum once
+// more and did radix-2 stages in pairs.  128 x 256 x 128 points, forward /
+// inverse: 49 / 49 us by passes, 22 / 18 by planes.
+template <int LX, int LZ>
+__global__ void __launch_bounds__((plane_size<LX, LZ>::THREADS))
+plane_forward_kernel(int ny, const double* __restrict__ x, double2* __restrict__ s, const double2* __restrict__ twx,
+                     const double2* __restrict__ twz)
+{
+    using P = plane_size<LX, LZ>;
+    constexpr int NX = P::NX, NZ = P::NZ, H = P::H, SX = P::SX, SZ = P::SZ, LD = P::LD, T = P::THREADS;
+    extern __shared__ double2 sh[];
+    double2* wx = sh + NZ * LD;
+    double2* wz = wx + NX;
+    const int j = blockIdx.x, tid = threadIdx.x;
+    plane_tables<P>(wx, wz, twx, twz);
+    // rows: points m0 + SX i of z[m] = (x[2m], x[2m+1])
+    constexpr int ROW_TASKS = NZ * SX, ROW_ITEMS = (ROW_TASKS + T - 1) / T;
+    double2 v[ROW_ITEMS][8];
+#pragma unroll
+    for (int u = 0; u < ROW_ITEMS; ++u) {
+        const int e = tid + u * T, row = e / SX, m0 = e % SX;
+        if (ROW_TASKS % T == 0 || e < ROW_TASKS) {
+            const double* src = x + ((size_t) row * ny + j) * NX + 2 * m0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const d2u8 q = *(const d2u8*) (src + 2 * SX * i);
+                v[u][i] = make_double2(q.x, q.y);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < ROW_ITEMS; ++u) {
+        const int e = tid + u * T, row = e / SX, m0 = e % SX;
+        if (ROW_TASKS % T == 0 || e < ROW_TASKS) {
+            dft<8, false>(v[u]);
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                sh[row * LD + swz(8 * m0 + q)] = q == 0 ? v[u][q] : cmul(v[u][q], wx[2 * m0 * q]);
+        }
+    }
+    __syncthreads();
+    // rows: the SX points of each q, giving Z[8 k + q] in place
+    for (int e = tid; e < NZ * 8; e += T) {
+        const int row = e >> 3, q = e & 7;
+        double2 w[SX];
+#pragma unroll
+        for (int m = 0; m < SX; ++m) w[m] = sh[row * LD + swz(8 * m + q)];
+        dft<SX, false>(w);
+#pragma unroll
+        for (int m = 0; m < SX; ++m) sh[row * LD + swz(8 * m + q)] = w[m];
+    }
+    __syncthreads();
+    // the rows' coefficients k and H - k from Z[k] and Z[H - k], and the
+    // columns' points m0 + SZ i
+    for (int e = tid; e < (H / 2 + 1) * SZ; e += T) {
+        const int k = e < H / 2 * SZ ? e % (H / 2) : H / 2, m0 = e < H / 2 * SZ ? e / (H / 2) : e - H / 2 * SZ;
+        const int at0 = swz(k), at1 = k == 0 ? H : swz(H - k);
+        const double2 wk = wx[k];
+        double2 a[8], b[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const double2* row = sh + (m0 + SZ * i) * LD;
+            const double2 z0 = row[at0], z1 = k == 0 ? z0 : row[at1];
+            const double2 ev = make_double2(0.5 * (z0.x + z1.x), 0.5 * (z0.y - z1.y));
+            const double2 od = make_double2(0.5 * (z0.y + z1.y), 0.5 * (z1.x - z0.x));
+            const double2 t = cmul(od, wk);
+            a[i] = make_double2(ev.x + t.x, ev.y + t.y);
+            b[i] = make_double2(ev.x - t.x, t.y - ev.y);
+        }
+        dft<8, false>(a);
+        dft<8, false>(b);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            double2* row = sh + (m0 + SZ * q) * LD;
+            const double2 w = wz[m0 * q];
+            row[at0] = cmul(a[q], w);
+            if (k != H / 2) row[at1] = cmul(b[q], w);
+        }
+    }
+    __syncthreads();
+    // columns: the SZ points of each q, giving kz = 8 m + q
+    for (int e = tid; e < LD * 8; e += T) {
+        const int kx = e % LD, q = e / LD, at = kx == H ? H : swz(kx);
+        double2 w[SZ];
+#pragma unroll
+        for (int m = 0; m < SZ; ++m) w[m] = sh[(SZ * q + m) * LD + at];
+        dft<SZ, false>(w);
+#pragma unroll
+        for (int m = 0; m < SZ; ++m) s[((size_t) (8 * m + q) * ny + j) * spec_ld(LD) + kx] = w[m];
+    }
+}
+
+// Inverse of plane_forward_kernel, scaled by `scale`.
+template <int LX, int LZ>
+__global__ void __launch_bounds__((plane_size<LX, LZ>::THREADS))
+plane_inverse_kernel(int ny, const double2* __restrict__ s, double* __restrict__ x, double scale,
+                     const double2* __restrict__ twx, const double2* __restrict__ twz)
+{
+    using P = plane_size<LX, LZ>;
+    constexpr int NX = P::NX, NZ = P::NZ, H = P::H, SX = P::SX, SZ = P::SZ, LD = P::LD, T = P::THREADS;
+    extern __shared__ double2 sh[];
+    double2* wx = sh + NZ * LD;
+    double2* wz = wx + NX;
+    const int j = blockIdx.x, tid = threadIdx.x;
+    plane_tables<P>(wx, wz, twx, twz);
+    __syncthreads();
+    // columns: points kz = m0 + 8 i
+    for (int e = tid; e < LD * 8; e += T) {
+        const int kx = e % LD, m0 = e / LD, at = kx == H ? H : swz(kx);
+        double2 w[SZ];
+#pragma unroll
+        for (int i = 0; i < SZ; ++i) w[i] = s[((size_t) (m0 + 8 * i) * ny + j) * spec_ld(LD) + kx];
+        dft<SZ, true>(w);
+#pragma unroll
+        for (int q = 0; q < SZ; ++q) sh[(SZ * m0 + q) * LD + at] = q == 0 ? w[q] : cmul(w[q], conj2(wz[m0 * q]));
+    }
+    __syncthreads();
+    // columns: the 8 points of each q, giving z = SZ m + q in place, and the
+    // rows' Z[k] and Z[H - k] (twice their value) from the coefficients k and
+    // H - k
+    for (int e = tid; e < (H / 2 + 1) * SZ; e += T) {
+        const int k = e < H / 2 * SZ ? e % (H / 2) : H / 2, q = e < H / 2 * SZ ? e / (H / 2) : e - H / 2 * SZ;
+        const int at0 = swz(k), at1 = k == 0 ? H : swz(H - k);
+        const double2 wk = conj2(wx[k]);
+        double2 a[8], b[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const double2* row = sh + (SZ * m + q) * LD;
+            a[m] = row[at0];
+            b[m] = row[at1];
+        }
+        dft<8, true>(a);
+        dft<8, true>(b);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const double2 ev = make_double2(a[m].x + b[m].x, a[m].y - b[m].y);
+            const double2 od = cmul(make_double2(a[m].x - b[m].x, a[m].y + b[m].y), wk);
+            double2* row = sh + (SZ * m + q) * LD;
+            row[at0] = make_double2(ev.x - od.y, ev.y + od.x);
+            if (k != 0 && k != H / 2) row[at1] = make_double2(ev.x + od.y, od.x - ev.y);
+        }
+    }
+    __syncthreads();
+    // rows: points m0 + SX i, in place
+    for (int e = tid; e < NZ * SX; e += T) {
+        const int row = e / SX, m0 = e % SX;
+        double2 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = sh[row * LD + swz(m0 + SX * i)];
+        dft<8, true>(v);
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            sh[row * LD + swz(m0 + SX * q)] = q == 0 ? v[q] : cmul(v[q], conj2(wx[2 * m0 * q]));
+    }
+    __syncthreads();
+    // rows: the SX points of each q, giving z[8 m + q] = (x[2 (8 m + q)], ...)
+    for (int e = tid; e < NZ * 8; e += T) {
+        const int row = e >> 3, q = e & 7;
+        double2 w[SX];
+#pragma unroll
+        for (int m = 0; m < SX; ++m) w[m] = sh[row * LD + swz(SX * q + m)];
+        dft<SX, true>(w);
+        double* dst = x + ((size_t) row * ny + j) * NX + 2 * q;
+#pragma unroll
+        for (int m = 0; m < SX; ++m) *(d2u8*) (dst + 16 * m) = d2u8{w[m].x * scale, w[m].y * scale};
     }
 }
 
@@ -439,6 +685,31 @@ static ibm_status fft_alloc(ibm_ctx* ctx, ibm_fft* p, size_t bytes, void** out)
     return IBM_OK;
 }
 
+// The plane kernels of nx x nz points, or null where the sizes are not among
+// theirs (32 to 128: a larger plane does not fit the LDS).
+struct plane_kernels {
+    void (*forward)(int, const double*, double2*, const double2*, const double2*);
+    void (*inverse)(int, const double2*, double*, double, const double2*, const double2*);
+    int threads;
+    size_t lds;
+};
+
+template <int LX, int LZ>
+static plane_kernels plane_of()
+{
+    return {plane_forward_kernel<LX, LZ>, plane_inverse_kernel<LX, LZ>, plane_size<LX, LZ>::THREADS, plane_size<LX, LZ>::LDS};
+}
+
+constexpr int PLANE_MIN = 5, PLANE_SIZES = 3;
+static plane_kernels plane_kernels_of(int lx, int lz)
+{
+    static const plane_kernels table[PLANE_SIZES][PLANE_SIZES] = {{plane_of<5, 5>(), plane_of<5, 6>(), plane_of<5, 7>()},
+                                                                  {plane_of<6, 5>(), plane_of<6, 6>(), plane_of<6, 7>()},
+                                                                  {plane_of<7, 5>(), plane_of<7, 6>(), plane_of<7, 7>()}};
+    const int i = lx - PLANE_MIN, k = lz - PLANE_MIN;
+    return i >= 0 && i < PLANE_SIZES && k >= 0 && k < PLANE_SIZES ? table[i][k] : plane_kernels{};
+}
+
 static ibm_status fft_lds_attributes(ibm_ctx* ctx)
 {
     static std::mutex lock;
@@ -447,6 +718,12 @@ static ibm_status fft_lds_attributes(ibm_ctx* ctx)
     if (done) return IBM_OK;
     IBM_HIP(ctx, hipFuncSetAttribute((const void*) zfft_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int) MAX_DYNAMIC_LDS));
+    for (int lx = PLANE_MIN; lx < PLANE_MIN + PLANE_SIZES; ++lx)
+        for (int lz = PLANE_MIN; lz < PLANE_MIN + PLANE_SIZES; ++lz) {
+            const plane_kernels k = plane_kernels_of(lx, lz);
+            IBM_HIP(ctx, hipFuncSetAttribute((const void*) k.forward, hipFuncAttributeMaxDynamicSharedMemorySize, (int) k.lds));
+            IBM_HIP(ctx, hipFuncSetAttribute((const void*) k.inverse, hipFuncAttributeMaxDynamicSharedMemorySize, (int) k.lds));
+        }
     done = true;
     return IBM_OK;
 }
@@ -459,17 +736,28 @@ ibm_status fft_solve(ibm_ctx* ctx, ibm_fft* p, double sigma, double tau, const d
     if (!std::isfinite(sigma) || !std::isfinite(tau)) return fail(ctx, IBM_ERR_ARG, "non-finite operator coefficients");
     const int rows = p->ny * p->nz;
     const double points = (double) p->nx * p->ny * p->nz, coeffs = (double) p->nh * p->ny * p->nz;
-    // b read and x written once; the coefficients written and read four times
-    prof_scope prof(ctx, "fft_solve", 8.0 * 2.0 * points + 16.0 * 8.0 * coeffs);
+    const plane_kernels plane = plane_kernels_of(p->lx, p->lz);
+    // Planes wherever their sizes fit: both transforms of 128 x ny x 128 points
+    // take 27 (planes 14) us at ny = 128, 15 (12) at 32 and 10 (10) at 4; of
+    // 32 x ny x 32 7 to 8 (4 to 5) at any ny.
+    const bool by_planes = plane.forward != nullptr;
+    // b read and x written once; the coefficients written and read twice by
+    // planes, four times by passes
+    prof_scope prof(ctx, "fft_solve", 8.0 * 2.0 * points + 16.0 * (by_planes ? 4.0 : 8.0) * coeffs);
     const int rpb = FFT_THREADS / (p->nx / 2);
     const size_t xlds = sizeof(double2) * (rpb * p->nx + p->nx / 2);
-    xfft_forward_kernel<<<(rows + rpb - 1) / rpb, FFT_THREADS, xlds, ctx->stream>>>(p->nx, p->lx, rows, b, p->spec,
-                                                                                      p->twx);
-    IBM_LAUNCH_CHECK(ctx);
     const dim3 zgrid((p->nh + ZT - 1) / ZT, p->ny);
     const size_t zlds = sizeof(double2) * (ZT * p->nz + p->nz / 2);
-    zfft_kernel<<<zgrid, FFT_THREADS, zlds, ctx->stream>>>(p->nh, p->ny, p->nz, p->lz, p->spec, p->twz, 0);
-    IBM_LAUNCH_CHECK(ctx);
+    if (by_planes) {
+        plane.forward<<<p->ny, plane.threads, plane.lds, ctx->stream>>>(p->ny, b, p->spec, p->twx, p->twz);
+        IBM_LAUNCH_CHECK(ctx);
+    } else {
+        xfft_forward_kernel<<<(rows + rpb - 1) / rpb, FFT_THREADS, xlds, ctx->stream>>>(p->nx, p->lx, rows, b, p->spec,
+                                                                                        p->twx);
+        IBM_LAUNCH_CHECK(ctx);
+        zfft_kernel<<<zgrid, FFT_THREADS, zlds, ctx->stream>>>(p->nh, p->ny, p->nz, p->lz, p->spec, p->twz, 0);
+        IBM_LAUNCH_CHECK(ctx);
+    }
     const int singular = sigma == 0.0 && p->neumann;
     const dim3 tgrid((p->nh + LINE_MODES - 1) / LINE_MODES, p->nz);
     auto lines = [&](auto kernel) {
@@ -481,10 +769,16 @@ ibm_status fft_solve(ibm_ctx* ctx, ibm_fft* p, double sigma, double tau, const d
     else if (p->ny <= 16 * LINE_CHUNKS) lines(line_kernel<16>);
     else lines(line_kernel<(MAX_WALL_POINTS + LINE_CHUNKS - 1) / LINE_CHUNKS>);
     IBM_LAUNCH_CHECK(ctx);
+    const double scale = 1.0 / ((double) p->nx * p->nz);
+    if (by_planes) {
+        plane.inverse<<<p->ny, plane.threads, plane.lds, ctx->stream>>>(p->ny, p->spec, x, scale, p->twx, p->twz);
+        IBM_LAUNCH_CHECK(ctx);
+        return IBM_OK;
+    }
     zfft_kernel<<<zgrid, FFT_THREADS, zlds, ctx->stream>>>(p->nh, p->ny, p->nz, p->lz, p->spec, p->twz, 1);
     IBM_LAUNCH_CHECK(ctx);
-    xfft_inverse_kernel<<<(rows + rpb - 1) / rpb, FFT_THREADS, xlds, ctx->stream>>>(
-        p->nx, p->lx, rows, p->spec, x, 1.0 / ((double) p->nx * p->nz), p->twx);
+    xfft_inverse_kernel<<<(rows + rpb - 1) / rpb, FFT_THREADS, xlds, ctx->stream>>>(p->nx, p->lx, rows, p->spec, x, scale,
+                                                                                    p->twx);
     IBM_LAUNCH_CHECK(ctx);
     return IBM_OK;
 }
