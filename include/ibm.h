@@ -196,8 +196,8 @@ ibm_status ibm_spread_sets_noalloc(ibm_ctx* ctx, const ibm_grid* grids, ibm_delt
  * of component c.  Every periodic axis must have a multiple of 8 cells.
  * The spread bins every marker into 8 x 8 x 8-cell bricks of its box,
  * accumulates each brick's stencils once in a 64-bit fixed-point LDS tile
- * and merges the tiles: deterministic, no floating-point atomics.  The call
- * synchronises the context stream to upload the offsets. */
+ * and merges the tiles: deterministic, no floating-point atomics.  Above
+ * 2047 boxes the call synchronises the context stream to upload the offsets. */
 ibm_status ibm_spread_boxes(ibm_ctx* ctx, const ibm_grid* grids, ibm_delta delta, int nboxes, const int* offsets,
                             const double* x, const double* f, double* const* fe);
 /* The matching interpolation: ul (SoA, offsets[nboxes] markers) from

@@ -44,7 +44,8 @@ def test_blocks_and_short_axes(ibm, orc, ctx, cells, walls, n):
         assert np.abs(ul - ref).max() <= 1e-12 * max(np.abs(u).max() for u in ue), delta
 
 
-@pytest.mark.parametrize("counts", [[3], [0, 5, 0, 0, 200, 1, 0], [1] * 63 + [0, 2], [0] * 64 + [70], [2, 0] * 2100 + [300]])
+@pytest.mark.parametrize("counts", [[3], [0, 5, 0, 0, 200, 1, 0], [1] * 63 + [0, 2], [0] * 64 + [70], [2, 0] * 2100 + [300],
+                                    [1] * 511, [1] * 512, [1] * 2047, [1] * 2048])
 def test_boxes_of_uneven_counts(ibm, orc, ctx, counts):
     cells = (8, 8, 8)
     spec, grids, refinement = _domain(ibm, cells, ())
