@@ -21,9 +21,10 @@
 //   16  split BF16: a = a_hi + a_lo with a_hi = bf16(a), a_lo = bf16(a -
 //       a_hi); a b ~ a_hi b_hi + a_hi b_lo + a_lo b_hi with
 //       v_mfma_f32_16x16x32_bf16 and FP32 accumulation.
-// The block tile is 128 (samples) x 128 (columns) with the contraction
-// staged through LDS in 128-byte rows (144-byte stride, conflict-free for
-// the 16-byte fragment reads), four waves each owning a 64 x 64 quadrant.
+// The block tile is 128 (samples) x 128 (columns), or 64 x 64 (FP32, and split
+// BF16 of few tiles), with the contraction staged through LDS in 128-byte rows
+// (144-byte stride, conflict-free for the 16-byte fragment reads), four waves
+// each owning a quadrant.
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <cstring>
@@ -139,7 +140,7 @@ __device__ inline void mfma_step(const u4& xa, const u4& eb, const u4& xa_lo, co
     }
 }
 
-// One 128 x 128 tile of Y per block.  The MFMA "A" operand is the X tile
+// One T x T tile of Y per block.  The MFMA "A" operand is the X tile
 // (output rows = columns of Y) and "B" the operator tile, so a lane's four
 // results are four columns of Y at one sample row and the 16 lanes of a
 // group store 16 consecutive samples (128 contiguous bytes).
@@ -151,16 +152,16 @@ __device__ inline void mfma_step(const u4& xa, const u4& eb, const u4& xa_lo, co
 // Results: lane l holds four rows of column l % 16: rows 4 (l / 16) + r,
 // r = 0..3, for the FP32-accumulating instructions, but rows (l / 16) + 4 r
 // for v_mfma_f64_16x16x4 (both measured on gfx950).
-template <int MODE, int WN, int RB = ROWB, int NB = 1>
+template <int MODE, int WN, int RB = ROWB, int NB = 1, int T = TILE>
 __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 {
     constexpr int PL = planes(MODE);
     constexpr int THREADS = 128 * WN;                // waves: 2 along the samples x WN along the columns
-    constexpr int JN = 8 / WN;                       // 16-column blocks per wave
+    constexpr int IN = T / 32, JN = T / 16 / WN;     // 16-sample and 16-column blocks per wave
     constexpr int RS = RB + 16;                      // LDS row stride: 16-row fragment reads hit disjoint banks
-    constexpr int LOADS = TILE * RB / 16 / THREADS;  // 16-byte staging loads per thread, tile and plane
+    constexpr int LOADS = T * RB / 16 / THREADS;     // 16-byte staging loads per thread, tile and plane
     using acc_t = typename std::conditional<MODE == MODE_F64, d4, f4>::type;
-    __shared__ __attribute__((aligned(16))) unsigned char ldsb[NB][PL][2][TILE * RS];
+    __shared__ __attribute__((aligned(16))) unsigned char ldsb[NB][PL][2][T * RS];
 
     // Blocks reach the XCDs round-robin (block i on XCD i % 8).  XCD x takes
     // the x-th eighth of every group's tiles, in order, so that the XCDs get
@@ -193,8 +194,8 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
     const unsigned char* srcX[PL];
 #pragma unroll
     for (int p = 0; p < PL; ++p) {
-        srcE[p] = g.E[p] + (long) tm * TILE * row_bytes;
-        srcX[p] = g.X[p] + (long) tn * TILE * row_bytes;
+        srcE[p] = g.E[p] + (long) tm * T * row_bytes;
+        srcX[p] = g.X[p] + (long) tn * T * row_bytes;
     }
     u4 pe[PL][LOADS], px[PL][LOADS];
     long goff[LOADS];
@@ -213,11 +214,11 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
             px[p][i] = *(const u4*) (srcX[p] + goff[i] + (long) (c) * RB);         \
         }
 
-    acc_t acc[JN][4];
+    acc_t acc[JN][IN];
 #pragma unroll
     for (int j = 0; j < JN; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[j][i] = acc_t{};
+        for (int i = 0; i < IN; ++i) acc[j][i] = acc_t{};
 
     const int frow = lane & 15, fgrp = lane >> 4;
 #define RBF_STORE(buf)                                                                \
@@ -254,16 +255,16 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
                 RBF_LOAD(c + 1);
             }
         }
-        const unsigned char (*lds)[2][TILE * RS] = ldsb[buf];
+        const unsigned char (*lds)[2][T * RS] = ldsb[buf];
 #pragma unroll
         for (int s = 0; s < RB / 64; ++s) {
-            u4 ef[PL][4], xf[PL][JN];
+            u4 ef[PL][IN], xf[PL][JN];
             const int off = s * 64 + fgrp * 16;
 #pragma unroll
             for (int p = 0; p < PL; ++p) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    ef[p][i] = *(const u4*) (&lds[p][0][(wm * 64 + i * 16 + frow) * RS + off]);
+                for (int i = 0; i < IN; ++i)
+                    ef[p][i] = *(const u4*) (&lds[p][0][(wm * 16 * IN + i * 16 + frow) * RS + off]);
 #pragma unroll
                 for (int j = 0; j < JN; ++j)
                     xf[p][j] = *(const u4*) (&lds[p][1][(wn * 16 * JN + j * 16 + frow) * RS + off]);
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 #pragma unroll
             for (int j = 0; j < JN; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < IN; ++i)
                     mfma_step<MODE>(xf[0][j], ef[0][i], xf[PL - 1][j], ef[PL - 1][i], acc[j][i]);
         }
         if constexpr (NB == 2) __syncthreads();
@@ -279,13 +280,13 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 #undef RBF_LOAD
 #undef RBF_STORE
 
-    const int m_base = tm * TILE + wm * 64 + frow;
-    const int n_base = tn * TILE + wn * 16 * JN + (MODE == MODE_F64 ? fgrp : fgrp * 4);
+    const int m_base = tm * T + wm * 16 * IN + frow;
+    const int n_base = tn * T + wn * 16 * JN + (MODE == MODE_F64 ? fgrp : fgrp * 4);
     constexpr int RSTEP = MODE == MODE_F64 ? 4 : 1;
 #pragma unroll
     for (int j = 0; j < JN; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < IN; ++i) {
             int m = m_base + i * 16;
             if (m >= g.M) continue;
 #pragma unroll
@@ -505,6 +506,30 @@ void launch_f64(int wn, const gemm_groups& G, int blocks, hipStream_t stream)
     else rbf_gemm_kernel<MODE_F64, 2><<<blocks, NTHREADS, 0, stream>>>(G);
 }
 
+// FP32 products, and split-BF16 ones of few tiles, take 64 x 64 tiles with two
+// LDS buffers: a quarter of the work per tile fills the chip evenly where 128 x
+// 128 tiles leave CUs with one tile more than others or with none (a CU runs
+// 8832 x 2210 operators at 165 us a 128-column FP32 tile, however few there
+// are), and pads the columns to 64.  128 / 64, us, three operators 8832 x 2210:
+// FP32 with 24 / 192 / 600 / 1200 columns 167 / 304 / 748 / 1333 -> 91 / 212 /
+// 652 / 1185; split BF16 with 24 / 192 / 600 71 / 122 / 270 -> 45 / 114 / 328.
+// A small split-BF16 tile takes 0.38 of the time of a large one (measured on
+// operators from 330 x 300 to 8832 x 2210, 3 to 1200 columns), and the large
+// ones run in rounds of 256: the smaller estimate is taken.  The multiply
+// sequence of an output is the same either way.
+constexpr int SMALL_TILE = 64;
+bool small_tiles(int mode, const gemm_groups& G)
+{
+    if (mode == MODE_F32) return true;
+    long large = 0, small = 0;
+    for (int q = 0; q < G.count; ++q) {
+        const gemm_group& g = G.g[q];
+        large += (long) ((g.M + TILE - 1) / TILE) * ((g.N + TILE - 1) / TILE);
+        small += (long) ((g.M + SMALL_TILE - 1) / SMALL_TILE) * ((g.N + SMALL_TILE - 1) / SMALL_TILE);
+    }
+    return 0.38 * small < 256.0 * ((large + 255) / 256);
+}
+
 constexpr int THIN_COLUMNS = 64;       // columns of a full tile of rbf_thin_kernel
 
 void launch_thin(int k, const gemm_groups& T, hipStream_t stream)
@@ -696,15 +721,17 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
         flops += 2.0 * ops[b]->M * (double) N[b] * ops[b]->K * std::max(0, std::min(j1, ops[b]->nops) - j0);
     void* work = nullptr;
     if (nres) IBM_TRY(scratch(ctx, SLOT_RBF_WORK, res_work_bytes(nres, products), &work));
-    int blocks = 0;
+    int blocks = 0, edge = TILE;
     if (tiles) {
         // Longest contraction first: each XCD takes its share of the groups
         // in group order, so the short tiles come last and fill the tail.
         std::stable_sort(G.g, G.g + G.count, [](const gemm_group& a, const gemm_group& b) { return a.Kp > b.Kp; });
+        if (mode != MODE_F64 && small_tiles(mode, G)) edge = SMALL_TILE;
         tiles = 0;
         for (int q = 0; q < G.count; ++q) {
             G.g[q].first_tile = tiles;
-            tiles += (round_up(G.g[q].M, TILE) / TILE) * G.g[q].tiles_n;
+            G.g[q].tiles_n = (G.g[q].N + edge - 1) / edge;
+            tiles += (G.g[q].M + edge - 1) / edge * G.g[q].tiles_n;
         }
         G.total_tiles = tiles;
         // blocks: 8 x the most tiles any XCD takes (its share of every group)
@@ -737,9 +764,10 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
     if (mode == MODE_F64) {
         launch_f64(wn, G, blocks, stream);
     } else if (mode == MODE_F32) {
-        rbf_gemm_kernel<MODE_F32, 2><<<blocks, NTHREADS, 0, stream>>>(G);
+        rbf_gemm_kernel<MODE_F32, 2, ROWB, 2, SMALL_TILE><<<blocks, NTHREADS, 0, stream>>>(G);
     } else {
-        rbf_gemm_kernel<MODE_BF16X3, 2><<<blocks, NTHREADS, 0, stream>>>(G);
+        if (edge == SMALL_TILE) rbf_gemm_kernel<MODE_BF16X3, 2, ROWB, 2, SMALL_TILE><<<blocks, NTHREADS, 0, stream>>>(G);
+        else rbf_gemm_kernel<MODE_BF16X3, 2><<<blocks, NTHREADS, 0, stream>>>(G);
     }
     IBM_LAUNCH_CHECK(ctx);
     return IBM_OK;
