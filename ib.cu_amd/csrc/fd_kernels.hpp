@@ -92,8 +92,13 @@ template <typename T>
 struct advection_op {
     twopoint_op<T> A[3], B[3], D[3];
 };
+// All three components in one launch.
 template <typename T>
-ibm_status launch_advection(ibm_ctx* ctx, const advection_op<T>& Op, const T* const* u, int comp, T* H);
+struct advection_ops {
+    advection_op<T> c[3];
+};
+template <typename T>
+ibm_status launch_advection(ibm_ctx* ctx, const advection_ops<T>& ops, const T* const* u, T* const* H);
 
 
 // *out = max |x_i|

@@ -1447,25 +1447,45 @@ __global__ void __launch_bounds__(COARSE_THREADS) coarse_vcycle_kernel(coarse_le
 // Two-point operators (differential / average along one axis)
 // out = alpha * op x + beta * out
 // ---------------------------------------------------------------------------
+// The two source rows along the operator's axis of destination row r, and the
+// factors of their values: a row off a walled axis is the end row times the
+// ghost coefficient, one off a periodic axis wraps.  Selections and no
+// branches, so that all loads of a point are on their way together (the factor
+// 1 inside changes no bit).
+template <typename T>
+struct two_rows {
+    int i0, i1;
+    T f0, f1;
+};
+
+template <typename T>
+__device__ inline two_rows<T> rows_of(const twopoint_op<T>& P, int cols, int r)
+{
+    const T below = P.periodic ? T(1) : P.int_lo, above = P.periodic ? T(1) : P.int_hi;
+    auto row = [&](int idx, int& i, T& f) {
+        const int lo = P.periodic ? idx + cols : 0, hi = P.periodic ? idx - cols : cols - 1;
+        i = idx < 0 ? lo : (idx >= cols ? hi : idx);
+        f = idx < 0 ? below : (idx >= cols ? above : T(1));
+    };
+    two_rows<T> w;
+    row(r - P.s1, w.i0, w.f0);
+    row(r + 1 - P.s1, w.i1, w.f1);
+    return w;
+}
+
 // Value of the operator at destination point c.
 template <typename T>
 __device__ inline T twopoint_value(const twopoint_op<T>& P, const int c[3], const T* __restrict__ x)
 {
     // 32-bit indices: the launchers keep every grid below 2^32 points
     const int v = P.view;
-    const int cols = P.sn[v];
     const unsigned sn0 = (unsigned) P.sn[0], sn1 = (unsigned) P.sn[1];
     const unsigned stride = v == 0 ? 1u : (v == 1 ? sn0 : sn0 * sn1);
-    int base[3] = {c[0], c[1], c[2]};
-    base[v] = 0;
-    const unsigned b0 = (unsigned) base[0] + sn0 * ((unsigned) base[1] + sn1 * (unsigned) base[2]);
-    auto fetch = [&](int idx) -> T {
-        if (idx >= 0 && idx < cols) return x[b0 + stride * (unsigned) idx];
-        if (P.periodic) return x[b0 + stride * (unsigned) (idx < 0 ? idx + cols : idx - cols)];
-        return idx < 0 ? P.int_lo * x[b0] : P.int_hi * x[b0 + stride * (unsigned) (cols - 1)];
-    };
-    const int r = c[v];
-    return P.c0 * fetch(r - P.s1) + P.c1 * fetch(r + 1 - P.s1);
+    const int r = v == 0 ? c[0] : (v == 1 ? c[1] : c[2]);
+    const unsigned b0 = (v == 0 ? 0u : (unsigned) c[0]) +
+                        sn0 * ((v == 1 ? 0u : (unsigned) c[1]) + sn1 * (v == 2 ? 0u : (unsigned) c[2]));
+    const two_rows<T> w = rows_of(P, v == 0 ? P.sn[0] : (v == 1 ? P.sn[1] : P.sn[2]), r);
+    return P.c0 * (w.f0 * x[b0 + stride * (unsigned) w.i0]) + P.c1 * (w.f1 * x[b0 + stride * (unsigned) w.i1]);
 }
 
 template <typename T>
@@ -1487,101 +1507,101 @@ __global__ void twopoint_kernel(twopoint_op<T> P, T alpha, const T* __restrict__
     out[t] = o;
 }
 
-// One point of a two-point operator whose source values come from a functor
-// src(x, y, z) of source-grid coordinates (same fetch rules as
-// twopoint_kernel: periodic wrap, or the ghost coefficient times the end
-// value).
-template <typename T, typename F>
-__device__ inline T twopoint_at(const twopoint_op<T>& P, int x, int y, int z, const F& src)
-{
-    int c[3] = {x, y, z};
-    const int v = P.view, cols = P.sn[v], r = c[v];
-    auto fetch = [&](int idx) -> T {
-        if (idx < 0 || idx >= cols) {
-            if (P.periodic) {
-                idx = idx < 0 ? idx + cols : idx - cols;
-            } else {
-                T g = idx < 0 ? P.int_lo : P.int_hi;
-                c[v] = idx < 0 ? 0 : cols - 1;
-                return g * src(c[0], c[1], c[2]);
-            }
-        }
-        c[v] = idx;
-        return src(c[0], c[1], c[2]);
-    };
-    T f0 = fetch(r - P.s1);
-    T f1 = fetch(r + 1 - P.s1);
-    return P.c0 * f0 + P.c1 * f1;
-}
-
-// twopoint_at with the view a compile-time constant (no run-time indexing
-// of the coordinate triple); the same fetches and the same arithmetic.
-template <int V, typename T, typename F>
-__device__ inline T twopoint_at_v(const twopoint_op<T>& P, int x, int y, int z, const F& src)
-{
-    const int cols = P.sn[V], r = V == 0 ? x : (V == 1 ? y : z);
-    auto at = [&](int idx) -> T {
-        return V == 0 ? src(idx, y, z) : (V == 1 ? src(x, idx, z) : src(x, y, idx));
-    };
-    auto fetch = [&](int idx) -> T {
-        if (idx < 0 || idx >= cols) {
-            if (P.periodic) {
-                idx = idx < 0 ? idx + cols : idx - cols;
-            } else {
-                T g = idx < 0 ? P.int_lo : P.int_hi;
-                return g * at(idx < 0 ? 0 : cols - 1);
-            }
-        }
-        return at(idx);
-    };
-    T f0 = fetch(r - P.s1);
-    T f1 = fetch(r + 1 - P.s1);
-    return P.c0 * f0 + P.c1 * f1;
-}
-
 // ins::advection for one component in one pass:
 //   H^i = sum_j D_j [ (A_i u^j) o (A_j u^i) ]
 // evaluated point by point on u^i's grid (j summed in order 0, 1, 2).  The
 // component I is a template parameter, so every operator's axis is known
-// at compile time (D_j and A_j along j, A_i along I).
+// at compile time (D_j and A_j along j, A_i along I; for j = I both averages
+// are the same, which the launcher checks).  Bound by instruction issue: 20
+// loads and 40 multiply-adds per point, and without care ten times as many
+// instructions for their rows.  A thread therefore marches along z: its rows
+// in x and y are found once, those in z are the workgroup's (scalar), and the
+// product of a plane is kept for the next.  All components, us: 108 x 108 x 126
+// points 80 with a thread per point and a branch per fetch, 82 without the
+// branches, 62 marching, 55 with the components in one launch (fewer tails);
+// 128 x 256 x 128 226 / 122.
+// The parts of one launch: component i's blocks first[i] to first[i + 1].
+struct advection_split {
+    unsigned first[4], plane_blocks[3];
+    int planes[3];
+};
+
 template <typename T, int I>
-__global__ void advection_kernel(advection_op<T> Op, const T* __restrict__ u0, const T* __restrict__ u1,
-                                 const T* __restrict__ u2, T* __restrict__ H)
+__device__ inline void advect(const advection_op<T>& Op, const advection_split& S, unsigned block, const T* __restrict__ u0,
+                              const T* __restrict__ u1, const T* __restrict__ u2, T* __restrict__ H)
 {
+    const unsigned plane_blocks = S.plane_blocks[I];
+    const int planes = S.planes[I];
     const int* dn = Op.D[0].dn;
-    const size_t total = (size_t) dn[0] * dn[1] * dn[2];
-    size_t t = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= total) return;
-    const unsigned tt = (unsigned) t, q = tt / (unsigned) dn[0];
-    const int cx = (int) (tt - q * (unsigned) dn[0]);
-    const int cy = (int) (q % (unsigned) dn[1]);
-    const int cz = (int) (q / (unsigned) dn[1]);
+    const unsigned n0 = (unsigned) dn[0], area = n0 * (unsigned) dn[1];
+    const unsigned slab = block / plane_blocks, t = (block - slab * plane_blocks) * 256 + threadIdx.x;
+    if (t >= area) return;
+    const int cy = (int) (t / n0), cx = (int) (t - (unsigned) cy * n0);
+    const int z0 = (int) slab * planes, z1 = min(z0 + planes, dn[2]);
     const T* ui = I == 0 ? u0 : (I == 1 ? u1 : u2);
-    T acc = 0;
-    auto term = [&](auto J) {
+    // 32-bit indices inside a plane: the launcher keeps every grid below 2^32 points
+    auto at = [](const T* u, const int* n, int x, int y, int z) -> T {
+        const T* plane = u + (size_t) z * (unsigned) n[0] * (unsigned) n[1];
+        return plane[(unsigned) x + (unsigned) n[0] * (unsigned) y];
+    };
+    // (A_i u^j) o (A_j u^i) at row p along j of the point (cx, cy, z)
+    auto product = [&](auto J, int p, int z) -> T {
         constexpr int j = decltype(J)::value;
         const twopoint_op<T>& A = Op.A[j];
         const twopoint_op<T>& B = Op.B[j];
         const T* uj = j == 0 ? u0 : (j == 1 ? u1 : u2);
-        // 32-bit indices: the launcher keeps every grid below 2^32 points
-        const unsigned as0 = (unsigned) A.sn[0], as1 = (unsigned) A.sn[1];
-        const unsigned bs0 = (unsigned) B.sn[0], bs1 = (unsigned) B.sn[1];
-        auto prod = [&](int x, int y, int z) -> T {
-            T a = twopoint_at_v<I>(A, x, y, z, [&](int p, int q2, int r) -> T {
-                return uj[(unsigned) p + as0 * ((unsigned) q2 + as1 * (unsigned) r)];
-            });
-            T b = twopoint_at_v<j>(B, x, y, z, [&](int p, int q2, int r) -> T {
-                return ui[(unsigned) p + bs0 * ((unsigned) q2 + bs1 * (unsigned) r)];
-            });
-            return a * b;
-        };
-        T d = twopoint_at_v<j>(Op.D[j], cx, cy, cz, prod);
-        acc = j == 0 ? d : acc + d;
+        const int x = j == 0 ? p : cx, y = j == 1 ? p : cy, w = j == 2 ? p : z;
+        const two_rows<T> a = rows_of(A, A.sn[I], I == 0 ? x : (I == 1 ? y : w));
+        const T va = A.c0 * (a.f0 * at(uj, A.sn, I == 0 ? a.i0 : x, I == 1 ? a.i0 : y, I == 2 ? a.i0 : w)) +
+                     A.c1 * (a.f1 * at(uj, A.sn, I == 0 ? a.i1 : x, I == 1 ? a.i1 : y, I == 2 ? a.i1 : w));
+        if constexpr (j == I) return va * va;
+        const two_rows<T> b = rows_of(B, B.sn[j], p);
+        const T vb = B.c0 * (b.f0 * at(ui, B.sn, j == 0 ? b.i0 : x, j == 1 ? b.i0 : y, j == 2 ? b.i0 : w)) +
+                     B.c1 * (b.f1 * at(ui, B.sn, j == 0 ? b.i1 : x, j == 1 ? b.i1 : y, j == 2 ? b.i1 : w));
+        return va * vb;
     };
-    term(std::integral_constant<int, 0>{});
-    term(std::integral_constant<int, 1>{});
-    term(std::integral_constant<int, 2>{});
-    H[t] = acc;
+    const std::integral_constant<int, 0> X;
+    const std::integral_constant<int, 1> Y;
+    const std::integral_constant<int, 2> Z;
+    const twopoint_op<T>& D0 = Op.D[0];
+    const twopoint_op<T>& D1 = Op.D[1];
+    const twopoint_op<T>& D2 = Op.D[2];
+    const two_rows<T> dx = rows_of(D0, D0.sn[0], cx), dy = rows_of(D1, D1.sn[1], cy);
+    int kept_row = -1;
+    T kept = 0;
+    for (int z = z0; z < z1; ++z) {
+        T acc = D0.c0 * (dx.f0 * product(X, dx.i0, z)) + D0.c1 * (dx.f1 * product(X, dx.i1, z));
+        acc = acc + (D1.c0 * (dy.f0 * product(Y, dy.i0, z)) + D1.c1 * (dy.f1 * product(Y, dy.i1, z)));
+        const two_rows<T> dz = rows_of(D2, D2.sn[2], z);
+        const T before = dz.i0 == kept_row ? kept : product(Z, dz.i0, z);
+        kept = product(Z, dz.i1, z);
+        kept_row = dz.i1;
+        acc = acc + (D2.c0 * (dz.f0 * before) + D2.c1 * (dz.f1 * kept));
+        H[(size_t) z * area + t] = acc;
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256, 4)
+advection_kernel(advection_ops<T> Op, advection_split S, const T* __restrict__ u0, const T* __restrict__ u1,
+                 const T* __restrict__ u2, T* __restrict__ H0, T* __restrict__ H1, T* __restrict__ H2)
+{
+    // XCD x takes the x-th eighth of a component's blocks: neighbouring planes in one L2
+    unsigned k = blockIdx.x >> 3;
+    const unsigned xcd = blockIdx.x & 7;
+    auto run = [&](auto I) {
+        constexpr int i = decltype(I)::value;
+        const unsigned n = S.first[i + 1] - S.first[i], lo = xcd * n / 8, hi = (xcd + 1) * n / 8;
+        if (k < hi - lo) {
+            advect<T, i>(Op.c[i], S, lo + k, u0, u1, u2, i == 0 ? H0 : (i == 1 ? H1 : H2));
+            return true;
+        }
+        k -= hi - lo;
+        return false;
+    };
+    if (run(std::integral_constant<int, 0>{})) return;
+    if (run(std::integral_constant<int, 1>{})) return;
+    run(std::integral_constant<int, 2>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -2115,28 +2135,47 @@ ibm_status launch_twopoint(ibm_ctx* ctx, const twopoint_op<T>& P, T alpha, const
 }
 
 template <typename T>
-ibm_status launch_advection(ibm_ctx* ctx, const advection_op<T>& Op, const T* const* u, int comp, T* H)
+ibm_status launch_advection(ibm_ctx* ctx, const advection_ops<T>& ops, const T* const* u, T* const* H)
 {
-    const int* dn = Op.D[0].dn;
-    size_t n = (size_t) dn[0] * dn[1] * dn[2];
-    if (!n) return IBM_OK;
-    if (n > MAX_GRID_POINTS) return fail(ctx, IBM_ERR_SIZE, "grid too large");
-    double nsrc = 0;
-    for (int d = 0; d < 3; ++d) {
-        const size_t na = (size_t) Op.A[d].sn[0] * Op.A[d].sn[1] * Op.A[d].sn[2];
-        const size_t nb = (size_t) Op.B[d].sn[0] * Op.B[d].sn[1] * Op.B[d].sn[2];
-        if (na > MAX_GRID_POINTS || nb > MAX_GRID_POINTS) return fail(ctx, IBM_ERR_SIZE, "grid too large");
-        nsrc += (double) na;
+    advection_split S{};
+    double work = 0;
+    for (int i = 0; i < 3; ++i) {
+        const advection_op<T>& Op = ops.c[i];
+        const int* dn = Op.D[0].dn;
+        const size_t n = (size_t) dn[0] * dn[1] * dn[2];
+        if (n > MAX_GRID_POINTS) return fail(ctx, IBM_ERR_SIZE, "grid too large");
+        for (int d = 0; d < 3; ++d) {
+            const size_t na = (size_t) Op.A[d].sn[0] * Op.A[d].sn[1] * Op.A[d].sn[2];
+            const size_t nb = (size_t) Op.B[d].sn[0] * Op.B[d].sn[1] * Op.B[d].sn[2];
+            if (na > MAX_GRID_POINTS || nb > MAX_GRID_POINTS) return fail(ctx, IBM_ERR_SIZE, "grid too large");
+            work += (double) na;
+        }
+        work += (double) n;
+        for (int j = 0; j < 3; ++j)
+            if (Op.D[j].view != j || Op.B[j].view != j || Op.A[j].view != i)
+                return fail(ctx, IBM_ERR_ARG, "advection operators along unexpected axes");
+        const twopoint_op<T>&a = Op.A[i], &b = Op.B[i];
+        if (!std::equal(a.sn, a.sn + 3, b.sn) || a.s1 != b.s1 || a.periodic != b.periodic || a.c0 != b.c0 || a.c1 != b.c1 ||
+            a.int_lo != b.int_lo || a.int_hi != b.int_hi)
+            return fail(ctx, IBM_ERR_ARG, "advection operators differ in component %d's own average", i);
+        // planes per block: four blocks per CU of each component where the grid has them
+        const size_t plane_blocks = ((size_t) dn[0] * dn[1] + 255) / 256;
+        S.planes[i] = (int) std::min<size_t>(16, std::max<size_t>(1, plane_blocks * dn[2] / 1024));
+        S.plane_blocks[i] = (unsigned) plane_blocks;
+        S.first[i + 1] = S.first[i] + (unsigned) (plane_blocks * ((dn[2] + S.planes[i] - 1) / S.planes[i]));
     }
-    prof_scope prof(ctx, "advection", (double) sizeof(T) * (nsrc + n));   // u^0..2 read once, H^i written
-    if (comp < 0 || comp > 2) return fail(ctx, IBM_ERR_ARG, "advection component %d", comp);
-    for (int j = 0; j < 3; ++j)
-        if (Op.D[j].view != j || Op.B[j].view != j || Op.A[j].view != comp)
-            return fail(ctx, IBM_ERR_ARG, "advection operators along unexpected axes");
-    const unsigned blocks = (unsigned) ((n + 255) / 256);
-    if (comp == 0) advection_kernel<T, 0><<<blocks, 256, 0, ctx->stream>>>(Op, u[0], u[1], u[2], H);
-    else if (comp == 1) advection_kernel<T, 1><<<blocks, 256, 0, ctx->stream>>>(Op, u[0], u[1], u[2], H);
-    else advection_kernel<T, 2><<<blocks, 256, 0, ctx->stream>>>(Op, u[0], u[1], u[2], H);
+    if (!S.first[3]) return IBM_OK;
+    unsigned per_xcd = 0;
+    for (unsigned x = 0; x < 8; ++x) {
+        unsigned k = 0;
+        for (int i = 0; i < 3; ++i) {
+            const unsigned n = S.first[i + 1] - S.first[i];
+            k += (x + 1) * n / 8 - x * n / 8;
+        }
+        per_xcd = std::max(per_xcd, k);
+    }
+    prof_scope prof(ctx, "advection", (double) sizeof(T) * work);   // per component u^0..2 read once, H^i written
+    advection_kernel<T><<<8 * per_xcd, 256, 0, ctx->stream>>>(ops, S, u[0], u[1], u[2], H[0], H[1], H[2]);
     IBM_LAUNCH_CHECK(ctx);
     return IBM_OK;
 }
@@ -2346,7 +2385,7 @@ ibm_status prepare_coarse_vcycle(ibm_ctx* ctx, size_t lds_bytes)
     template ibm_status launch_twopoint<T>(ibm_ctx*, const twopoint_op<T>&, T, const T*, T, T*);      \
     template ibm_status launch_coarse_vcycle<T>(ibm_ctx*, const coarse_levels<T>&);                   \
     template ibm_status prepare_coarse_vcycle<T>(ibm_ctx*, size_t);                   \
-    template ibm_status launch_advection<T>(ibm_ctx*, const advection_op<T>&, const T* const*, int, T*);
+    template ibm_status launch_advection<T>(ibm_ctx*, const advection_ops<T>&, const T* const*, T* const*);
 IBM_INSTANTIATE(double)
 IBM_INSTANTIATE(float)
 template ibm_status launch_axpby<double, double>(ibm_ctx*, size_t, double, const double*, double, double*);

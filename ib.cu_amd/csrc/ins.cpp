@@ -206,8 +206,9 @@ ibm_status ibm_advection(ibm_ctx* ctx, const ibm_grid* u_grids, const double* co
     twopoint_op<double> avg_ij[3][3];      // A_i applied to u^j
     for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j) IBM_TRY(make_twopoint(u_grids[j], i, 1, &avg_ij[i][j], &ga[i][j]));
+    advection_ops<double> ops;
     for (int i = 0; i < 3; ++i) {
-        advection_op<double> Op;
+        advection_op<double>& Op = ops.c[i];
         for (int j = 0; j < 3; ++j) {
             const ibm_grid& g = ga[i][j];                        // grid of A_i u^j
             if (!same_points(g, ga[j][i])) return fail(ctx, IBM_ERR_SIZE, "advection products on different grids");
@@ -217,9 +218,8 @@ ibm_status ibm_advection(ibm_ctx* ctx, const ibm_grid* u_grids, const double* co
             Op.A[j] = avg_ij[i][j];
             Op.B[j] = avg_ij[j][i];
         }
-        IBM_TRY(launch_advection<double>(ctx, Op, u, i, H[i]));
     }
-    return IBM_OK;
+    return launch_advection<double>(ctx, ops, u, H);
 }
 
 } // extern "C"
