@@ -197,9 +197,11 @@ __global__ void bin_count_kernel(marker_sets sets, kgrids g, bin_desc bd, int wi
         double p[3] = {x[l], x[n + l], x[2 * n + l]};
         int q[3];
         bin = 0;
+        bool placed = true;                 // false at a NaN or infinite position
         int stride = 1;
         for (int j = 0; j < 3; ++j) {
             stencil_axis st = kstencil(g.a[bd.fc[j]][j], p[j]);
+            placed = placed && isfinite(st.d);
             q[j] = st.base + bd.fs[j];
             int qb = q[j] - bd.qmin[j];
             qb = qb < 0 ? 0 : (qb >= bd.nb[j] ? bd.nb[j] - 1 : qb);
@@ -219,10 +221,10 @@ __global__ void bin_count_kernel(marker_sets sets, kgrids g, bin_desc bd, int wi
             const double f0 = fabs(f[l]), f1 = fabs(f[n + l]), f2 = fabs(f[2 * n + l]);
             double a = f0 > f1 ? f0 : f1;
             a = a > f2 ? a : f2;
-            // A non-finite force is recorded as the canonical NaN, whose bit
-            // pattern exceeds every finite and infinite one, so it survives
-            // the integer maxima below and poisons the spread result.
-            if (!(isfinite(f0) && isfinite(f1) && isfinite(f2))) a = __longlong_as_double(0x7ff8000000000000ll);
+            // A non-finite force or position is recorded as the canonical NaN,
+            // whose bit pattern exceeds every finite and infinite one, so it
+            // survives the integer maxima below and poisons the spread result.
+            if (!(placed && isfinite(f0) && isfinite(f1) && isfinite(f2))) a = __longlong_as_double(0x7ff8000000000000ll);
             fbits = (unsigned long long) __double_as_longlong(a);
         }
     }
@@ -502,7 +504,7 @@ spread_brick_kernel(kgrids g, bin_desc bd, int delta, int total,
             for (int k = 0; k < n; ++k) pos_list[o + k] = b + k;
         }
     __syncthreads();
-    // A NaN or infinite force makes the bound non-finite: every point is then
+    // A NaN or infinite force or position makes the bound non-finite: every point is then
     // written as NaN (the accumulation below still runs, on a dummy quantum).
     const bool poisoned = !(bound_s <= 1.7976931348623157e308);
     int e2 = 0;
@@ -1090,9 +1092,11 @@ tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const i
         const int m = m0 + 64 * i;
         const bool valid = m < sets.total;
         int br[3], sub = 0;
+        bool placed = true;                 // false at a NaN or infinite position, whose weights are NaN
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             stencil_axis st = kstencil(g.a[bd.fc[j]][j], p[i][j]);
+            placed = placed && isfinite(st.d);
             int qb = st.base + bd.fs[j] - bd.qmin[j];
             qb = qb < 0 ? 0 : (qb >= bd.nb[j] ? bd.nb[j] - 1 : qb);
             br[j] = qb / TB;
@@ -1103,10 +1107,11 @@ tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const i
         const double f0 = fabs(f[i][0]), f1 = fabs(f[i][1]), f2 = fabs(f[i][2]);
         double a = f0 > f1 ? f0 : f1;
         a = a > f2 ? a : f2;
-        // A non-finite force is recorded as the canonical NaN, whose bit
-        // pattern exceeds every finite and infinite one, so it survives the
-        // integer maxima and poisons the spread result.
-        if (!(isfinite(f0) && isfinite(f1) && isfinite(f2))) a = __longlong_as_double(0x7ff8000000000000ll);
+        // A non-finite force or position is recorded as the canonical NaN,
+        // whose bit pattern exceeds every finite and infinite one, so it
+        // survives the integer maxima and poisons the spread result (the
+        // integers below cannot carry a NaN).
+        if (!(placed && isfinite(f0) && isfinite(f1) && isfinite(f2))) a = __longlong_as_double(0x7ff8000000000000ll);
         if (valid) {
             key[m] = bin[i];
             const unsigned long long bits = (unsigned long long) __double_as_longlong(a);

@@ -160,7 +160,9 @@ ibm_status ibm_profile_work(ibm_ctx* ctx, const char* name, double* total);
  * Grid points whose stencil index falls outside a solid dimension are
  * dropped (ib/indexing.h:35-62).  Every point of fe[c] is written (no
  * accumulation into existing contents).  Deterministic: the result does not
- * depend on scheduling (no floating-point atomics in global memory). */
+ * depend on scheduling (no floating-point atomics in global memory).  A NaN or
+ * infinite force or position makes every value of every component NaN (in
+ * each form of the spread; in a batch of boxes, in every box). */
 ibm_status ibm_spread(ibm_ctx* ctx, const ibm_grid* grids /* [3] */, ibm_delta delta,
                       int n, const double* x, const double* f,
                       double* const* fe /* [3] device pointers */);
