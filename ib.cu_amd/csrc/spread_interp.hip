@@ -1362,13 +1362,14 @@ tile_spread_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, int de
     const int b1 = (r / td.nbr[0]) % td.nbr[1];
     const int b2 = r / (td.nbr[0] * td.nbr[1]);
     const int bq[3] = {b0 * TB, b1 * TB, b2 * TB};
-    // The quantum's inverse is a power of two: applied to the force first, it
+    // The quantum's inverse is a power of two: applied to the scaled force, it
     // scales every product exactly as it would scale the finished one (a
     // product that ends at 1/2 or more has no subnormal factor on the way).
-    const double inv_q = scale->inv_q;
+    // Not to res3 alone: for forces near 1e-288 the inverse is near the end of
+    // the range and the product would be infinite.
+    const double inv_q = scale->inv_q, res3 = g.res3[c];
     // values of a force below this (in quanta) stay below 2^51: see make_scale
     const double fast_below = 0x1p51 / (delta == IBM_DELTA_BSPLINE3 ? 0.3 : 0.126);
-    const double force_scale = g.res3[c] * inv_q;
 #pragma unroll 1
     for (int c0 = s0; c0 < s1; c0 += CHUNK_MARKERS) {
         const int n = min(s1 - c0, CHUNK_MARKERS);
@@ -1414,7 +1415,7 @@ tile_spread_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, int de
                 const int rank = min(atomicAdd(&count[o[0] + 9 * (o[1] + 9 * o[2])], 1), 63);
                 at[k] = rank << 16 | atomicAdd(&level[rank], 1);
                 offsets01[i] = make_double2(d[0], d[1]);
-                offset2_force[i] = make_double2(d[2], f[k] * force_scale);
+                offset2_force[i] = make_double2(d[2], f[k] * res3 * inv_q);
                 corner[i] = (unsigned short) (o[0] + TT * (o[1] + TT * o[2]));
             }
         }
