@@ -1886,14 +1886,28 @@ ibm_status spread_tiles(ibm_ctx* ctx, const kgrids& kg, const bin_desc& bd, int 
     return IBM_OK;
 }
 
+// Whether the tiles of one box's bricks can be held in the context's scratch
+// (up to 16 GiB, kept like every scratch buffer): false, with the failure
+// cleared, where the device's memory is taken.
+bool tiles_held(ibm_ctx* ctx, const bin_desc& bd)
+{
+    void* p;
+    const std::string before = ctx->error;
+    if (scratch(ctx, SLOT_TILES, TILE_BYTES * (size_t) bricks_of(bd), &p) == IBM_OK) return true;
+    (void) hipGetLastError();
+    ctx->error = before;
+    return false;
+}
+
 // The public spread.  ibm_spread_sets and ibm_spread_sets_noalloc give the
 // same bits, so the path depends on the markers and grids alone: tiles where
 // a brick's tiles for the whole grid fit the fixed workspace, or where the
 // input is beyond what the fixed workspace takes at all; else (grids of few
-// bins and many mostly empty bricks) the brick kernel.  Measured (us, brick
-// kernel / tiles, binning included): C4 channel with 2.39 M markers 1802 /
-// 580, 100^3 periodic with 176,000 markers 268 / 120, one sphere of 2562
-// markers on 32^3 89 / 41.
+// bins and many mostly empty bricks, or no memory left for the tiles, where
+// the results are as accurate but not the same bits) the brick kernel.
+// Measured (us, brick kernel / tiles, binning included): C4 channel with
+// 2.39 M markers 1802 / 580, 100^3 periodic with 176,000 markers 268 / 120,
+// one sphere of 2562 markers on 32^3 89 / 41.
 ibm_status spread_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const marker_sets& sets,
                        double* const* fe, unsigned char* fixed_workspace = nullptr)
 {
@@ -1903,7 +1917,8 @@ ibm_status spread_sets(ibm_ctx* ctx, const ibm_grid* grids, int delta, const mar
     if (fixed_workspace) IBM_TRY(static_limits(ctx, sets.total, bd.nbins));
     IBM_TRY(narrow_axes_limit(ctx, kg));
     const bool beyond = (size_t) sets.total > STATIC_MAX_MARKERS || (size_t) bd.nbins > STATIC_MAX_BINS;
-    if (bricks_of(bd) <= (long long) STATIC_MAX_BRICKS || (beyond && tiles_fit(bd, 1)))
+    const bool by_tiles = bricks_of(bd) <= (long long) STATIC_MAX_BRICKS || (beyond && tiles_fit(bd, 1));
+    if (by_tiles && (fixed_workspace || tiles_held(ctx, bd)))
         return spread_tiles(ctx, kg, bd, delta, sets, 1, nullptr, fe, fixed_workspace);
     return spread_bricks(ctx, kg, bd, delta, sets, fe, fixed_workspace);
 }
@@ -1917,7 +1932,7 @@ ibm_status spread_sets_step(ibm_ctx* ctx, const ibm_grid* grids, int delta, int 
     kgrids kg;
     bin_desc bd;
     IBM_TRY(spread_setup(ctx, grids, delta, fe, &kg, &bd));
-    const bool fit = tiles_fit(bd, 1);
+    const bool fit = tiles_fit(bd, 1) && tiles_held(ctx, bd);
     if (!fit || !whole_bricks(kg)) IBM_TRY(narrow_axes_limit(ctx, kg));
     if (fit) return spread_tiles(ctx, kg, bd, delta, s, 1, nullptr, fe, nullptr);
     return spread_bricks(ctx, kg, bd, delta, s, fe, nullptr);
