@@ -15,8 +15,9 @@
 // the operator at creation, X per call.  One launch covers every
 // (cell type, operator) pair.  Precisions:
 //   64  few columns on v_mfma_f64_16x16x4 (rbf_thin_kernel); more through
-//       residues on the INT8 matrix cores (rbf_residue.hip), or, where an
-//       operator has no residue planes, on FP64 128 x 128 tiles;
+//       residues on the INT8 matrix cores (rbf_residue.hip), but for the
+//       columns that residues do not hold as well and for operators without
+//       residue planes, which run on FP64 128 x 128 tiles;
 //   32  v_mfma_f32_16x16x4 on FP32 operands, FP32 accumulation;
 //   16  split BF16: a = a_hi + a_lo with a_hi = bf16(a), a_lo = bf16(a -
 //       a_hi); a b ~ a_hi b_hi + a_hi b_lo + a_lo b_hi with
@@ -61,6 +62,7 @@ struct gemm_group {
     const unsigned char* E[2];   // operator planes: rows_pad x Kp elements
     const unsigned char* X[2];   // data-site planes: cols_pad x Kp elements
     double* Y;                   // M x N, column-major, ld = M
+    const int* list;             // LISTED: the number of columns to take of X and Y, then their indices
     int M, N, Kp, tiles_n, first_tile;
 };
 
@@ -68,6 +70,9 @@ struct gemm_groups {
     gemm_group g[MAX_GROUPS];
     int count, total_tiles;
 };
+
+// Listed columns up to this many run in rbf_thin_kernel.
+constexpr int LISTED_THIN = 64;
 
 __device__ inline uint16_t bf16_bits(float f)
 {
@@ -152,7 +157,11 @@ __device__ inline void mfma_step(const u4& xa, const u4& eb, const u4& xa_lo, co
 // Results: lane l holds four rows of column l % 16: rows 4 (l / 16) + r,
 // r = 0..3, for the FP32-accumulating instructions, but rows (l / 16) + 4 r
 // for v_mfma_f64_16x16x4 (both measured on gfx950).
-template <int MODE, int WN, int RB = ROWB, int NB = 1, int T = TILE>
+//
+// LISTED: only the columns of the group's list, unless they are few enough
+// for rbf_thin_kernel; the grid is that of all columns, since the list is
+// known on the device alone.
+template <int MODE, int WN, int RB = ROWB, int NB = 1, int T = TILE, bool LISTED = false>
 __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 {
     constexpr int PL = planes(MODE);
@@ -182,6 +191,8 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
     if (gi < 0) return;                              // whole block exits together
     const gemm_group g = G.g[gi];
     int tm = t / g.tiles_n, tn = t - tm * g.tiles_n;
+    const int N = LISTED ? g.list[0] : g.N;
+    if (LISTED && (N <= LISTED_THIN || tn * T >= N)) return;     // whole block
     const long row_bytes = (long) g.Kp * elem_bytes(MODE);
     const int nchunks = (int) (row_bytes / RB);
 
@@ -195,23 +206,25 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 #pragma unroll
     for (int p = 0; p < PL; ++p) {
         srcE[p] = g.E[p] + (long) tm * T * row_bytes;
-        srcX[p] = g.X[p] + (long) tn * T * row_bytes;
+        srcX[p] = g.X[p] + (LISTED ? 0 : (long) tn * T * row_bytes);
     }
     u4 pe[PL][LOADS], px[PL][LOADS];
-    long goff[LOADS];
+    long goff[LOADS], xoff[LOADS];
     int loff[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
         int idx = tid + THREADS * i;
         int r = idx / (RB / 16), q = idx % (RB / 16);
         goff[i] = (long) r * row_bytes + q * 16;
+        // past the list's end its last column again (not stored)
+        xoff[i] = LISTED ? (long) g.list[1 + min(tn * T + r, N - 1)] * row_bytes + q * 16 : goff[i];
         loff[i] = r * RS + q * 16;
     }
 #define RBF_LOAD(c)                                                                   \
     _Pragma("unroll") for (int p = 0; p < PL; ++p)                                    \
         _Pragma("unroll") for (int i = 0; i < LOADS; ++i) {                           \
             pe[p][i] = *(const u4*) (srcE[p] + goff[i] + (long) (c) * RB);         \
-            px[p][i] = *(const u4*) (srcX[p] + goff[i] + (long) (c) * RB);         \
+            px[p][i] = *(const u4*) (srcX[p] + xoff[i] + (long) (c) * RB);         \
         }
 
     acc_t acc[JN][IN];
@@ -292,7 +305,7 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 int n = n_base + j * 16 + r * RSTEP;
-                if (n < g.N) g.Y[m + (long) g.M * n] = (double) acc[j][i][r];
+                if (n < N) g.Y[m + (long) g.M * (LISTED ? g.list[1 + n] : n)] = (double) acc[j][i][r];
             }
         }
 }
@@ -309,7 +322,8 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 // copy rate); 715 x 503, 24 columns 70 -> 15.
 constexpr int THIN_ROWS = 32, THIN_RB = 256, THIN_RS = THIN_RB + 16, THIN_AHEAD = 3, THIN_THREADS = 128;
 
-template <int NB>
+// LISTED: as in rbf_gemm_kernel, up to LISTED_THIN columns.
+template <int NB, bool LISTED = false>
 __global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
 {
     constexpr int XLOADS = NB * 16 * THIN_RB / 16 / THIN_THREADS;    // 16-byte staging loads per thread
@@ -318,6 +332,8 @@ __global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
     while (gi + 1 < G.count && (int) blockIdx.x >= G.g[gi + 1].first_tile) ++gi;
     const gemm_group g = G.g[gi];
     const int tile = (int) blockIdx.x - g.first_tile, row_tile = tile / g.tiles_n, col0 = (tile - row_tile * g.tiles_n) * (16 * NB);
+    const int N = LISTED ? g.list[0] : g.N;
+    if (LISTED && (N > LISTED_THIN || col0 >= N)) return;        // whole block
     const int row0 = row_tile * THIN_ROWS + (threadIdx.x >> 6) * 16;
     const long row_bytes = (long) g.Kp * 8;
     const int nchunks = (int) (row_bytes / THIN_RB);
@@ -328,7 +344,7 @@ __global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
 #pragma unroll
     for (int i = 0; i < XLOADS; ++i) {
         const int idx = threadIdx.x + THIN_THREADS * i, r = idx / (THIN_RB / 16), q = idx % (THIN_RB / 16);
-        x[i] = g.X[0] + (long) (col0 + r) * row_bytes + q * 16;
+        x[i] = g.X[0] + (long) (LISTED ? g.list[1 + min(col0 + r, N - 1)] : col0 + r) * row_bytes + q * 16;
         xo[i] = r * THIN_RS + q * 16;
     }
     u4 pe[THIN_AHEAD][4], px[XLOADS];
@@ -387,7 +403,7 @@ __global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int n = col0 + b * 16 + fgrp + 4 * r;
-            if (n < g.N) g.Y[m + (long) g.M * n] = acc[b][r];
+            if (n < N) g.Y[m + (long) g.M * (LISTED ? g.list[1 + n] : n)] = acc[b][r];
         }
 }
 
@@ -622,6 +638,57 @@ size_t packed_offset(int count, ibm_rbf* const* ops, const int* N, const double*
     return at;
 }
 
+// Blocks of a grid in which XCD x takes the x-th eighth of every group's
+// tiles: 8 times the most that any XCD takes.
+int xcd_blocks(const gemm_groups& G)
+{
+    int per_xcd = 0;
+    for (int x = 0; x < 8; ++x) {
+        int n = 0;
+        for (int q = 0; q < G.count; ++q) {
+            const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : G.total_tiles) - G.g[q].first_tile;
+            n += (x + 1) * tq / 8 - x * tq / 8;
+        }
+        per_xcd = std::max(per_xcd, n);
+    }
+    return 8 * per_xcd;
+}
+
+// FP64 products of the columns that the residue path has listed.  The lists
+// are on the device: the thin kernel's launch takes the short ones and the
+// tiles' the others, blocks without columns leave at once.
+ibm_status listed_products(ibm_ctx* ctx, hipStream_t stream, int count, const res_product* p)
+{
+    constexpr int NB = 2;
+    gemm_groups thin{}, tiles{};
+    for (int i = 0; i < count; ++i) {
+        const res_packed x = res_columns_at(p[i].X, p[i].N, p[i].K);
+        gemm_group g{};
+        g.E[0] = g.E[1] = (const unsigned char*) p[i].E64;
+        g.X[0] = g.X[1] = (const unsigned char*) x.rows;
+        g.Y = p[i].Y;
+        g.list = p[i].list;
+        g.M = p[i].M;
+        g.N = p[i].N;
+        g.Kp = (int) x.ld;
+        g.tiles_n = (std::min(g.N, LISTED_THIN) + 16 * NB - 1) / (16 * NB);
+        g.first_tile = thin.total_tiles;
+        thin.g[thin.count++] = g;
+        thin.total_tiles += (g.M + THIN_ROWS - 1) / THIN_ROWS * g.tiles_n;
+        if (g.N <= LISTED_THIN) continue;
+        g.tiles_n = (g.N + TILE - 1) / TILE;
+        g.first_tile = tiles.total_tiles;
+        tiles.g[tiles.count++] = g;
+        tiles.total_tiles += (g.M + TILE - 1) / TILE * g.tiles_n;
+    }
+    rbf_thin_kernel<NB, true><<<thin.total_tiles, THIN_THREADS, 0, stream>>>(thin);
+    IBM_LAUNCH_CHECK(ctx);
+    if (tiles.count)
+        rbf_gemm_kernel<MODE_F64, DEFAULT_WAVES_N, ROWB, 2, TILE, true><<<xcd_blocks(tiles), 512, 0, stream>>>(tiles);
+    IBM_LAUNCH_CHECK(ctx);
+    return IBM_OK;
+}
+
 // The residue path's products of operators [j0, j1) (operands and outputs
 // unset without X / Y: for sizes only).
 int residue_products(int count, ibm_rbf* const* ops, const int* N, const double* const* X, double* const* Y, int j0,
@@ -632,10 +699,9 @@ int residue_products(int count, ibm_rbf* const* ops, const int* N, const double*
         const ibm_rbf& op = *ops[b];
         if (N[b] == 0 || !by_residues(&op, N[b])) continue;
         for (int j = j0; j < std::min(j1, op.nops); ++j)
-            out[n++] = res_product{op.res + (size_t) j * op.res_bytes,
+            out[n++] = res_product{op.res + (size_t) j * op.res_bytes, (const double*) op.plane(j, 0),
                                    X ? packed + packed_offset(count, ops, N, X, b, nullptr) : nullptr,
-                                   (const double*) op.plane(j, 0), X ? X[b] : nullptr,
-                                   Y ? Y[b] + (size_t) j * op.M * N[b] : nullptr, op.M, N[b], op.K, op.Kp};
+                                   Y ? Y[b] + (size_t) j * op.M * N[b] : nullptr, op.M, N[b], op.K, nullptr};
     }
     return n;
 }
@@ -734,21 +800,14 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
             tiles += (G.g[q].M + edge - 1) / edge * G.g[q].tiles_n;
         }
         G.total_tiles = tiles;
-        // blocks: 8 x the most tiles any XCD takes (its share of every group)
-        int per_xcd = 0;
-        for (int x = 0; x < 8; ++x) {
-            int n = 0;
-            for (int q = 0; q < G.count; ++q) {
-                const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : tiles) - G.g[q].first_tile;
-                n += (x + 1) * tq / 8 - x * tq / 8;
-            }
-            per_xcd = std::max(per_xcd, n);
-        }
-        blocks = 8 * per_xcd;
+        blocks = xcd_blocks(G);
     }
     const int wn = mode == MODE_F64 && tiles ? f64_variant(ctx, stream, G, blocks) : 2;
     prof_scope prof(ctx, "rbf_gemm", flops);
-    if (nres) IBM_TRY(res_products(ctx, stream, nres, products, (unsigned char*) work));
+    if (nres) {
+        IBM_TRY(res_products(ctx, stream, nres, products, (unsigned char*) work));
+        IBM_TRY(listed_products(ctx, stream, nres, products));
+    }
     for (int k = 0; k < 4; ++k) {
         gemm_groups& T = thin[k];
         if (!T.count) continue;
@@ -802,7 +861,7 @@ ibm_status ibm_rbf_create(ibm_ctx* ctx, int precision, int M, int K, int nops, c
         delete op;
         return fail(ctx, IBM_ERR_HIP, "out of device memory for a %zu-byte operator", bytes);
     }
-    // FP64 operators also keep their residue planes (fifteen bytes per
+    // FP64 operators also keep their residue planes (sixteen bytes per
     // element beside the eight); without the memory for them, or with
     // elements they cannot represent, every product runs on the FP64 matrix
     // cores.

@@ -11,12 +11,32 @@
 // The scales are
 //   sum_k |E'_mk| <= 2^62,   max_k |X'_kn| <= 2^54,
 // so |C| <= 2^116 < P / 2, P = prod p_l = 2^117.8, and the only errors are
-// the operands' rounding (2^-62 of the row's 1-norm, 2^-54 of the column's
-// maximum) and one rounding of the result.  Measured on the RBC and platelet
-// operators (values and all derivatives, 300 to 2210 data sites) against
-// long-double products, the error is 0.03 to 0.66 of the FP64 fused
-// multiply-add chain's in the 2-norm and 0.01 to 0.74 in the maximum; one
-// modulus fewer (2^109) would be 4 to 65 times the chain's.
+// the operands' rounding and one rounding of the result:
+//   |Y - E X|_mn <= 2^(ex - 55) sum_k |E_mk| + 2^(e - 63) sum_k |X_kn|
+//                   + 2^-53 |Y_mn|,
+// 2^e and 2^ex the powers of two above row m's 1-norm and column n's maximum.
+// That is a bound on norms.  An FP64 chain of fused multiply-adds is within
+// K 2^-53 sum_k |E_mk||X_kn| of each output, which can be far less where a
+// row's weight lies on a column's small values; so every column is checked,
+// and one that could exceed the chain's bound anywhere (plus the last
+// rounding) goes to the FP64 matrix cores:
+//   * a column whose values are all of one magnitude, more or less
+//     (COLUMN_NARROW; column_scale_kernel), cannot: sum_k |E_mk||X_kn| >=
+//     min_k |X_kn| sum_k |E_mk|.  Coordinates of a cell that does not lie
+//     across a coordinate plane are such columns;
+//   * of others (COLUMN_WIDE) a sixteenth product bounds sum_k |E_mk||X_kn|
+//     from below for every output: magnitudes rounded down to seven bits,
+//     S = sum_k floor(2^(7 - em) |E_mk|) floor(2^(7 - ex) |X_kn|) in INT32,
+//     2^em the power of two above row m's maximum, and
+//     S 2^(em + ex - 14) <= sum_k |E_mk||X_kn|.  For the few outputs below
+//     their row's threshold the sum itself is formed; one that is too small
+//     sends its column to the FP64 products;
+//   * columns of mostly negligible values (which would fail), or with a NaN
+//     or an infinity, go there at once (COLUMN_F64).
+// Measured on the RBC and platelet operators (values and all derivatives, 300
+// to 2210 data sites) against long-double products, the error is 0.03 to 0.66
+// of the FP64 fused multiply-add chain's in the 2-norm and 0.01 to 0.74 in
+// the maximum; one modulus fewer (2^109) would be 4 to 65 times the chain's.
 //
 // What bounds it: FP64 matrix cores are dense at 78.6 TFLOP/s (measured 72.6
 // for a large library product), INT8 at 5.0 POP/s; with random operands the
@@ -26,7 +46,6 @@
 // zeros), so 15 products are worth about 120 FP64 TFLOP/s.
 #include <hip/hip_runtime.h>
 #include <algorithm>
-#include <climits>
 #include <vector>
 #include "rbf_residue.hpp"
 
@@ -88,7 +107,6 @@ constexpr crt_table make_crt()
 }
 
 constexpr int SCALE_E = 62, SCALE_X = 54;
-constexpr int BAD_COLUMN = INT_MIN;           // scale of a column with a NaN or an infinity
 
 // 1.5 * 2^52: x + ROUND holds rint(x) in its low bits (|x| < 2^51), so that
 // x + ROUND - ROUND is rint(x) and the low word of x + ROUND, for an integer
@@ -153,25 +171,60 @@ __device__ inline size_t run_offset(int row, int run, int chunks)
     return ((size_t) (row >> 4) * chunks + (run >> 2)) * 1024 + ((row & 15) + 16 * (run & 3)) * 16;
 }
 
-// Scale of operator row m (one wavefront per row): 2^(62 - e), sum |E| < 2^e.
+// Sixteen consecutive elements' magnitudes in seven bits, |x| < 2^e.
+__device__ inline void store_magnitudes(const double (&x)[16], int e, unsigned char* at)
+{
+    i4 w;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        unsigned v = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v |= (unsigned) ldexp(fabs(x[4 * q + i]), 7 - e) << (8 * i);
+        w[q] = (int) v;
+    }
+    *(i4*) at = w;
+}
+
+// Of operator row m (one wavefront per row): the scale 2^(62 - e), sum |E| <
+// 2^e, of its integers; the exponent em of its maximum; and the least
+// magnitude product S for which the operands' rounding stays within the
+// chain's bound,
+//   2^(ex - 55) sum |E| + 2^(e - 63) K 2^ex <= K 2^-53 S 2^(em + ex - 14),
+// i.e. S >= 2^(12 - em) sum |E| / K + 2^(e - em + 4).
 __global__ __launch_bounds__(256) void operator_scale_kernel(const double* __restrict__ E, long lde, int M, int K,
-                                                             int* __restrict__ scale, int* __restrict__ flag)
+                                                             int* __restrict__ scale, int* __restrict__ top,
+                                                             int* __restrict__ least, int* __restrict__ flag)
 {
     const int m = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (m >= M) return;
-    double s = 0;
-    for (int k = lane; k < K; k += 64) s += fabs(E[k + lde * m]);
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    double s = 0, t = 0;
+    for (int k = lane; k < K; k += 64) {
+        const double v = fabs(E[k + lde * m]);
+        s += v;
+        t = fmax(t, v);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        s += __shfl_xor(s, off, 64);
+        t = fmax(t, __shfl_xor(t, off, 64));
+    }
     if (lane == 0) {
-        int e = 0;
-        if (!isfinite(s)) *flag = 1;
-        else if (s > 0) frexp(s * (1 + 0x1p-40), &e);      // the sum's own rounding
+        int e = 0, em = 0, bound = 0;
+        if (!isfinite(s)) {
+            *flag = 1;
+        } else if (s > 0) {
+            frexp(s * (1 + 0x1p-40), &e);      // the sum's own rounding
+            frexp(t, &em);
+            bound = (int) (ldexp(s, 12 - em) / K + ldexp(16.0, e - em)) + 2;
+        }
         scale[m] = SCALE_E - e;
+        top[m] = em;
+        least[m] = bound;
     }
 }
 
 __global__ __launch_bounds__(256) void operator_split_kernel(const double* __restrict__ E, long lde, int M, int K,
                                                              int rows, int chunks, const int* __restrict__ scale,
+                                                             const int* __restrict__ top,
                                                              unsigned char* __restrict__ planes, size_t plane)
 {
     const long i = (long) blockIdx.x * 256 + threadIdx.x;
@@ -180,83 +233,146 @@ __global__ __launch_bounds__(256) void operator_split_kernel(const double* __res
     // consecutive lanes take the 16 rows of a fragment, then its runs of k
     const int frag_row = (int) (i / ((long) runs * 16)), in = (int) (i - (long) frag_row * runs * 16);
     const int row = frag_row * 16 + (in & 15), run = in >> 4;
-    double h[16], d[16];
+    double x[16], h[16], d[16];
     const int s = row < M ? scale[row] : 0;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
         const int k = run * 16 + j;
-        split_element(row < M && k < K ? E[k + lde * row] : 0.0, s, h[j], d[j]);
+        x[j] = row < M && k < K ? E[k + lde * row] : 0.0;
+        split_element(x[j], s, h[j], d[j]);
     }
-    store_residues<0, RES_MODULI>(h, d, planes + run_offset(row, run, chunks), plane);
+    unsigned char* at = planes + run_offset(row, run, chunks);
+    store_residues<0, RES_MODULI>(h, d, at, plane);
+    store_magnitudes(x, row < M ? top[row] : 0, at + RES_MODULI * plane);
 }
 
+struct column_part {
+    const double* X;
+    res_packed to;
+    int N, K;
+};
 struct column_set {
-    res_columns c[RES_MAX_COLUMNS];
+    column_part c[RES_MAX_COLUMNS];
 };
 
-__device__ inline int* column_scales(const res_columns& c, int chunks)
-{
-    const size_t rows = (size_t) ((c.N + RES_BN - 1) / RES_BN) * RES_BN;
-    return (int*) (c.planes + RES_MODULI * rows * chunks * 64);
-}
-
-// Scale of column n: 2^(54 - e), max |x| < 2^e; one block per column.
+// Scale 2^(54 - ex) of column n's integers, max |x| < 2^ex, and its class; one
+// block per column.  Narrow: the operands' rounding is within the chain's
+// bound for every row,
+//   2^(ex - 55) + 2^-62 sum |x| <= K 2^-53 min |x|
+// (2^e <= 2 sum |E|): 1 : 800 for 2210 values of even distribution.  Columns
+// of which more than half lies below 2^-7 of the maximum have no seven-bit
+// magnitudes to speak of; those of a maximum below 2^-1000 are left to FP64 as
+// the sums here would underflow.
 __global__ __launch_bounds__(256) void column_scale_kernel(column_set set)
 {
-    __shared__ double part[4];
-    const res_columns c = set.c[blockIdx.y];
-    const int n = blockIdx.x;
+    __shared__ double part[3][4];
+    __shared__ int small[4];
+    const column_part& c = set.c[blockIdx.y];
+    const int n = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (n >= c.N) return;                                      // whole block
-    const double* x = c.X + (size_t) n * c.K;
-    double m = 0;
+    const int K = c.K;
+    const double* x = c.X + (size_t) n * K;
+    double top = 0, low = INFINITY, sum = 0;                   // sum: in units of 2^20, so that it cannot overflow
 #pragma unroll 8
-    for (int k = threadIdx.x; k < c.K; k += 256) {
+    for (int k = threadIdx.x; k < K; k += 256) {
         const double v = fabs(x[k]);
-        m = isfinite(v) ? fmax(m, v) : INFINITY;
+        top = isfinite(v) ? fmax(top, v) : INFINITY;
+        low = fmin(low, v);
+        sum += v * 0x1p-20;
     }
-    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    for (int off = 32; off > 0; off >>= 1) {
+        top = fmax(top, __shfl_xor(top, off, 64));
+        low = fmin(low, __shfl_xor(low, off, 64));
+        sum += __shfl_xor(sum, off, 64);
+    }
+    if (lane == 0) {
+        part[0][wave] = top;
+        part[1][wave] = low;
+        part[2][wave] = sum;
+    }
     __syncthreads();
+    top = fmax(fmax(part[0][0], part[0][1]), fmax(part[0][2], part[0][3]));
+    low = fmin(fmin(part[1][0], part[1][1]), fmin(part[1][2], part[1][3]));
+    sum = (part[2][0] + part[2][1]) + (part[2][2] + part[2][3]);
+    int ex = 0, kind = COLUMN_F64;
+    if (top == 0) {
+        kind = COLUMN_NARROW;
+    } else if (top >= 0x1p-1000 && isfinite(top)) {
+        frexp(top, &ex);
+        if (ldexp(1.0, ex - 22) + 0x1p-9 * sum <= K * 0x1p-20 * low) {
+            kind = COLUMN_NARROW;
+        } else {
+            int below = 0;
+            for (int k = threadIdx.x; k < K; k += 256) below += fabs(x[k]) < 0x1p-7 * top;
+            for (int off = 32; off > 0; off >>= 1) below += __shfl_xor(below, off, 64);
+            if (lane == 0) small[wave] = below;
+            __syncthreads();
+            kind = 2 * (small[0] + small[1] + small[2] + small[3]) > K ? COLUMN_F64 : COLUMN_WIDE;
+        }
+    }
     if (threadIdx.x == 0) {
-        m = fmax(fmax(part[0], part[1]), fmax(part[2], part[3]));
-        int e = 0;
-        if (isfinite(m) && m > 0) frexp(m, &e);
-        column_scales(c, (c.K + 63) / 64)[n] = isfinite(m) ? SCALE_X - e : BAD_COLUMN;
+        c.to.scale[n] = SCALE_X - ex;
+        c.to.kind[n] = kind;
     }
 }
 
 // Residues of 16 columns x 256 elements for a third of the moduli
-// (blockIdx.z): rows of 2 KB staged through LDS, so that both the loads and
-// the 1 KB fragment stores are contiguous (one block per column, whose
-// threads load and store scattered 128- and 16-byte pieces: 41 us for 600
-// columns of 2210 elements).  Padding columns get zeros.
+// (blockIdx.z; the last third also writes the magnitudes, and the FP64 rows of
+// the columns that may need them): rows of 2 KB staged through LDS, so that
+// both the loads and the 1 KB fragment stores are contiguous (one block per
+// column, whose threads load and store scattered 128- and 16-byte pieces:
+// 41 us for 600 columns of 2210 elements).  Padding columns, and those
+// without residues, get zeros.
 constexpr int SPLIT_PARTS = 3, SPLIT_K = 256, SPLIT_LD = SPLIT_K + SPLIT_K / 16 + 1;
 static_assert(RES_MODULI == 15);
 
 __global__ __launch_bounds__(256) void column_split_kernel(column_set set, int k_blocks)
 {
     __shared__ double sx[16][SPLIT_LD];                        // element k at k + k / 16
-    const res_columns c = set.c[blockIdx.y];
-    const int chunks = (c.K + 63) / 64, runs = chunks * 4;
-    const int rows = (c.N + RES_BN - 1) / RES_BN * RES_BN;
+    __shared__ int kinds[16];
+    const column_part& c = set.c[blockIdx.y];
+    const int N = c.N, K = c.K;
+    const int chunks = (K + 63) / 64, runs = chunks * 4;
+    const int rows = (N + RES_BN - 1) / RES_BN * RES_BN;
     const int n0 = (int) (blockIdx.x / k_blocks) * 16, k0 = (int) (blockIdx.x % k_blocks) * SPLIT_K;
-    if (n0 >= rows || k0 >= c.K) return;                       // whole block
+    if (n0 >= rows || k0 >= K) return;                         // whole block
     for (int i = threadIdx.x; i < 16 * SPLIT_K; i += 256) {
         const int r = i / SPLIT_K, k = i - r * SPLIT_K;
-        sx[r][k + (k >> 4)] = n0 + r < c.N && k0 + k < c.K ? c.X[(size_t) (n0 + r) * c.K + k0 + k] : 0.0;
+        sx[r][k + (k >> 4)] = n0 + r < N && k0 + k < K ? c.X[(size_t) (n0 + r) * K + k0 + k] : 0.0;
     }
+    if (threadIdx.x < 16) kinds[threadIdx.x] = n0 + (int) threadIdx.x < N ? c.to.kind[n0 + threadIdx.x] : -1;
     __syncthreads();
+    if (blockIdx.z == 0 && k0 == 0 && threadIdx.x == 0) {
+        int live = 0;
+        for (int r = 0; r < 16; ++r) live |= (kinds[r] == COLUMN_NARROW || kinds[r] == COLUMN_WIDE) | (kinds[r] == COLUMN_WIDE) << 1;
+        c.to.live[n0 / 16] = live;
+    }
+    if (blockIdx.z == 2)
+        for (int r = 0; r < 16; ++r) {
+            const int k = threadIdx.x;
+            if (kinds[r] > COLUMN_NARROW && k0 + k < (int) c.to.ld)
+                c.to.rows[(size_t) (n0 + r) * c.to.ld + k0 + k] = sx[r][k + (k >> 4)];
+        }
     const int r = threadIdx.x & 15, run = threadIdx.x >> 4;
     if (k0 / 16 + run >= runs) return;
-    const int s = n0 + r < c.N ? column_scales(c, chunks)[n0 + r] : BAD_COLUMN;
-    double h[16], d[16];
+    const bool has = kinds[r] == COLUMN_NARROW || kinds[r] == COLUMN_WIDE;
+    const int s = has ? c.to.scale[n0 + r] : 0;
+    double x[16], h[16], d[16];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) split_element(s != BAD_COLUMN ? sx[r][run * 17 + j] : 0.0, s, h[j], d[j]);
-    unsigned char* at = c.planes + run_offset(n0 + r, k0 / 16 + run, chunks);
+    for (int j = 0; j < 16; ++j) {
+        x[j] = has ? sx[r][run * 17 + j] : 0.0;
+        split_element(x[j], s, h[j], d[j]);
+    }
+    unsigned char* at = c.to.planes + run_offset(n0 + r, k0 / 16 + run, chunks);
     const size_t plane = (size_t) rows * chunks * 64;
-    if (blockIdx.z == 0) store_residues<0, 5>(h, d, at, plane);
-    else if (blockIdx.z == 1) store_residues<5, 10>(h, d, at, plane);
-    else store_residues<10, 15>(h, d, at, plane);
+    if (blockIdx.z == 0) {
+        store_residues<0, 5>(h, d, at, plane);
+    } else if (blockIdx.z == 1) {
+        store_residues<5, 10>(h, d, at, plane);
+    } else {
+        store_residues<10, 15>(h, d, at, plane);
+        store_magnitudes(x, SCALE_X - s, at + RES_MODULI * plane);
+    }
 }
 
 // ----------------------------------------------------------------------
@@ -279,11 +395,19 @@ static_assert(EF * 16 == RES_BM && XF * 16 == RES_BN && LOADS * WAVES == EF + XF
 struct unit_group {
     const unsigned char* E;
     const unsigned char* X;
+    const double* E64;           // FP64 rows of the operator and of the wide columns,
+    const double* X64;           // 64 * chunks apart
+    const int* e_scale;          // per row of the operator
+    const int* least;            // per row, see operator_scale_kernel
+    const int* x_scale;          // per column
+    const int* kind;             // per column
+    const int* live;             // per 16 columns
+    int* flags;                  // per column: set where an output could exceed the chain's bound
     size_t e_plane, x_plane;     // bytes of one modulus' plane
+    int M, N, K;
     int chunks, tiles_n;
     int tile0, tiles;            // tiles [tile0, tile0 + tiles) of the product, here tiles first_tile..
     int first_tile;
-    int pad;
 };
 struct unit_groups {
     unit_group g[RBF_MAX_GROUPS];
@@ -303,23 +427,40 @@ __global__ __launch_bounds__(RES_THREADS, 4) void residue_gemm_kernel(unit_group
     __shared__ __attribute__((aligned(16))) unsigned char s2[EF + XF][1024];
     // Blocks reach the XCDs round-robin: XCD x takes the x-th eighth of every
     // group's units, in order (modulus, row tile, column tile), so that the
-    // blocks sharing an operator row tile and a modulus' columns share an L2.
+    // blocks sharing an operator row tile and a modulus' columns share an L2;
+    // then its eighth of the magnitude products, most of which have nothing
+    // to do.
     const int xcd = blockIdx.x & 7;
-    int k = blockIdx.x >> 3, gi = -1, u = 0;
+    int k = blockIdx.x >> 3, gi = -1, l = 0, local = 0;
     for (int q = 0; q < G.count; ++q) {
         const long n = (long) G.g[q].tiles * RES_MODULI;
         const int lo = (int) (xcd * n / 8), hi = (int) ((xcd + 1) * n / 8);
         if (k < hi - lo) {
             gi = q;
-            u = lo + k;
+            l = (lo + k) / G.g[q].tiles;
+            local = lo + k - l * G.g[q].tiles;
             break;
         }
         k -= hi - lo;
     }
+    if (gi < 0)
+        for (int q = 0; q < G.count; ++q) {
+            const int n = G.g[q].tiles, lo = xcd * n / 8, hi = (xcd + 1) * n / 8;
+            if (k < hi - lo) {
+                gi = q;
+                l = RES_MODULI;
+                local = lo + k;
+                break;
+            }
+            k -= hi - lo;
+        }
     if (gi < 0) return;                              // whole block exits together
     const unit_group g = G.g[gi];
-    const int l = u / g.tiles, local = u - l * g.tiles, t = g.tile0 + local;
-    const int tm = t / g.tiles_n, tn = t - tm * g.tiles_n;
+    const int t = g.tile0 + local, tm = t / g.tiles_n, tn = t - tm * g.tiles_n;
+    int live = 0;
+#pragma unroll
+    for (int i = 0; i < XF; ++i) live |= g.live[tn * XF + i];
+    if (!(live & (l == RES_MODULI ? 2 : 1))) return;           // whole block
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave % WM, wn = wave / WM;
     const size_t frag_row = (size_t) g.chunks * 1024;
@@ -376,8 +517,66 @@ __global__ __launch_bounds__(RES_THREADS, 4) void residue_gemm_kernel(unit_group
     }
     __builtin_amdgcn_s_waitcnt(7 << 4);                        // no load into LDS outlives the block
     // The first operand's rows are columns of Y: a lane holds rows
-    // 4 (lane / 16) + i of X's fragment at sample lane % 16; their four
-    // residues make one word.
+    // 4 (lane / 16) + i of X's fragment at sample lane % 16.
+    if (l == RES_MODULI) {
+        // Magnitudes: outputs of wide columns below their row's bound.  Mostly
+        // that is the seven bits' doing (a sample beside a data site whose
+        // value is below 2^-7 of the column's largest: some tens among the
+        // five million outputs of an operator on cells that lie across a
+        // coordinate plane), and the FP64 pass for a single column costs a
+        // fifth of the whole evaluation.  So a wavefront lists up to REFINED
+        // of its outputs and forms their sums together; of more, the columns
+        // are flagged at once.
+        constexpr int REFINED = 16;
+        __syncthreads();                                       // s0 is free
+        int* listed = (int*) s0[wave];
+        int count = 0;
+#pragma unroll
+        for (int a = 0; a < FM; ++a) {
+            const int m = tm * RES_BM + (wm * FM + a) * 16 + (lane & 15);
+            const int least = m < g.M ? g.least[m] : 0;
+#pragma unroll
+            for (int b = 0; b < FN; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int n = tn * RES_BN + (wn * FN + b) * 16 + 4 * (lane >> 4) + i;
+                    const bool below = acc[a][b][i] < least && n < g.N && g.kind[n] == COLUMN_WIDE;
+                    const unsigned long long mask = __ballot(below);
+                    const int at = count + __popcll(mask & ((1ull << lane) - 1));
+                    if (below && at < REFINED) listed[at] = m - tm * RES_BM | (n - tn * RES_BN) << 8;
+                    if (below && at >= REFINED) g.flags[n] = 1;
+                    count += __popcll(mask);
+                }
+        }
+        __syncthreads();
+        const int K = g.K;
+        const size_t ld = (size_t) g.chunks * 64;
+        for (int r = 0; r < min(count, REFINED); ++r) {
+            const int m = tm * RES_BM + (listed[r] & 255), n = tn * RES_BN + (listed[r] >> 8);
+            const double* e = g.E64 + ld * m;
+            const double* x = g.X64 + ld * n;
+            double se = 0, sx = 0, ex = 0;
+#pragma unroll 4
+            for (int k = lane; k < K; k += 64) {
+                const double ve = fabs(e[k]), vx = fabs(x[k]);
+                se += ve;
+                sx += vx;
+                ex = fma(ve, vx, ex);
+            }
+            for (int off = 32; off > 0; off >>= 1) {
+                se += __shfl_xor(se, off, 64);
+                sx += __shfl_xor(sx, off, 64);
+                ex += __shfl_xor(ex, off, 64);
+            }
+            // half a unit of X's integers times sum |E|, half a unit of E's
+            // times sum |X| (the units are 2^-scale), against the chain's
+            // bound; 2^-30 for the sums' own rounding
+            if (ldexp(se, -1 - g.x_scale[n]) + ldexp(sx, -1 - g.e_scale[m]) > (1 - 0x1p-30) * 0x1p-53 * K * ex && lane == 0)
+                g.flags[n] = 1;
+        }
+        return;
+    }
+    // residues: those of the four rows make one word
     const double p = P[l], inv = 1.0 / p;
     const size_t tile = (size_t) (g.first_tile + local);
 #pragma unroll
@@ -394,14 +593,51 @@ __global__ __launch_bounds__(RES_THREADS, 4) void residue_gemm_kernel(unit_group
         }
 }
 
+// Clears the flags of every product's columns.
+__global__ __launch_bounds__(256) void clear_flags_kernel(int* __restrict__ flags, int n)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) flags[i] = 0;
+}
+
+struct list_group {
+    const int* kind;
+    const int* flags;
+    int* list;
+    int N, pad;
+};
+struct list_groups {
+    list_group g[RBF_MAX_GROUPS];
+};
+
+// Each product's columns that need FP64 products, in order (one block per product).
+__global__ __launch_bounds__(256) void list_kernel(list_groups G)
+{
+    __shared__ int wave_count[4];
+    const list_group g = G.g[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int found = 0;
+    for (int n0 = 0; n0 < g.N; n0 += 256) {
+        const int n = n0 + (int) threadIdx.x;
+        const bool on = n < g.N && (g.kind[n] == COLUMN_F64 || (g.kind[n] == COLUMN_WIDE && g.flags[n]));
+        const unsigned long long mask = __ballot(on);
+        if (lane == 0) wave_count[wave] = __popcll(mask);
+        __syncthreads();
+        int at = found;
+        for (int w = 0; w < wave; ++w) at += wave_count[w];
+        if (on) g.list[1 + at + __popcll(mask & ((1ull << lane) - 1))] = n;
+        found += wave_count[0] + wave_count[1] + wave_count[2] + wave_count[3];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) g.list[0] = found;
+}
+
 struct crt_group {
     const int* e_scale;
     const int* x_scale;
-    const double* E64;
-    const double* X64;
+    const int* live;             // per 16 columns
     double* Y;
-    long ld64;
-    int M, N, K, tiles_n, tile0, first_tile;
+    int M, N, tiles_n, tile0, first_tile, pad;
 };
 struct crt_groups {
     crt_group g[RBF_MAX_GROUPS];
@@ -412,7 +648,8 @@ struct crt_groups {
 // A thread takes four outputs (columns 4 (lane / 16) + 0..3 at one sample);
 // block (tile, column fragment b of wave row wn): its four waves x FM row
 // fragments cover the tile's 256 samples, so that every column is stored in
-// one run of 2 KB.
+// one run of 2 KB.  What it leaves in a column without residues is overwritten
+// by the FP64 product.
 __global__ __launch_bounds__(256) void crt_kernel(crt_groups G, const unsigned* __restrict__ res)
 {
     constexpr crt_table T = make_crt();
@@ -424,15 +661,10 @@ __global__ __launch_bounds__(256) void crt_kernel(crt_groups G, const unsigned* 
     const int lane = threadIdx.x & 63, wm = threadIdx.x >> 6;
     const int wn = xf / FN, b = xf - wn * FN, wave = wn * WM + wm;
     const int n0 = tn * RES_BN + xf * 16 + 4 * (lane >> 4);
-    if (tn * RES_BN + xf * 16 >= g.N) return;
+    if (tn * RES_BN + xf * 16 >= g.N || !(g.live[tn * XF + xf] & 1)) return;
     int xs[4];
-    bool bad[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        xs[i] = n0 + i < g.N ? g.x_scale[n0 + i] : 0;
-        bad[i] = xs[i] == BAD_COLUMN;
-        xs[i] = bad[i] ? 0 : xs[i];
-    }
+    for (int i = 0; i < 4; ++i) xs[i] = n0 + i < g.N ? g.x_scale[n0 + i] : 0;
 #pragma unroll
     for (int a = 0; a < FM; ++a) {
         const int m = tm * RES_BM + (wm * FM + a) * 16 + (lane & 15);
@@ -453,14 +685,7 @@ __global__ __launch_bounds__(256) void crt_kernel(crt_groups G, const unsigned* 
                 lo = fma(T.lo[l], d, lo);
             }
             const double Q = nearest(h, T.p_inv);
-            double y = ldexp(fma(-Q, T.p_hi, h) + fma(-Q, T.p_lo, lo), -(es + xs[i]));
-            if (bad[i]) {
-                // a NaN or an infinity in the column: the plain product
-                const double* e = g.E64 + g.ld64 * m;
-                const double* x = g.X64 + (size_t) (n0 + i) * g.K;
-                y = 0.0;
-                for (int k = 0; k < g.K; ++k) y = fma(e[k], x[k], y);
-            }
+            const double y = ldexp(fma(-Q, T.p_hi, h) + fma(-Q, T.p_lo, lo), -(es + xs[i]));
             g.Y[m + (size_t) g.M * (n0 + i)] = y;
         }
     }
@@ -476,10 +701,11 @@ void res_pack_operator(hipStream_t s, const double* E, long lde, int M, int K, u
 {
     const size_t plane = res_plane_bytes(M, RES_BM, K);
     const int rows = res_ceil(M, RES_BM) * RES_BM, chunks = res_chunks(K);
-    int* scale = (int*) (planes + RES_MODULI * plane);
-    operator_scale_kernel<<<res_ceil(M, 4), 256, 0, s>>>(E, lde, M, K, scale, flag);
+    int* scale = (int*) (planes + RES_PLANES * plane);
+    operator_scale_kernel<<<res_ceil(M, 4), 256, 0, s>>>(E, lde, M, K, scale, scale + M, scale + 2 * (size_t) M, flag);
     const long runs = (long) rows * chunks * 4;
-    operator_split_kernel<<<(unsigned) ((runs + 255) / 256), 256, 0, s>>>(E, lde, M, K, rows, chunks, scale, planes, plane);
+    operator_split_kernel<<<(unsigned) ((runs + 255) / 256), 256, 0, s>>>(E, lde, M, K, rows, chunks, scale, scale + M,
+                                                                          planes, plane);
 }
 
 void res_pack_columns(hipStream_t s, int count, const res_columns* c)
@@ -487,7 +713,7 @@ void res_pack_columns(hipStream_t s, int count, const res_columns* c)
     column_set set{};
     int n = 0, k = 0;
     for (int i = 0; i < count; ++i) {
-        set.c[i] = c[i];
+        set.c[i] = column_part{c[i].X, res_columns_at(c[i].packed, c[i].N, c[i].K), c[i].N, c[i].K};
         n = std::max(n, c[i].N);
         k = std::max(k, c[i].K);
     }
@@ -496,15 +722,36 @@ void res_pack_columns(hipStream_t s, int count, const res_columns* c)
     column_split_kernel<<<dim3((unsigned) (rows / 16 * k_blocks), (unsigned) count, SPLIT_PARTS), 256, 0, s>>>(set, k_blocks);
 }
 
-size_t res_work_bytes(int count, const res_product* p)
+static size_t tile_bytes(int count, const res_product* p)
 {
     long tiles = 0;
     for (int i = 0; i < count; ++i) tiles += tiles_of(p[i]);
     return (size_t) std::min<long>(tiles, RES_LAUNCH_TILES) * RES_TILE_BYTES;
 }
 
-ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, const res_product* p, unsigned char* work)
+size_t res_work_bytes(int count, const res_product* p)
 {
+    size_t columns = 0;
+    for (int i = 0; i < count; ++i) columns += (size_t) p[i].N;
+    return tile_bytes(count, p) + sizeof(int) * (2 * columns + (size_t) count);
+}
+
+ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, res_product* p, unsigned char* work)
+{
+    int columns = 0;
+    for (int i = 0; i < count; ++i) columns += p[i].N;
+    int* const flags = (int*) (work + tile_bytes(count, p));
+    int* flags_of[RBF_MAX_GROUPS];
+    list_groups L{};
+    for (int i = 0, at = 0; i < count; at += p[i++].N) {
+        const res_packed x = res_columns_at(p[i].X, p[i].N, p[i].K);
+        flags_of[i] = flags + at;
+        int* list = flags + columns + at + i;
+        p[i].list = list;
+        L.g[i] = list_group{x.kind, flags_of[i], list, p[i].N, 0};
+    }
+    clear_flags_kernel<<<(unsigned) res_ceil(columns, 256), 256, 0, s>>>(flags, columns);
+    IBM_LAUNCH_CHECK(ctx);
     // Launches of equal parts, at most RES_LAUNCH_TILES tiles (the residues of
     // a launch are recombined before the next overwrites them), longest
     // contraction first: the short units come last and fill the tail.
@@ -526,17 +773,20 @@ ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, const res_produc
         for (const span& sp : spans) {
             const res_product& r = p[sp.product];
             const size_t ep = res_plane_bytes(r.M, RES_BM, r.K), xp = res_plane_bytes(r.N, RES_BN, r.K);
+            const int* e_scale = (const int*) (r.E + RES_PLANES * ep);
+            const res_packed x = res_columns_at(r.X, r.N, r.K);
             const int tn = res_ceil(r.N, RES_BN);
-            U.g[U.count++] = unit_group{r.E, r.X, ep, xp, res_chunks(r.K), tn, sp.tile0, sp.tiles, first, 0};
-            C.g[C.count++] = crt_group{(const int*) (r.E + RES_MODULI * ep), (const int*) (r.X + RES_MODULI * xp), r.E64,
-                                       r.X64, r.Y, r.ld64, r.M, r.N, r.K, tn, sp.tile0, first};
+            U.g[U.count++] = unit_group{r.E, r.X, r.E64, x.rows, e_scale, e_scale + 2 * (size_t) r.M, x.scale, x.kind,
+                                        x.live, flags_of[sp.product], ep, xp, r.M, r.N, r.K, res_chunks(r.K), tn,
+                                        sp.tile0, sp.tiles, first};
+            C.g[C.count++] = crt_group{e_scale, x.scale, x.live, r.Y, r.M, r.N, tn, sp.tile0, first, 0};
             first += sp.tiles;
         }
         for (int x = 0; x < 8; ++x) {
             long n = 0;
             for (int q = 0; q < U.count; ++q) {
-                const long units = (long) U.g[q].tiles * RES_MODULI;
-                n += (x + 1) * units / 8 - x * units / 8;
+                const long tiles = U.g[q].tiles, units = tiles * RES_MODULI;
+                n += (x + 1) * units / 8 - x * units / 8 + (x + 1) * tiles / 8 - x * tiles / 8;
             }
             per_xcd = std::max(per_xcd, n);
         }
@@ -558,7 +808,10 @@ ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, const res_produc
             if (taken == most || (int) spans.size() == RBF_MAX_GROUPS) IBM_TRY(flush());
         }
     }
-    return flush();
+    IBM_TRY(flush());
+    list_kernel<<<(unsigned) count, 256, 0, s>>>(L);
+    IBM_LAUNCH_CHECK(ctx);
+    return IBM_OK;
 }
 
 } // namespace ibm

@@ -1,7 +1,8 @@
 // FP64 products of an RBF evaluation on the INT8 matrix cores
 // (rbf_residue.hip): Y = E^T X through residues modulo fifteen coprime
-// moduli.  rbf.hip decides which batch entries take this path and owns the
-// buffers.
+// moduli, and the columns that need FP64 products instead.  rbf.hip decides
+// which batch entries take this path, owns the buffers and multiplies those
+// columns.
 #pragma once
 #include "context.hpp"
 
@@ -24,13 +25,43 @@ inline size_t res_plane_bytes(int rows, int block, int K)
 {
     return (size_t) res_ceil(rows, block) * block * (size_t) res_chunks(K) * 64;
 }
-// Residue planes of an M x K operator / of N columns, and one int of scale
-// per row / column behind them.
-inline size_t res_operator_bytes(int M, int K) { return RES_MODULI * res_plane_bytes(M, RES_BM, K) + sizeof(int) * (size_t) M; }
-inline size_t res_columns_bytes(int N, int K)
+// One plane per modulus and one of seven-bit magnitudes.
+constexpr int RES_PLANES = RES_MODULI + 1;
+inline size_t res_align(size_t b) { return (b + 255) & ~size_t(255); }
+
+// An M x K operator: its planes, and per row the scale of its integers, the
+// exponent of its largest element and the least magnitude product that the
+// integers are good for (see operator_scale_kernel).
+inline size_t res_operator_bytes(int M, int K) { return RES_PLANES * res_plane_bytes(M, RES_BM, K) + 3 * sizeof(int) * (size_t) M; }
+
+// Classes of a column.
+enum { COLUMN_NARROW = 0, COLUMN_WIDE = 1, COLUMN_F64 = 2 };
+
+// N packed columns of K elements: the planes; per column its integers' scale
+// and its class; per 16 columns bit 0 if one has residues, bit 1 if one is
+// wide; and the columns themselves, rows of `ld` doubles, zero past K (written
+// where the class is not COLUMN_NARROW).
+struct res_packed {
+    unsigned char* planes;
+    int *scale, *kind, *live;
+    double* rows;
+    size_t ld, bytes;
+};
+inline res_packed res_columns_at(unsigned char* base, int N, int K)
 {
-    return RES_MODULI * res_plane_bytes(N, RES_BN, K) + (sizeof(int) * (size_t) N + 255) / 256 * 256;
+    res_packed p;
+    const size_t n = (size_t) N, planes = RES_PLANES * res_plane_bytes(N, RES_BN, K), ints = res_align(sizeof(int) * n);
+    p.planes = base;
+    p.scale = (int*) (base + planes);
+    p.kind = (int*) (base + planes + ints);
+    p.live = (int*) (base + planes + 2 * ints);
+    const size_t head = planes + 2 * ints + res_align(sizeof(int) * (size_t) (res_ceil(N, RES_BN) * (RES_BN / 16)));
+    p.rows = (double*) (base + head);
+    p.ld = (size_t) res_chunks(K) * 64;
+    p.bytes = head + sizeof(double) * n * p.ld;
+    return p;
 }
+inline size_t res_columns_bytes(int N, int K) { return res_columns_at(nullptr, N, K).bytes; }
 
 // Rows [0, M) of E (element k of row m at E[k + lde m]) into `planes`;
 // *flag (device, cleared by the caller) is set when a row cannot be
@@ -39,7 +70,7 @@ void res_pack_operator(hipStream_t s, const double* E, long lde, int M, int K, u
 
 struct res_columns {
     const double* X;           // N columns of K elements
-    unsigned char* planes;     // res_columns_bytes
+    unsigned char* packed;     // res_columns_bytes
     int N, K;
 };
 constexpr int RES_MAX_COLUMNS = 2 * IBM_MAX_CELL_TYPES;
@@ -47,15 +78,15 @@ void res_pack_columns(hipStream_t s, int count, const res_columns* c);
 
 struct res_product {
     const unsigned char* E;    // operator planes
-    const unsigned char* X;    // column planes
-    const double* E64;         // FP64 rows of the operator (stride ld64) and
-    const double* X64;         // the columns: for columns that hold a NaN or an infinity
+    const double* E64;         // its FP64 rows, zero past K, 64 res_chunks(K) apart
+    unsigned char* X;          // packed columns
     double* Y;                 // M x N, column-major
     int M, N, K;
-    long ld64;
+    const int* list;           // out: [0] the number of columns that need FP64 products, then their indices
 };
-// Every product; `work` holds res_work_bytes of their tiles.
+// Every product, but for the columns in its list; `work` holds
+// res_work_bytes: the tiles' residues, the lists and their flags.
 size_t res_work_bytes(int count, const res_product* p);
-ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, const res_product* p, unsigned char* work);
+ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, res_product* p, unsigned char* work);
 
 } // namespace ibm

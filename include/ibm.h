@@ -372,7 +372,7 @@ typedef struct ibm_rbf ibm_rbf;
 
 /* Arithmetic of an RBF evaluation. */
 enum {
-    IBM_RBF_F64 = 64,      /* FP64 matrix cores */
+    IBM_RBF_F64 = 64,      /* FP64 accuracy (see ibm_rbf_eval) */
     IBM_RBF_F32 = 32,      /* FP32 operands and accumulation */
     IBM_RBF_BF16X3 = 16    /* split BF16 (hi*hi + hi*lo + lo*hi), FP32 accumulation */
 };
@@ -382,7 +382,11 @@ enum {
  * rows are used: the slice E[0:K, 0:M] that bases::operators holds as its
  * evaluator / derivative matrices, K = data sites, M = sample sites
  * (bases/operators.h:145-177; the LU solve that produces E is setup).
- * The operator keeps its own packed copy; E may be freed afterwards. */
+ * The operator keeps its own packed copy; E may be freed afterwards.  In
+ * FP64 that is 24 bytes per element (with K padded to a multiple of 64 and M
+ * to one of 128 or 256): the element, and 16 bytes that evaluations of many
+ * columns use.  Where the device has no memory for the latter, or an element
+ * is not finite, the operator goes without, and those run slower. */
 ibm_status ibm_rbf_create(ibm_ctx* ctx, int precision, int M, int K, int nops, const double* const* E, int lde,
                           ibm_rbf** out);
 ibm_status ibm_rbf_destroy(ibm_rbf* op);
@@ -392,7 +396,18 @@ ibm_status ibm_rbf_destroy(ibm_rbf* op);
  * K x N[b] column-major (ld = K; column comp * ncells + cell, as
  * bases/container.h:54 lays out data-site coordinates); Y[b] receives
  * nops consecutive M x N[b] column-major blocks.  All entries share one
- * precision. */
+ * precision.
+ *
+ * FP64: every output is within (K + 1) 2^-53 sum_k |E_k||X_k| of the exact
+ * product (short of overflow and underflow), the bound of a chain of K fused
+ * multiply-adds.  Entries of up to 64 columns, and of more while K <= 550 and
+ * M K N < 9e7, run on the FP64 matrix cores; others through residues on the
+ * INT8 matrix cores, but for the columns that those would not hold to that
+ * bound (values of very different magnitude that matter to some output, NaN,
+ * infinities), which run on the FP64 ones.  So the bits of an output depend on
+ * N (two entries of 64 columns need not agree in the last bits with one of
+ * 128), but not on the other columns' values or on the other entries of the
+ * batch. */
 ibm_status ibm_rbf_eval(ibm_ctx* ctx, int count, ibm_rbf* const* ops, const int* N, const double* const* X,
                         double* const* Y);
 
@@ -402,9 +417,10 @@ ibm_status ibm_rbf_eval(ibm_ctx* ctx, int count, ibm_rbf* const* ops, const int*
  * 64 x 32-output waves (half the registers, twice the waves per SIMD) over
  * two LDS buffers (one barrier per contraction chunk), 0 (the default) times
  * both on the first eager launch of each shape and keeps the faster for the
- * process.  Evaluations of 65 columns or more run on the INT8 matrix cores
- * instead (as accurate as the FP64 ones: see rbf_residue.hip), whatever the
- * variant.  Every setting gives bitwise the same results.  Process-wide. */
+ * process.  Only products of more than 64 columns (or, with K <= 550, of
+ * M K N >= 9e7) by operators without residue storage (see ibm_rbf_create)
+ * take these kernels.  Every setting gives bitwise the same results.
+ * Process-wide. */
 ibm_status ibm_rbf_gemm_variant(int waves_n);
 
 /* Operator construction on the device (bases/operators.h:145-190,
