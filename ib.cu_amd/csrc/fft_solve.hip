@@ -712,10 +712,12 @@ static plane_kernels plane_kernels_of(int lx, int lz)
 
 static ibm_status fft_lds_attributes(ibm_ctx* ctx)
 {
+    // an attribute of a kernel on one device
     static std::mutex lock;
-    static bool done = false;
+    static std::vector<bool> done;
     std::lock_guard<std::mutex> guard(lock);
-    if (done) return IBM_OK;
+    if ((int) done.size() <= ctx->device) done.resize(ctx->device + 1);
+    if (done[ctx->device]) return IBM_OK;
     IBM_HIP(ctx, hipFuncSetAttribute((const void*) zfft_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int) MAX_DYNAMIC_LDS));
     for (int lx = PLANE_MIN; lx < PLANE_MIN + PLANE_SIZES; ++lx)
@@ -724,7 +726,7 @@ static ibm_status fft_lds_attributes(ibm_ctx* ctx)
             IBM_HIP(ctx, hipFuncSetAttribute((const void*) k.forward, hipFuncAttributeMaxDynamicSharedMemorySize, (int) k.lds));
             IBM_HIP(ctx, hipFuncSetAttribute((const void*) k.inverse, hipFuncAttributeMaxDynamicSharedMemorySize, (int) k.lds));
         }
-    done = true;
+    done[ctx->device] = true;
     return IBM_OK;
 }
 
