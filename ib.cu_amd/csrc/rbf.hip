@@ -31,6 +31,7 @@
 #include <cstring>
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -71,7 +72,7 @@ struct gemm_groups {
     int count, total_tiles;
 };
 
-// Listed columns up to this many run in rbf_thin_kernel.
+// Listed columns up to this many run in listed_thin_kernel.
 constexpr int LISTED_THIN = 64;
 
 __device__ inline uint16_t bf16_bits(float f)
@@ -158,11 +159,9 @@ __device__ inline void mfma_step(const u4& xa, const u4& eb, const u4& xa_lo, co
 // r = 0..3, for the FP32-accumulating instructions, but rows (l / 16) + 4 r
 // for v_mfma_f64_16x16x4 (both measured on gfx950).
 //
-// LISTED: only the columns of the group's list, unless they are few enough
-// for rbf_thin_kernel; the grid is that of all columns, since the list is
-// known on the device alone.
-template <int MODE, int WN, int RB = ROWB, int NB = 1, int T = TILE, bool LISTED = false>
-__global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
+// LISTED: columns [0, N) of the group's list.
+template <int MODE, int WN, int RB, int NB, int T, bool LISTED>
+__device__ inline void gemm_tile(const gemm_group& g, int N, int tm, int tn)
 {
     constexpr int PL = planes(MODE);
     constexpr int THREADS = 128 * WN;                // waves: 2 along the samples x WN along the columns
@@ -172,27 +171,6 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
     using acc_t = typename std::conditional<MODE == MODE_F64, d4, f4>::type;
     __shared__ __attribute__((aligned(16))) unsigned char ldsb[NB][PL][2][T * RS];
 
-    // Blocks reach the XCDs round-robin (block i on XCD i % 8).  XCD x takes
-    // the x-th eighth of every group's tiles, in order, so that the XCDs get
-    // equal work however the groups' contraction lengths differ, and the
-    // tiles sharing an operator row block share an L2.
-    const int xcd = blockIdx.x & 7;
-    int k = blockIdx.x >> 3, gi = -1, t = 0;
-    for (int q = 0; q < G.count; ++q) {
-        const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : G.total_tiles) - G.g[q].first_tile;
-        const int lo = xcd * tq / 8, hi = (xcd + 1) * tq / 8;
-        if (k < hi - lo) {
-            gi = q;
-            t = lo + k;
-            break;
-        }
-        k -= hi - lo;
-    }
-    if (gi < 0) return;                              // whole block exits together
-    const gemm_group g = G.g[gi];
-    int tm = t / g.tiles_n, tn = t - tm * g.tiles_n;
-    const int N = LISTED ? g.list[0] : g.N;
-    if (LISTED && (N <= LISTED_THIN || tn * T >= N)) return;     // whole block
     const long row_bytes = (long) g.Kp * elem_bytes(MODE);
     const int nchunks = (int) (row_bytes / RB);
 
@@ -310,6 +288,82 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
         }
 }
 
+template <int MODE, int WN, int RB = ROWB, int NB = 1, int T = TILE>
+__global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
+{
+    // Blocks reach the XCDs round-robin (block i on XCD i % 8).  XCD x takes
+    // the x-th eighth of every group's tiles, in order, so that the XCDs get
+    // equal work however the groups' contraction lengths differ, and the
+    // tiles sharing an operator row block share an L2.
+    const int xcd = blockIdx.x & 7;
+    int k = blockIdx.x >> 3, gi = -1, t = 0;
+    for (int q = 0; q < G.count; ++q) {
+        const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : G.total_tiles) - G.g[q].first_tile;
+        const int lo = xcd * tq / 8, hi = (xcd + 1) * tq / 8;
+        if (k < hi - lo) {
+            gi = q;
+            t = lo + k;
+            break;
+        }
+        k -= hi - lo;
+    }
+    if (gi < 0) return;                              // whole block exits together
+    const gemm_group g = G.g[gi];
+    const int tm = t / g.tiles_n, tn = t - tm * g.tiles_n;
+    gemm_tile<MODE, WN, RB, NB, T, false>(g, g.N, tm, tn);
+}
+
+// The next of a block's tiles of the listed columns, turn by turn: XCD x takes
+// the x-th eighth of every group's tiles.  The lists' lengths are known on
+// the device alone, so the blocks of a launch of one size share out the tiles
+// that there are (a block for each tile that there could be, most often for
+// none: 39 us of the suspension step in a kernel trace; so 27, five to ten a
+// launch).  Lists of [least, most] columns count, in tiles of `rows` x `cols`.
+__device__ inline bool listed_tile(const gemm_groups& G, int turn, int rows, int cols, int least, int most, int& group,
+                                   int& tm, int& tn)
+{
+    const int xcd = blockIdx.x & 7;
+    int k = turn;
+    for (int q = 0; q < G.count; ++q) {
+        const int N = G.g[q].list[0];
+        if (N < least || N > most) continue;
+        const int tiles_n = (N + cols - 1) / cols, tq = (G.g[q].M + rows - 1) / rows * tiles_n;
+        const int lo = (int) ((long) xcd * tq / 8), hi = (int) ((long) (xcd + 1) * tq / 8);
+        if (k < hi - lo) {
+            group = q;
+            tm = (lo + k) / tiles_n;
+            tn = lo + k - tm * tiles_n;
+            return true;
+        }
+        k -= hi - lo;
+    }
+    return false;
+}
+
+// Whether any list has [least, most] columns: a lane for each (the walk above
+// is a chain of loads).
+__device__ inline bool any_listed(const gemm_groups& G, int least, int most)
+{
+    static_assert(MAX_GROUPS <= 64);
+    const int lane = threadIdx.x & 63, N = lane < G.count ? G.g[lane].list[0] : 0;
+    return __ballot(N >= least && N <= most) != 0;
+}
+
+constexpr int LISTED_WAVES_N = 4, LISTED_BLOCKS = 512;       // two blocks per CU
+
+// FP64 tiles of the lists that are too long for listed_thin_kernel.
+__global__ __launch_bounds__(128 * LISTED_WAVES_N, 4) void listed_gemm_kernel(gemm_groups G)
+{
+    if (!any_listed(G, LISTED_THIN + 1, INT_MAX)) return;        // whole block
+    int q, tm, tn;
+    for (int turn = blockIdx.x >> 3; listed_tile(G, turn, TILE, TILE, LISTED_THIN + 1, INT_MAX, q, tm, tn);
+         turn += gridDim.x >> 3) {
+        const gemm_group g = G.g[q];
+        gemm_tile<MODE_F64, LISTED_WAVES_N, ROWB, 2, TILE, true>(g, g.list[0], tm, tn);
+        __syncthreads();
+    }
+}
+
 // FP64 products of few columns, in column tiles of at most 64: bound by
 // reading the operator (once; its matrix-core time is 0.3 NB of that).  A
 // wave owns 16 samples and the tile's columns, so that operator rows go
@@ -322,18 +376,12 @@ __global__ __launch_bounds__(128 * WN, 2) void rbf_gemm_kernel(gemm_groups G)
 // copy rate); 715 x 503, 24 columns 70 -> 15.
 constexpr int THIN_ROWS = 32, THIN_RB = 256, THIN_RS = THIN_RB + 16, THIN_AHEAD = 3, THIN_THREADS = 128;
 
-// LISTED: as in rbf_gemm_kernel, up to LISTED_THIN columns.
-template <int NB, bool LISTED = false>
-__global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
+// LISTED: columns [0, N) of the group's list.
+template <int NB, bool LISTED>
+__device__ inline void thin_tile(const gemm_group& g, int N, int row_tile, int col0)
 {
     constexpr int XLOADS = NB * 16 * THIN_RB / 16 / THIN_THREADS;    // 16-byte staging loads per thread
     __shared__ __attribute__((aligned(16))) unsigned char lds[2][NB * 16 * THIN_RS];
-    int gi = 0;
-    while (gi + 1 < G.count && (int) blockIdx.x >= G.g[gi + 1].first_tile) ++gi;
-    const gemm_group g = G.g[gi];
-    const int tile = (int) blockIdx.x - g.first_tile, row_tile = tile / g.tiles_n, col0 = (tile - row_tile * g.tiles_n) * (16 * NB);
-    const int N = LISTED ? g.list[0] : g.N;
-    if (LISTED && (N > LISTED_THIN || col0 >= N)) return;        // whole block
     const int row0 = row_tile * THIN_ROWS + (threadIdx.x >> 6) * 16;
     const long row_bytes = (long) g.Kp * 8;
     const int nchunks = (int) (row_bytes / THIN_RB);
@@ -405,6 +453,30 @@ __global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
             const int n = col0 + b * 16 + fgrp + 4 * r;
             if (n < N) g.Y[m + (long) g.M * (LISTED ? g.list[1 + n] : n)] = acc[b][r];
         }
+}
+
+template <int NB>
+__global__ __launch_bounds__(THIN_THREADS) void rbf_thin_kernel(gemm_groups G)
+{
+    int gi = 0;
+    while (gi + 1 < G.count && (int) blockIdx.x >= G.g[gi + 1].first_tile) ++gi;
+    const gemm_group g = G.g[gi];
+    const int tile = (int) blockIdx.x - g.first_tile, row_tile = tile / g.tiles_n;
+    thin_tile<NB, false>(g, g.N, row_tile, (tile - row_tile * g.tiles_n) * (16 * NB));
+}
+
+// Lists of up to LISTED_THIN columns, in column tiles of 32.
+constexpr int LISTED_NB = 2, LISTED_THIN_BLOCKS = 1024;      // four blocks per CU
+__global__ __launch_bounds__(THIN_THREADS) void listed_thin_kernel(gemm_groups G)
+{
+    if (!any_listed(G, 1, LISTED_THIN)) return;                  // whole block
+    int q, tm, tn;
+    for (int turn = blockIdx.x >> 3; listed_tile(G, turn, THIN_ROWS, 16 * LISTED_NB, 1, LISTED_THIN, q, tm, tn);
+         turn += gridDim.x >> 3) {
+        const gemm_group g = G.g[q];
+        thin_tile<LISTED_NB, true>(g, g.list[0], tm, tn * 16 * LISTED_NB);
+        __syncthreads();
+    }
 }
 
 // Surface geometry of one cell per block from the evaluated position and
@@ -638,32 +710,14 @@ size_t packed_offset(int count, ibm_rbf* const* ops, const int* N, const double*
     return at;
 }
 
-// Blocks of a grid in which XCD x takes the x-th eighth of every group's
-// tiles: 8 times the most that any XCD takes.
-int xcd_blocks(const gemm_groups& G)
-{
-    int per_xcd = 0;
-    for (int x = 0; x < 8; ++x) {
-        int n = 0;
-        for (int q = 0; q < G.count; ++q) {
-            const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : G.total_tiles) - G.g[q].first_tile;
-            n += (x + 1) * tq / 8 - x * tq / 8;
-        }
-        per_xcd = std::max(per_xcd, n);
-    }
-    return 8 * per_xcd;
-}
-
-// FP64 products of the columns that the residue path has listed.  The lists
-// are on the device: the thin kernel's launch takes the short ones and the
-// tiles' the others, blocks without columns leave at once.
+// FP64 products of the columns that the residue path has listed.
 ibm_status listed_products(ibm_ctx* ctx, hipStream_t stream, int count, const res_product* p)
 {
-    constexpr int NB = 2;
-    gemm_groups thin{}, tiles{};
+    gemm_groups G{};
+    bool long_lists = false;
     for (int i = 0; i < count; ++i) {
         const res_packed x = res_columns_at(p[i].X, p[i].N, p[i].K);
-        gemm_group g{};
+        gemm_group& g = G.g[G.count++];
         g.E[0] = g.E[1] = (const unsigned char*) p[i].E64;
         g.X[0] = g.X[1] = (const unsigned char*) x.rows;
         g.Y = p[i].Y;
@@ -671,20 +725,11 @@ ibm_status listed_products(ibm_ctx* ctx, hipStream_t stream, int count, const re
         g.M = p[i].M;
         g.N = p[i].N;
         g.Kp = (int) x.ld;
-        g.tiles_n = (std::min(g.N, LISTED_THIN) + 16 * NB - 1) / (16 * NB);
-        g.first_tile = thin.total_tiles;
-        thin.g[thin.count++] = g;
-        thin.total_tiles += (g.M + THIN_ROWS - 1) / THIN_ROWS * g.tiles_n;
-        if (g.N <= LISTED_THIN) continue;
-        g.tiles_n = (g.N + TILE - 1) / TILE;
-        g.first_tile = tiles.total_tiles;
-        tiles.g[tiles.count++] = g;
-        tiles.total_tiles += (g.M + TILE - 1) / TILE * g.tiles_n;
+        long_lists = long_lists || p[i].N > LISTED_THIN;
     }
-    rbf_thin_kernel<NB, true><<<thin.total_tiles, THIN_THREADS, 0, stream>>>(thin);
+    listed_thin_kernel<<<LISTED_THIN_BLOCKS, THIN_THREADS, 0, stream>>>(G);
     IBM_LAUNCH_CHECK(ctx);
-    if (tiles.count)
-        rbf_gemm_kernel<MODE_F64, DEFAULT_WAVES_N, ROWB, 2, TILE, true><<<xcd_blocks(tiles), 512, 0, stream>>>(tiles);
+    if (long_lists) listed_gemm_kernel<<<LISTED_BLOCKS, 128 * LISTED_WAVES_N, 0, stream>>>(G);
     IBM_LAUNCH_CHECK(ctx);
     return IBM_OK;
 }
@@ -800,7 +845,17 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
             tiles += (G.g[q].M + edge - 1) / edge * G.g[q].tiles_n;
         }
         G.total_tiles = tiles;
-        blocks = xcd_blocks(G);
+        // blocks: 8 x the most tiles any XCD takes (its share of every group)
+        int per_xcd = 0;
+        for (int x = 0; x < 8; ++x) {
+            int n = 0;
+            for (int q = 0; q < G.count; ++q) {
+                const int tq = (q + 1 < G.count ? G.g[q + 1].first_tile : tiles) - G.g[q].first_tile;
+                n += (x + 1) * tq / 8 - x * tq / 8;
+            }
+            per_xcd = std::max(per_xcd, n);
+        }
+        blocks = 8 * per_xcd;
     }
     const int wn = mode == MODE_F64 && tiles ? f64_variant(ctx, stream, G, blocks) : 2;
     prof_scope prof(ctx, "rbf_gemm", flops);
