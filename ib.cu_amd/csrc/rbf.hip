@@ -785,6 +785,15 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
         return fail(ctx, IBM_ERR_ARG, "no packed operand");
     }
 
+    res_product products[MAX_GROUPS];
+    const int nres = residue_products(count, ops, N, X, Y, j0, j1, *packed, products);
+    void* work = nullptr;
+    int* flags = nullptr;
+    int nflags = 0;
+    if (nres) {
+        IBM_TRY(scratch(ctx, SLOT_RBF_WORK, res_work_bytes(nres, products), &work));
+        flags = res_flags(nres, products, (unsigned char*) work, &nflags);
+    }
     gemm_groups G{}, thin[4]{};        // thin[k]: rbf_thin_kernel's entries with tiles of 16 (k + 1) columns
     int tiles = 0, ncols = 0;
     res_columns cols[RES_MAX_COLUMNS];
@@ -797,7 +806,7 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
             if (do_pack && owner == b) {
                 cols[ncols++] = res_columns{X[b], hi, N[b], op.K};
                 if (ncols == RES_MAX_COLUMNS) {
-                    res_pack_columns(stream, ncols, cols);
+                    res_pack_columns(stream, ncols, cols, nullptr, 0);
                     ncols = 0;
                 }
             }
@@ -823,15 +832,11 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
             if (!is_thin) tiles += (op.rows_pad / TILE) * g.tiles_n;
         }
     }
-    if (ncols) res_pack_columns(stream, ncols, cols);
+    if (ncols) res_pack_columns(stream, ncols, cols, flags, nflags);
     IBM_LAUNCH_CHECK(ctx);
-    res_product products[MAX_GROUPS];
-    const int nres = residue_products(count, ops, N, X, Y, j0, j1, *packed, products);
     double flops = 0;
     for (int b = 0; b < count; ++b)
         flops += 2.0 * ops[b]->M * (double) N[b] * ops[b]->K * std::max(0, std::min(j1, ops[b]->nops) - j0);
-    void* work = nullptr;
-    if (nres) IBM_TRY(scratch(ctx, SLOT_RBF_WORK, res_work_bytes(nres, products), &work));
     int blocks = 0, edge = TILE;
     if (tiles) {
         // Longest contraction first: each XCD takes its share of the groups
@@ -860,7 +865,7 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
     const int wn = mode == MODE_F64 && tiles ? f64_variant(ctx, stream, G, blocks) : 2;
     prof_scope prof(ctx, "rbf_gemm", flops);
     if (nres) {
-        IBM_TRY(res_products(ctx, stream, nres, products, (unsigned char*) work));
+        IBM_TRY(res_products(ctx, stream, nres, products, (unsigned char*) work, ncols > 0));
         IBM_TRY(listed_products(ctx, stream, nres, products));
     }
     for (int k = 0; k < 4; ++k) {

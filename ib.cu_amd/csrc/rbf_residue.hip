@@ -78,8 +78,9 @@ constexpr u128 weight(int l)
 
 // High part: a multiple of 2^77, so that sums of 15 of them times residues
 // (below 15 * 2^117.8 * 2^7 < 2^129) and multiples of P's high part are
-// exact in FP64; the low parts are below 2^77 and enter with FP64 rounding,
-// 2^-60 of an integer of C's unit size or less.
+// exact in FP64; the low parts are below 2^77, their sums below 2^88, and
+// enter with FP64 rounding: 2^35 to 2^39 units of C, 2^-77 of its bound or
+// less.
 constexpr int HIGH = 77;
 constexpr double high_part(u128 v) { return (double) (unsigned long long) (v >> HIGH) * 0x1p77; }
 constexpr double low_part(u128 v)
@@ -263,8 +264,12 @@ struct column_set {
 // of which more than half lies below 2^-7 of the maximum have no seven-bit
 // magnitudes to speak of; those of a maximum below 2^-1000 are left to FP64 as
 // the sums here would underflow.
-__global__ __launch_bounds__(256) void column_scale_kernel(column_set set)
+// Also clears the flags of the products that follow.
+__global__ __launch_bounds__(256) void column_scale_kernel(column_set set, int* __restrict__ flags, int nflags)
 {
+    for (int i = (int) (blockIdx.y * gridDim.x + blockIdx.x) * 256 + (int) threadIdx.x; i < nflags;
+         i += (int) (gridDim.x * gridDim.y) * 256)
+        flags[i] = 0;
     __shared__ double part[3][4];
     __shared__ int small[4];
     const column_part& c = set.c[blockIdx.y];
@@ -524,39 +529,52 @@ __global__ __launch_bounds__(RES_THREADS, 4) void residue_gemm_kernel(unit_group
         // value is below 2^-7 of the column's largest: some tens among the
         // five million outputs of an operator on cells that lie across a
         // coordinate plane), and the FP64 pass for a single column costs a
-        // fifth of the whole evaluation.  So a wavefront lists up to REFINED
-        // of its outputs and forms their sums together; of more, the columns
-        // are flagged at once.
-        constexpr int REFINED = 16;
+        // fifth of the whole evaluation.  So a wavefront lists its outputs and
+        // forms their sums, all lanes together.  A column with more than
+        // REFINED of them among the wavefront's 64 rows is flagged at once
+        // (its own outputs decide, whatever its neighbours hold).
+        constexpr int REFINED = 4;
+        static_assert(REFINED * 16 * FN * sizeof(int) <= sizeof(s0[0]));
         __syncthreads();                                       // s0 is free
         int* listed = (int*) s0[wave];
         int count = 0;
 #pragma unroll
-        for (int a = 0; a < FM; ++a) {
-            const int m = tm * RES_BM + (wm * FM + a) * 16 + (lane & 15);
-            const int least = m < g.M ? g.least[m] : 0;
+        for (int b = 0; b < FN; ++b)
 #pragma unroll
-            for (int b = 0; b < FN; ++b)
+            for (int i = 0; i < 4; ++i) {
+                const int n = tn * RES_BN + (wn * FN + b) * 16 + 4 * (lane >> 4) + i;
+                const bool wide = n < g.N && g.kind[n] == COLUMN_WIDE;
+                unsigned long long below[FM];
+                int found = 0;                                 // of column n
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int n = tn * RES_BN + (wn * FN + b) * 16 + 4 * (lane >> 4) + i;
-                    const bool below = acc[a][b][i] < least && n < g.N && g.kind[n] == COLUMN_WIDE;
-                    const unsigned long long mask = __ballot(below);
-                    const int at = count + __popcll(mask & ((1ull << lane) - 1));
-                    if (below && at < REFINED) listed[at] = m - tm * RES_BM | (n - tn * RES_BN) << 8;
-                    if (below && at >= REFINED) g.flags[n] = 1;
+                for (int a = 0; a < FM; ++a) {
+                    const int m = tm * RES_BM + (wm * FM + a) * 16 + (lane & 15);
+                    below[a] = __ballot(wide && m < g.M && acc[a][b][i] < g.least[m]);
+                    found += __popcll(below[a] >> (lane & 48) & 0xffff);
+                }
+                const bool many = found > REFINED;
+                if (many && (lane & 15) == 0) g.flags[n] = 1;
+#pragma unroll
+                for (int a = 0; a < FM; ++a) {
+                    const bool own = !many && (below[a] >> lane & 1);
+                    const unsigned long long mask = __ballot(own);
+                    if (own)
+                        listed[count + __popcll(mask & ((1ull << lane) - 1))] =
+                            (wm * FM + a) * 16 + (lane & 15) | (n - tn * RES_BN) << 8;
                     count += __popcll(mask);
                 }
-        }
+            }
         __syncthreads();
         const int K = g.K;
         const size_t ld = (size_t) g.chunks * 64;
-        for (int r = 0; r < min(count, REFINED); ++r) {
-            const int m = tm * RES_BM + (listed[r] & 255), n = tn * RES_BN + (listed[r] >> 8);
+        for (int r = 0; r < count; ++r) {
+            const int entry = __builtin_amdgcn_readfirstlane(listed[r]);
+            const int m = tm * RES_BM + (entry & 255), n = tn * RES_BN + (entry >> 8);
+            if (__hip_atomic_load(&g.flags[n], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) continue;
             const double* e = g.E64 + ld * m;
             const double* x = g.X64 + ld * n;
             double se = 0, sx = 0, ex = 0;
-#pragma unroll 4
+#pragma unroll 8
             for (int k = lane; k < K; k += 64) {
                 const double ve = fabs(e[k]), vx = fabs(x[k]);
                 se += ve;
@@ -572,7 +590,7 @@ __global__ __launch_bounds__(RES_THREADS, 4) void residue_gemm_kernel(unit_group
             // times sum |X| (the units are 2^-scale), against the chain's
             // bound; 2^-30 for the sums' own rounding
             if (ldexp(se, -1 - g.x_scale[n]) + ldexp(sx, -1 - g.e_scale[m]) > (1 - 0x1p-30) * 0x1p-53 * K * ex && lane == 0)
-                g.flags[n] = 1;
+                __hip_atomic_store(&g.flags[n], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
     }
@@ -708,7 +726,21 @@ void res_pack_operator(hipStream_t s, const double* E, long lde, int M, int K, u
                                                                           planes, plane);
 }
 
-void res_pack_columns(hipStream_t s, int count, const res_columns* c)
+static size_t tile_bytes(int count, const res_product* p)
+{
+    long tiles = 0;
+    for (int i = 0; i < count; ++i) tiles += tiles_of(p[i]);
+    return (size_t) std::min<long>(tiles, RES_LAUNCH_TILES) * RES_TILE_BYTES;
+}
+
+int* res_flags(int count, const res_product* p, unsigned char* work, int* n)
+{
+    *n = 0;
+    for (int i = 0; i < count; ++i) *n += p[i].N;
+    return (int*) (work + tile_bytes(count, p));
+}
+
+void res_pack_columns(hipStream_t s, int count, const res_columns* c, int* flags, int nflags)
 {
     column_set set{};
     int n = 0, k = 0;
@@ -718,15 +750,8 @@ void res_pack_columns(hipStream_t s, int count, const res_columns* c)
         k = std::max(k, c[i].K);
     }
     const int k_blocks = res_ceil(k, SPLIT_K), rows = res_ceil(n, RES_BN) * RES_BN;
-    column_scale_kernel<<<dim3((unsigned) n, (unsigned) count), 256, 0, s>>>(set);
+    column_scale_kernel<<<dim3((unsigned) n, (unsigned) count), 256, 0, s>>>(set, flags, nflags);
     column_split_kernel<<<dim3((unsigned) (rows / 16 * k_blocks), (unsigned) count, SPLIT_PARTS), 256, 0, s>>>(set, k_blocks);
-}
-
-static size_t tile_bytes(int count, const res_product* p)
-{
-    long tiles = 0;
-    for (int i = 0; i < count; ++i) tiles += tiles_of(p[i]);
-    return (size_t) std::min<long>(tiles, RES_LAUNCH_TILES) * RES_TILE_BYTES;
 }
 
 size_t res_work_bytes(int count, const res_product* p)
@@ -736,11 +761,10 @@ size_t res_work_bytes(int count, const res_product* p)
     return tile_bytes(count, p) + sizeof(int) * (2 * columns + (size_t) count);
 }
 
-ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, res_product* p, unsigned char* work)
+ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, res_product* p, unsigned char* work, bool cleared)
 {
-    int columns = 0;
-    for (int i = 0; i < count; ++i) columns += p[i].N;
-    int* const flags = (int*) (work + tile_bytes(count, p));
+    int columns;
+    int* const flags = res_flags(count, p, work, &columns);
     int* flags_of[RBF_MAX_GROUPS];
     list_groups L{};
     for (int i = 0, at = 0; i < count; at += p[i++].N) {
@@ -750,8 +774,10 @@ ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, res_product* p, 
         p[i].list = list;
         L.g[i] = list_group{x.kind, flags_of[i], list, p[i].N, 0};
     }
-    clear_flags_kernel<<<(unsigned) res_ceil(columns, 256), 256, 0, s>>>(flags, columns);
-    IBM_LAUNCH_CHECK(ctx);
+    if (!cleared) {
+        clear_flags_kernel<<<(unsigned) res_ceil(columns, 256), 256, 0, s>>>(flags, columns);
+        IBM_LAUNCH_CHECK(ctx);
+    }
     // Launches of equal parts, at most RES_LAUNCH_TILES tiles (the residues of
     // a launch are recombined before the next overwrites them), longest
     // contraction first: the short units come last and fill the tail.

@@ -74,7 +74,8 @@ struct res_columns {
     int N, K;
 };
 constexpr int RES_MAX_COLUMNS = 2 * IBM_MAX_CELL_TYPES;
-void res_pack_columns(hipStream_t s, int count, const res_columns* c);
+// Also clears `flags` (those of res_flags, or none).
+void res_pack_columns(hipStream_t s, int count, const res_columns* c, int* flags, int nflags);
 
 struct res_product {
     const unsigned char* E;    // operator planes
@@ -85,8 +86,10 @@ struct res_product {
     const int* list;           // out: [0] the number of columns that need FP64 products, then their indices
 };
 // Every product, but for the columns in its list; `work` holds
-// res_work_bytes: the tiles' residues, the lists and their flags.
+// res_work_bytes: the tiles' residues, the lists and their flags (*n of them),
+// which are cleared first unless the packing has done so.
 size_t res_work_bytes(int count, const res_product* p);
-ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, res_product* p, unsigned char* work);
+int* res_flags(int count, const res_product* p, unsigned char* work, int* n);
+ibm_status res_products(ibm_ctx* ctx, hipStream_t s, int count, res_product* p, unsigned char* work, bool cleared);
 
 } // namespace ibm

@@ -106,6 +106,11 @@ def test_columns_of_mixed_magnitude(ibm, ctx, kind):
     Y = Y.cpu().numpy()
     for j, E in enumerate(mats):
         _check(E, x, Y[j])
+    # every column's value is its own affair: other neighbours, the same bits
+    some = x[::3]
+    mixed = np.concatenate([_narrow(rng, 30, K), some, _narrow(rng, 40, K)])
+    (Z,) = ibm.rbf_eval(ctx, [op], [_t(mixed)])
+    assert np.array_equal(Z.cpu().numpy()[:, 30:30 + len(some)], Y[:, ::3])
     op.close()
 
 
