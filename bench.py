@@ -252,7 +252,7 @@ PMC_KERNELS = {"chebyshev_f32": "cheb_march_kernel<float", "chebyshev_f64": "che
                "stencil_f32": "stencil_kernel<float", "stencil_f64": "stencil_kernel<double",
                "restrict": "::restrict_kernel<", "residual_restrict": "residual_restrict_kernel",
                "prolong": "::prolong_add_kernel", "prolong_residual": "prolong_residual_kernel",
-               "rbf_gemm": ("residue_gemm_kernel", "crt_kernel"),
+               "rbf_gemm": ("list_kernel", "residue_gemm_kernel", "crt_kernel", "listed_thin_kernel", "listed_gemm_kernel"),
                "spread_brick": "spread_brick_kernel", "spread_tile": "tile_spread_kernel",
                "spread_merge": "tile_merge_kernel", "interp": "interp_kernel", "advection": "advection_kernel",
                "momentum_rhs": "momentum_rhs_kernel", "residual_update": "residual_update_kernel",

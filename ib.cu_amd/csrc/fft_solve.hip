@@ -14,8 +14,9 @@
 // 94-108).  The solve is: real-to-half-complex FFT along x, complex FFT
 // along z, one tridiagonal solve per mode (chunks of rows in registers), and
 // the inverse transforms -- the exact solution of the same discrete system the
-// multigrid iterates on.  The transforms of a y-plane are one memory pass where
-// the plane fits the LDS (three passes per solve) and two elsewhere (five).  The singular case (sigma = 0 with
+// multigrid iterates on.  The transforms of a y-plane are one memory pass in
+// LDS where both point counts are 32 to 128 (three passes per solve) and two
+// elsewhere (five).  The singular case (sigma = 0 with
 // Neumann walls: the pressure Poisson) solves the mean-free problem, as the
 // multigrid does: the (0, 0) mode's right-hand side loses its mean, its last
 // unknown is pinned and the solution's mean is removed.
@@ -686,7 +687,8 @@ static ibm_status fft_alloc(ibm_ctx* ctx, ibm_fft* p, size_t bytes, void** out)
 }
 
 // The plane kernels of nx x nz points, or null where the sizes are not among
-// theirs (32 to 128: a larger plane does not fit the LDS).
+// theirs: 32 to 128 each.  (256 x 32, 256 x 64, 512 x 32 and their transposes
+// would fit the LDS too; they take the five passes.)
 struct plane_kernels {
     void (*forward)(int, const double*, double2*, const double2*, const double2*);
     void (*inverse)(int, const double2*, double*, double, const double2*, const double2*);

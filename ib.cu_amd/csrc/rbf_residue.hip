@@ -387,10 +387,10 @@ __global__ __launch_bounds__(256) void column_split_kernel(column_set set, int k
 // they lie in memory (1 KB each, read conflict-free) by direct-to-LDS loads
 // into three buffers, two 64-element chunks ahead of the one multiplied, one
 // barrier a chunk.  Units (tile, modulus) rather than whole tiles keep the
-// last wave of blocks short.  Measured for 8832 x 2210 x 600 (16 moduli):
-// 0.219 ms; four waves of 64 x 128 0.228, 128 x 128 tiles 0.237, 256 x 256
-// tiles 0.289 (padding of the 600 columns), 32 x 32 x 32 instructions with
-// two buffers 0.232.
+// last wave of blocks short.  One operator 8832 x 2210 x 600 takes 0.19 ms (a
+// sixth of six); relative to that, four waves of 64 x 128 1.04, 128 x 128
+// tiles 1.08, 256 x 256 tiles 1.32 (padding of the 600 columns), 32 x 32 x 32
+// instructions with two buffers 1.06.
 // ----------------------------------------------------------------------
 constexpr int WM = 4, WN = 2, FM = 4, FN = 4;          // waves and fragments per wave
 constexpr int WAVES = WM * WN, EF = WM * FM, XF = WN * FN, LOADS = (EF + XF) / WAVES;

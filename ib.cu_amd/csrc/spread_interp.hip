@@ -849,7 +849,7 @@ int blocks_for(long long n, int threads) { return (int) ((n + threads - 1) / thr
 struct bin_work {
     int *count, *start, *key, *rank, *perm, *code;
     long long* tmp;
-    double* sorted;          // 6 * total doubles: positions, then forces (SoA; per-marker records in the tile path)
+    double* sorted;          // 6 * total doubles: positions, then forces (SoA)
     bin_stats* stats;
     void* scan_tmp;
     size_t scan_bytes;
@@ -1948,9 +1948,6 @@ ibm_status spread_boxes(ibm_ctx* ctx, const ibm_grid* grids, int delta, const ma
     if (!whole_bricks(kg))
         return fail(ctx, IBM_ERR_BAD_GRID, "batched spreading needs periodic axes of a multiple of %d cells", TB);
     IBM_TRY(spread_setup(ctx, grids, delta, fe, &kg, &bd));
-    for (int c = 0; c < 3; ++c)
-        if (kg.points[c][0] > 65535 * 128)
-            return fail(ctx, IBM_ERR_SIZE, "grid rows of %d points too long for the tile spread", kg.points[c][0]);
     if (bricks_of(bd) * nboxes > (INT_MAX - 1) / SUB)
         return fail(ctx, IBM_ERR_SIZE, "too many boxes or bins for one batched spread");
     return spread_tiles(ctx, kg, bd, delta, sets, nboxes, box_off, fe, nullptr);

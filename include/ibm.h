@@ -127,7 +127,9 @@ typedef struct ibm_ctx ibm_ctx;
 
 /* Creates a context bound to a HIP device.  The context owns its scratch
  * workspaces (grown on demand) and uses the null stream until
- * ibm_set_stream() is called.  One context per host thread. */
+ * ibm_set_stream() is called.  One context per host thread.  The first context
+ * on a device also allocates the fixed workspace of ibm_spread_sets_noalloc
+ * (184 MB, held until the process ends). */
 ibm_status ibm_create(ibm_ctx** ctx, int device);
 ibm_status ibm_destroy(ibm_ctx* ctx);
 /* stream is a hipStream_t passed as void* (0 = null stream). */
