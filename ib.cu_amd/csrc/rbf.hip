@@ -14,10 +14,11 @@
 // each is packed once into "rows x Kp" tiles (k fastest, zero padded):
 // the operator at creation, X per call.  One launch covers every
 // (cell type, operator) pair.  Precisions:
-//   64  few columns on v_mfma_f64_16x16x4 (rbf_thin_kernel); more through
-//       residues on the INT8 matrix cores (rbf_residue.hip), but for the
-//       columns that residues do not hold as well and for operators without
-//       residue planes, which run on FP64 128 x 128 tiles;
+//   64  few columns and short contractions on v_mfma_f64_16x16x4
+//       (rbf_thin_kernel where few blocks do, else 128 x 128 tiles); the
+//       others through residues on the INT8 matrix cores (rbf_residue.hip),
+//       but for the columns that residues do not hold as well and for
+//       operators without residue planes;
 //   32  v_mfma_f32_16x16x4 on FP32 operands, FP32 accumulation;
 //   16  split BF16: a = a_hi + a_lo with a_hi = bf16(a), a_lo = bf16(a -
 //       a_hi); a b ~ a_hi b_hi + a_hi b_lo + a_lo b_hi with
@@ -668,24 +669,34 @@ int f64_variant(ibm_ctx* ctx, hipStream_t stream, const gemm_groups& G, int bloc
     return pick;
 }
 
-// Whether an FP64 evaluation of N columns runs in rbf_thin_kernel: up to 64
-// columns, where reading the operator bounds it, and further on while the
-// contraction is short and the product small, where the residue path's four
-// launches take longer than the thin kernel's one.  Otherwise it goes through
-// residues (rbf_residue.hip) if the operator has them.  Measured (us, thin /
-// residues): one operator 584 x 311, 128 columns 17 / 24, 600 columns 19 / 29;
-// six of 715 x 503, 192 columns 29 / 42, 256 columns 50 / 43; six of
-// 1552 x 605, 66 columns 60 / 47; three of 2843 x 935, 66 columns 81 / 54.
-// The rule looks at one operator's shape only: an entry's path (and so every
-// bit of its result) does not depend on what it is batched with.
-constexpr int THIN_K = 550;
-constexpr double THIN_WORK = 9e7;
-bool by_thin_kernel(const ibm_rbf* op, int N)
+// Whether an FP64 evaluation of N columns goes through residues
+// (rbf_residue.hip) if the operator has them.  Those cost about 40 us of
+// launches and 40 bytes an output beside the products, so short contractions
+// do not gain by them (K = 440: equal to the FP64 tiles' time; K = 120, 600
+// columns, six operators of 8832 rows 405 us against 166; K = 40 four times
+// the tiles'), nor do few columns, nor a single column tile of a large output
+// while K is middling (three operators 8832 x 560, 65 columns 94 us against
+// 81, 8832 x 700 111 / 98, 8832 x 900 133 / 130).  The rule looks at one
+// operator's shape only: an entry's path (and so every bit of its result)
+// does not depend on what it is batched with.
+constexpr int RESIDUE_N = 65, RESIDUE_K = 551, RESIDUE_ONE_TILE_K = 801;
+constexpr long RESIDUE_ONE_TILE_OUTPUTS = 500000;
+bool by_residues(const ibm_rbf* op, int N)
 {
-    return op->mode == MODE_F64 &&
-           (N <= THIN_COLUMNS || (op->K <= THIN_K && (double) op->M * op->K * N < THIN_WORK));
+    if (!op->res || N < RESIDUE_N || op->K < RESIDUE_K) return false;
+    return op->K >= RESIDUE_ONE_TILE_K || N > TILE || (long) op->M * N < RESIDUE_ONE_TILE_OUTPUTS;
 }
-bool by_residues(const ibm_rbf* op, int N) { return op->res && !by_thin_kernel(op, N); }
+
+// Whether a launch's FP64 products of more than 64 columns run in
+// rbf_thin_kernel too, in tiles of 64 columns, or in the FP64 tiles: there as
+// long as all blocks are resident at once (four per CU), which keeps more of
+// the chip busy than few long tiles; beyond, the tiles' greater reuse wins.
+// Thin / tiles, us: six operators of 715 x 503, 192 columns (414 blocks)
+// 29 / 74; of 1500 x 440, 192 columns (846) 46 / 67; of 4000 x 440, 65
+// columns (1500) 66 / 65; three of 8832 x 440, 65 columns (1656) 83 / 65.  Over
+// 1000 shapes of 1 to 6 operators none was slower than in tiles.  Both give
+// the same bits.
+constexpr long THIN_MOST_BLOCKS = 1024;
 
 // Offset of entry b's packed columns in the evaluation's packed operand and,
 // at b = count, its total; entries with the same columns share a packing
@@ -794,6 +805,11 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
         IBM_TRY(scratch(ctx, SLOT_RBF_WORK, res_work_bytes(nres, products), &work));
         flags = res_flags(nres, products, (unsigned char*) work, &nflags);
     }
+    long thin_blocks = 0;
+    for (int b = 0; b < count && mode == MODE_F64; ++b)
+        if (N[b] > THIN_COLUMNS && !by_residues(ops[b], N[b]))
+            thin_blocks += (long) ((ops[b]->M + THIN_ROWS - 1) / THIN_ROWS) * ((N[b] + THIN_COLUMNS - 1) / THIN_COLUMNS) *
+                           std::max(0, std::min(j1, ops[b]->nops) - j0);
     gemm_groups G{}, thin[4]{};        // thin[k]: rbf_thin_kernel's entries with tiles of 16 (k + 1) columns
     int tiles = 0, ncols = 0;
     res_columns cols[RES_MAX_COLUMNS];
@@ -815,7 +831,7 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
         int cols_pad = round_up(N[b], TILE);
         unsigned char* lo = planes(mode) > 1 ? hi + (size_t) cols_pad * op.Kp * elem_bytes(mode) : nullptr;
         if (do_pack && owner == b) pack(mode, stream, X[b], op.K, N[b], op.K, cols_pad, op.Kp, hi, lo);
-        const bool is_thin = by_thin_kernel(&op, N[b]);
+        const bool is_thin = mode == MODE_F64 && (N[b] <= THIN_COLUMNS || thin_blocks <= THIN_MOST_BLOCKS);
         for (int j = j0; j < std::min(j1, op.nops); ++j) {
             gemm_groups& to = is_thin ? thin[std::min(N[b] - 1, THIN_COLUMNS - 1) / 16] : G;
             gemm_group& g = to.g[to.count++];

@@ -402,11 +402,11 @@ ibm_status ibm_rbf_destroy(ibm_rbf* op);
  *
  * FP64: every output is within (K + 1) 2^-53 sum_k |E_k||X_k| of the exact
  * product (short of overflow and underflow), the bound of a chain of K fused
- * multiply-adds.  Entries of up to 64 columns, and of more while K <= 550 and
- * M K N < 9e7, run on the FP64 matrix cores; others through residues on the
- * INT8 matrix cores, but for the columns that those would not hold to that
- * bound (values of very different magnitude that matter to some output, NaN,
- * infinities), which run on the FP64 ones.  So the bits of an output depend on
+ * multiply-adds.  Entries of up to 64 columns or with K <= 550 (or with
+ * K <= 800, up to 128 columns and M N >= 500,000) run on the FP64 matrix cores;
+ * others through residues on the INT8 matrix cores, but for the columns that
+ * those would not hold to that bound (values of very different magnitude that
+ * matter to some output, NaN, infinities), which run on the FP64 ones.  So the bits of an output depend on
  * N (two entries of 64 columns need not agree in the last bits with one of
  * 128), but not on the other columns' values or on the other entries of the
  * batch. */
@@ -419,9 +419,9 @@ ibm_status ibm_rbf_eval(ibm_ctx* ctx, int count, ibm_rbf* const* ops, const int*
  * 64 x 32-output waves (half the registers, twice the waves per SIMD) over
  * two LDS buffers (one barrier per contraction chunk), 0 (the default) times
  * both on the first eager launch of each shape and keeps the faster for the
- * process.  Only products of more than 64 columns (or, with K <= 550, of
- * M K N >= 9e7) by operators without residue storage (see ibm_rbf_create)
- * take these kernels.  Every setting gives bitwise the same results.
+ * process.  Products of more than 64 columns take these kernels where they
+ * run on the FP64 matrix cores (see ibm_rbf_eval, ibm_rbf_create) and are many
+ * enough to fill the chip.  Every setting gives bitwise the same results.
  * Process-wide. */
 ibm_status ibm_rbf_gemm_variant(int waves_n);
 

@@ -57,11 +57,11 @@ def test_narrow_columns_at_tile_edges(ibm, ctx, shape):
     op.close()
 
 
-# both sides of the few-column kernel's limits on the work (9e7) and on the
-# contraction (550)
-@pytest.mark.parametrize("shape", [(700, 321, 400), (700, 321, 401), (300, 550, 70), (300, 551, 70)],
-                         ids=lambda s: "x".join(map(str, s)))
-def test_limits_of_the_few_column_kernel(ibm, ctx, shape):
+# both sides of the rule between residues and FP64 products: columns (64),
+# contraction (550; 800 where one column tile has many outputs), outputs
+@pytest.mark.parametrize("shape", [(300, 600, 64), (300, 600, 65), (300, 550, 70), (300, 551, 70), (3907, 800, 128),
+                                   (3907, 801, 128), (3906, 800, 128), (3907, 800, 129)], ids=lambda s: "x".join(map(str, s)))
+def test_limits_of_the_residue_path(ibm, ctx, shape):
     M, K, N = shape
     rng = np.random.default_rng(N)
     E, x = rng.standard_normal((M, K)), _narrow(rng, N, K)
@@ -69,6 +69,27 @@ def test_limits_of_the_few_column_kernel(ibm, ctx, shape):
     (Y,) = ibm.rbf_eval(ctx, [op], [_t(x)])
     _check(E, x, Y.cpu().numpy()[0])
     op.close()
+
+
+# FP64 products of more than 64 columns on both sides of 1024 blocks of 32 x 64
+# outputs: the few-column kernel and the tiles, in equal bits
+@pytest.mark.parametrize("N", [65, 128, 129])
+def test_few_column_kernel_and_tiles_give_the_same_bits(ibm, ctx, N):
+    M, K = 7000, 90
+    rng = np.random.default_rng(N)
+    mats = [rng.standard_normal((M, K)) for _ in range(3)]
+    x = rng.standard_normal((N, K))
+    xd = _t(x)
+    op = ibm.RbfOperator(ctx, "f64", [_t(m) for m in mats], K)      # 1314 or 1971 blocks
+    (Y,) = ibm.rbf_eval(ctx, [op], [xd])
+    Y = Y.cpu().numpy()
+    op.close()
+    for j, E in enumerate(mats):
+        _check(E, x, Y[j])
+        one = ibm.RbfOperator(ctx, "f64", [_t(E)], K)                # 438 or 657
+        (Z,) = ibm.rbf_eval(ctx, [one], [xd])
+        assert np.array_equal(Z.cpu().numpy()[0], Y[j])
+        one.close()
 
 
 def _one_hot(rng, M, K):

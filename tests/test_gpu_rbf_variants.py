@@ -1,6 +1,7 @@
-"""The FP64 tile kernels of ibm_rbf_gemm_variant on the products that they
-still take: operators with a non-finite row keep no residue planes, and all
-their evaluations of more than 64 columns run on the FP64 tiles."""
+"""The FP64 tile kernels of ibm_rbf_gemm_variant on products that they take:
+more than 64 columns, too many blocks for the few-column kernel, and a short
+contraction or an operator that keeps no residue planes (with a non-finite
+row)."""
 import numpy as np
 import pytest
 
@@ -16,9 +17,9 @@ def _t(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
-# one tile, partial tiles in every direction, whole ones; K > 550 (else the
-# few-column kernel takes them)
-@pytest.mark.parametrize("shape", [(5, 551, 65), (129, 577, 129), (256, 640, 128), (1000, 705, 300)],
+# partial tiles in every direction, whole ones; more than 1024 blocks of 32 x 64
+# outputs over the two operators
+@pytest.mark.parametrize("shape", [(16385, 33, 65), (8705, 577, 128), (8321, 64, 129), (5505, 40, 300)],
                          ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
 def test_variants_agree_bitwise_and_match_the_oracle(ibm, ctx, shape, bad):
