@@ -1069,8 +1069,10 @@ __global__ void __launch_bounds__(256) tile_clear_kernel(int* __restrict__ count
 // finds its few distinct bins by ballots and takes each one's ranks with one
 // atomic.  2.39 M markers: 134 us with single-cell bins (a wavefront meets
 // twenty or more), 102 with 4 x 4 x 4-cell bins, 58 with four markers a
-// thread.
-constexpr int COUNT_ITEMS = 4;
+// thread.  Scattered markers share no bins: a round of ballots for each of a
+// wavefront's 256 would be a chain of 33 us (2000 markers; 13 so), so only the
+// first COUNT_GROUPS bins of 64 markers are found that way.
+constexpr int COUNT_ITEMS = 4, COUNT_GROUPS = 24;
 
 __global__ void __launch_bounds__(256)
 tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const int* __restrict__ box_off,
@@ -1086,6 +1088,7 @@ tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const i
         load_force(sets, m, f[i]);
     }
     unsigned long long fbits = 0;
+    int groups = COUNT_GROUPS;
     int bin[COUNT_ITEMS], leader[COUNT_ITEMS], before[COUNT_ITEMS], base[COUNT_ITEMS];
 #pragma unroll
     for (int i = 0; i < COUNT_ITEMS; ++i) {
@@ -1117,13 +1120,14 @@ tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const i
             const unsigned long long bits = (unsigned long long) __double_as_longlong(a);
             fbits = bits > fbits ? bits : fbits;
         }
-        // ranks inside a bin, one atomic per group of lanes sharing a bin
+        // ranks inside a bin, one atomic per group of lanes sharing a bin;
+        // lanes beyond the first bins take theirs alone
         const unsigned long long lt = (1ull << lane) - 1;
         unsigned long long todo = __ballot(valid);
         int size = 0;
         leader[i] = lane;
         before[i] = 0;
-        while (todo) {
+        for (int group = 0; todo && group < groups; ++group) {
             const int l = __ffsll((long long) todo) - 1;
             const int lbin = __shfl(bin[i], l, 64);
             const unsigned long long grp = __ballot(valid && bin[i] == lbin) & todo;
@@ -1134,6 +1138,8 @@ tile_count_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, const i
             if (lane == l) size = __popcll(grp);
             todo &= ~grp;
         }
+        if (todo >> lane & 1) size = 1;
+        if (todo) groups = 2;                                // scattered markers: the next are, too
         base[i] = 0;
         if (valid && leader[i] == lane) base[i] = atomicAdd(&count[bin[i]], size);
     }
