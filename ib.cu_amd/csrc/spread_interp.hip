@@ -18,6 +18,8 @@
 //     do are spread owner-computes: one workgroup per 8x8x8 brick of grid
 //     points gathers the (canonically ordered) markers of the bins whose
 //     stencils reach the brick into an LDS tile of the same integers;
+//   * few scattered markers on a large grid are gathered by the bricks of points
+//     (the same integers, no tiles in memory);
 //   * interpolation is two lanes per marker and component, each with half of
 //     every row of the separable sum sum_z wz sum_y wy sum_x wx u.
 #include <hip/hip_runtime.h>
@@ -1167,13 +1169,16 @@ tile_place_kernel(int total, const int* __restrict__ key, const int* __restrict_
 // three where the last bin of a periodic axis is partial), and |sum| <= reach
 // max_count max|f| max_c res3_c phi^3, phi the delta kernel's maximum.  A
 // non-finite bound marks the result as poisoned (all NaN).
+//
+// It also decides whether tile_gather_kernel takes the spread: where no bin
+// holds more than gather_most markers (0: never).
 struct tile_scale {
     double inv_q, q;
-    int poisoned, pad;
+    int poisoned, gather;
 };
 
-__device__ inline void make_scale(const kgrids& g, int delta, int reach, unsigned long long max_f, unsigned long long max_count,
-                                  tile_scale* out)
+__device__ inline void make_scale(const kgrids& g, int delta, int reach, int gather_most, unsigned long long max_f,
+                                  unsigned long long max_count, tile_scale* out)
 {
     const double phi3 = delta == IBM_DELTA_BSPLINE3 ? 0.3 : 0.126;     // (2/3)^3, (1/2)^3 with room for rounding
     const double res3 = fmax(g.res3[0], fmax(g.res3[1], g.res3[2]));
@@ -1185,16 +1190,17 @@ __device__ inline void make_scale(const kgrids& g, int delta, int reach, unsigne
     if (!s.poisoned && bound > 0) frexp(bound, &e2);
     s.inv_q = ldexp(1.0, 62 - e2);
     s.q = s.poisoned ? __longlong_as_double(0x7ff8000000000000ll) : ldexp(1.0, e2 - 62);
-    s.pad = 0;
+    s.gather = gather_most > 0 && max_count <= (unsigned long long) gather_most;
     *out = s;
 }
 
-__global__ void tile_scale_kernel(kgrids g, int delta, int reach, const bin_stats* __restrict__ stats, tile_scale* __restrict__ out)
+__global__ void tile_scale_kernel(kgrids g, int delta, int reach, int gather_most, const bin_stats* __restrict__ stats,
+                                  tile_scale* __restrict__ out)
 {
     const int tid = threadIdx.x;      // one wavefront
     unsigned long long fb = wave_max(stats->max_abs_f[tid]);
     unsigned long long cm = wave_max(stats->max_count[tid]);
-    if (tid == 0) make_scale(g, delta, reach, fb, cm, out);
+    if (tid == 0) make_scale(g, delta, reach, gather_most, fb, cm, out);
 }
 
 __global__ void __launch_bounds__(256) tile_max_kernel(const int* __restrict__ count, int keys, bin_stats* __restrict__ stats)
@@ -1220,7 +1226,7 @@ __device__ inline int4 load_counts(const int* __restrict__ count, int i, int end
 }
 
 __global__ void __launch_bounds__(SCAN_THREADS)
-tile_scan_kernel(kgrids g, int delta, int reach, const int* __restrict__ count, int keys, const bin_stats* __restrict__ stats,
+tile_scan_kernel(kgrids g, int delta, int reach, int gather_most, const int* __restrict__ count, int keys, const bin_stats* __restrict__ stats,
                  int* __restrict__ start, tile_scale* __restrict__ out)
 {
     __shared__ int wave_sum[SCAN_WAVES];
@@ -1271,7 +1277,7 @@ tile_scan_kernel(kgrids g, int delta, int reach, const int* __restrict__ count, 
     if (wave == 0) {
         const unsigned long long fb = wave_max(stats->max_abs_f[lane]);
         const unsigned long long cm = wave_max((unsigned long long) (lane < SCAN_WAVES ? wave_top[lane] : 0));
-        if (lane == 0) make_scale(g, delta, reach, fb, cm, out);
+        if (lane == 0) make_scale(g, delta, reach, gather_most, fb, cm, out);
     }
 }
 
@@ -1343,7 +1349,7 @@ constexpr int CHUNK_MARKERS = 512, ORIGINS = 9 * 9 * 9, THREAD_MARKERS = CHUNK_M
 __global__ void __launch_bounds__(TILE_THREADS, 4)
 tile_spread_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, int delta, const int* __restrict__ start,
                    const int* __restrict__ perm, const tile_scale* __restrict__ scale,
-                   unsigned long long* __restrict__ tiles, int* __restrict__ flags, int blocks, int chunk)
+                   unsigned long long* __restrict__ tiles, int* __restrict__ flags, int blocks, int chunk, int may_gather)
 {
     __shared__ __attribute__((aligned(16))) unsigned long long acc[TILE_PTS];
     __shared__ __attribute__((aligned(16))) double2 offsets01[CHUNK_MARKERS], offset2_force[CHUNK_MARKERS];
@@ -1358,6 +1364,7 @@ tile_spread_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, int de
     const int s0 = start[(size_t) brick * SUB];
     const int s1 = start[(size_t) (brick + 1) * SUB];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (may_gather && scale->gather) return;
     if (s1 == s0) {
         if (tid == 0 && c == 0) flags[brick] = 0;
         return;                                      // whole block
@@ -1498,8 +1505,9 @@ __global__ void __launch_bounds__(MERGE_THREADS)
 tile_merge_kernel(kgrids g, bin_desc bd, tile_desc td, int box0, unsigned chunk,
                   const unsigned long long* __restrict__ tiles, const int* __restrict__ flags,
                   const tile_scale* __restrict__ scale, double* __restrict__ fe0, double* __restrict__ fe1,
-                  double* __restrict__ fe2)
+                  double* __restrict__ fe2, int may_gather)
 {
+    if (may_gather && scale->gather) return;
     const int bz = blockIdx.y / 3, c = blockIdx.y - 3 * bz, box = box0 + bz;
     const unsigned block = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
     const unsigned at = block * MERGE_THREADS + threadIdx.x;
@@ -1565,6 +1573,183 @@ tile_merge_kernel(kgrids g, bin_desc bd, tile_desc td, int box0, unsigned chunk,
     }
     double* fe = c == 0 ? fe0 : (c == 1 ? fe1 : fe2);
     fe[(size_t) box * td.box_points[c] + at] = (double) sum * scale->q;
+}
+
+// Few scattered markers on a large grid: every brick would hold a marker or
+// some, and its tiles of 12^3 points be cleared, stored and merged for them.
+// Instead one workgroup per 8 x 8 x 8 points visits the markers of the bins
+// that reach them, adds what falls on them to an LDS tile and writes the
+// points: the same integers, so the same bits, without tiles in memory.  A
+// marker is visited by eight workgroups, so bins must hold few (GATHER_MOST,
+// looked at on the device when the bins are counted: clumped markers keep the
+// tiles; the launches of the path not taken leave at once), and the kernel is
+// launched where the grid has GATHER_BRICKS bricks (fewer are bound by their
+// launches) and on average at most GATHER_PER_BRICK markers a brick.  Bound by
+// the latency of its chain of loads and by writing the grids.  Scattered
+// markers, whole spread, us, brick kernel / tiles / this: 20,000 on
+// 128 x 256 x 128 244 / 376 / 193, 200,000 on 256^3 1031 / 1489 / 737, 20,000
+// on 100^3 (9 a brick) 121 / 155 / 97, 2000 on 64^3 50 / 55 / 44; above the
+// limit 20,000 on 64^3 (39 a brick) 63 / 57 / 101, 200,000 on 128^3 (49)
+// 278 / 224 / 383.
+constexpr int GATHER_MOST = 24, GATHER_BRICKS = 100, GATHER_PER_BRICK = 12;
+constexpr int GATHER_AXIS = 8, GATHER_THREADS = 256, GATHER_CHUNK = 128, GATHER_ENTRIES = 3 * GATHER_CHUNK;
+
+__global__ void __launch_bounds__(GATHER_THREADS, 4)
+tile_gather_kernel(marker_sets sets, kgrids g, bin_desc bd, tile_desc td, int delta, const int* __restrict__ start,
+                   const int* __restrict__ perm, const tile_scale* __restrict__ scale, double* __restrict__ fe0,
+                   double* __restrict__ fe1, double* __restrict__ fe2, int bricks_x, int bricks_y, int nbricks, int chunk)
+{
+    __shared__ unsigned long long acc[3][BRICK_PTS];
+    __shared__ __attribute__((aligned(16))) double2 offsets01[GATHER_ENTRIES], offset2_force[GATHER_ENTRIES];
+    __shared__ int bases[3][GATHER_ENTRIES];
+    __shared__ unsigned char component[GATHER_ENTRIES];
+    __shared__ int axis_bin[3][GATHER_AXIS], axis_bins[3], entries;
+    __shared__ int first[GATHER_THREADS], before[GATHER_THREADS + 1], wave_sum[GATHER_THREADS / 64];
+    // XCD x takes the x-th eighth: neighbouring bricks share its L2's markers
+    const int bid = (int) (blockIdx.x & 7) * chunk + (int) (blockIdx.x >> 3);
+    if ((int) (blockIdx.x >> 3) >= chunk || bid >= nbricks || !scale->gather) return;       // whole block
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int P0x = bid % bricks_x * BX, P0y = bid / bricks_x % bricks_y * BY, P0z = bid / (bricks_x * bricks_y) * BZ;
+    // per axis, the bins of four cells that hold any of the (up to 12) cells
+    // whose stencils reach the brick, each once
+    if (tid < 3) {
+        const int j = tid;
+        const region_dim r = brick_region<BX>(bd, g.a[bd.fc[j]][j], j, j == 0 ? P0x : (j == 1 ? P0y : P0z));
+        int n = 0;
+        for (int i = 0; i < r.count;) {
+            int q = r.first + i;
+            if (r.wrap) q = q < 0 ? q + r.wrap : (q >= r.wrap ? q - r.wrap : q);
+            const int end = r.wrap && q + 4 - (q & 3) > r.wrap ? r.wrap : q + 4 - (q & 3);
+            if (n == 0 || q >> 2 != axis_bin[j][0]) axis_bin[j][n++] = q >> 2;
+            i += end - q;
+        }
+        axis_bins[j] = n;
+    }
+    __syncthreads();
+    const int nx = axis_bins[0], ny = axis_bins[1], bins = nx * ny * axis_bins[2];     // at most 6 per axis
+    // the bins' markers, flattened
+    int own = 0;
+    if (tid < bins) {
+        const int cx = axis_bin[0][tid % nx], cy = axis_bin[1][tid / nx % ny], cz = axis_bin[2][tid / (nx * ny)];
+        const int key = (((cz >> 1) * td.nbr[1] + (cy >> 1)) * td.nbr[0] + (cx >> 1)) * SUB + ((cx & 1) | (cy & 1) << 1 | (cz & 1) << 2);
+        first[tid] = start[key];
+        own = start[key + 1] - first[tid];
+    }
+    int incl = own;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += y;
+    }
+    if (lane == 63) wave_sum[wave] = incl;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) incl += wave_sum[w];
+    before[tid + 1] = incl;
+    if (tid == 0) before[0] = 0;
+    int T = 0;
+    for (int w = 0; w < GATHER_THREADS / 64; ++w) T += wave_sum[w];
+    if (T > 0) {
+        for (int i = tid; i < 3 * BRICK_PTS; i += GATHER_THREADS) (&acc[0][0])[i] = 0ull;
+        const double inv_q = scale->inv_q;
+        const double fast_below = 0x1p51 / (delta == IBM_DELTA_BSPLINE3 ? 0.3 : 0.126);
+        for (int c0 = 0; c0 < T; c0 += GATHER_CHUNK) {
+            if (tid == 0) entries = 0;
+            __syncthreads();
+            // a thread per marker: its components whose stencils meet the brick
+            const int at = c0 + tid;
+            if (tid < GATHER_CHUNK && at < T) {
+                int lo = 0, hi = GATHER_THREADS;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (before[mid] <= at) lo = mid; else hi = mid;
+                }
+                const int m = perm[first[lo] + (at - before[lo])];
+                double p[3], f[3];
+                load_marker(sets, m, p);
+                load_force(sets, m, f);
+                int q[3], qb[3];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    q[j] = kstencil(g.a[bd.fc[j]][j], p[j]).base + bd.fs[j];
+                    const int b = q[j] - bd.qmin[j];
+                    qb[j] = b < 0 ? 0 : (b >= bd.nb[j] ? bd.nb[j] - 1 : b);
+                }
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    double d[3];
+                    int base[3];
+                    bool hit = true;
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) {
+                        const kaxis& a = g.a[c][j];
+                        const stencil_axis st = kstencil(a, p[j]);
+                        d[j] = st.d;
+                        base[j] = st.base;
+                        int s = st.base - q[j];
+                        if (!a.solid) {
+                            if (s > 2) s -= a.cells;
+                            else if (s < -3) s += a.cells;
+                        }
+                        const int o = (qb[j] & (TB - 1)) + s - bd.lo[j];
+                        bool any = false;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            any = any || brick_offset<BX>(a, st.base, k, j == 0 ? P0x : (j == 1 ? P0y : P0z)) >= 0;
+                        hit = hit && any && o >= 0 && o <= TT - 4;           // o: as in tile_spread_kernel
+                    }
+                    if (hit) {
+                        const int e = atomicAdd(&entries, 1);
+                        offsets01[e] = make_double2(d[0], d[1]);
+                        offset2_force[e] = make_double2(d[2], f[c] * g.res3[c] * inv_q);
+#pragma unroll
+                        for (int j = 0; j < 3; ++j) bases[j][e] = base[j];
+                        component[e] = (unsigned char) c;
+                    }
+                }
+            }
+            __syncthreads();
+            // four lanes per component of a marker, one plane of its stencil each
+            for (int i = tid; i < 4 * entries; i += GATHER_THREADS) {
+                const int e = i >> 2, sz = i & 3, c = component[e];
+                const int oz = brick_offset<BZ>(g.a[c][2], bases[2][e], sz, P0z);
+                if (oz < 0) continue;
+                int ox[4], oy[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    ox[k] = brick_offset<BX>(g.a[c][0], bases[0][e], k, P0x);
+                    oy[k] = brick_offset<BY>(g.a[c][1], bases[1][e], k, P0y);
+                }
+                const double2 d01 = offsets01[e], d2f = offset2_force[e];
+                double wx[4], wy[4], wz[4];
+                delta4(delta, d01.x, wx);
+                delta4(delta, d01.y, wy);
+                delta4(delta, d2f.x, wz);
+                const double z = sz == 0 ? wz[0] : (sz == 1 ? wz[1] : (sz == 2 ? wz[2] : wz[3]));
+                const bool fast = fabs(d2f.y) < fast_below;
+#pragma unroll
+                for (int sy = 0; sy < 4; ++sy) {
+                    if (oy[sy] < 0) continue;
+                    const double wyz = z * (wy[sy] * d2f.y);
+                    unsigned long long* row = &acc[c][BX * (oy[sy] + BY * oz)];
+#pragma unroll
+                    for (int sx = 0; sx < 4; ++sx) {
+                        if (ox[sx] < 0) continue;
+                        if (fast) add_value<true>(row + ox[sx], wx[sx], wyz);
+                        else add_value<false>(row + ox[sx], wx[sx], wyz);
+                    }
+                }
+            }
+            __syncthreads();
+        }
+    }
+    const double q = scale->q;
+    for (int i = tid; i < 3 * BRICK_PTS; i += GATHER_THREADS) {
+        const int c = i / BRICK_PTS, k = i - c * BRICK_PTS;
+        const int X = P0x + k % BX, Y = P0y + k / BX % BY, Z = P0z + k / (BX * BY);
+        const int* pt = g.points[c];
+        double* fe = c == 0 ? fe0 : (c == 1 ? fe1 : fe2);
+        if (X < pt[0] && Y < pt[1] && Z < pt[2])
+            fe[(size_t) X + (size_t) pt[0] * ((size_t) Y + (size_t) pt[1] * Z)] = T > 0 ? (double) (long long) acc[c][k] * q : 0.0 * q;
+    }
 }
 
 // Two doubles at 8-byte alignment (global loads need only dword alignment).
@@ -1839,6 +2024,8 @@ ibm_status spread_tiles(ibm_ctx* ctx, const kgrids& kg, const bin_desc& bd, int 
         }
     }
     const bool timed = fixed_workspace == nullptr;
+    const bool may_gather = nboxes == 1 && td.bricks >= GATHER_BRICKS && (long long) sets.total <= (long long) GATHER_PER_BRICK * td.bricks;
+    const int gather_most = may_gather ? GATHER_MOST : 0;
     {
         prof_scope prof(ctx, timed ? "bin" : nullptr);
         tile_clear_kernel<<<blocks_for((long long) td.keys + 1, 256), 256, 0, ctx->stream>>>(count, td.keys, stats);
@@ -1849,13 +2036,13 @@ ibm_status spread_tiles(ibm_ctx* ctx, const kgrids& kg, const bin_desc& bd, int 
             IBM_LAUNCH_CHECK(ctx);
         }
         if (td.keys <= SCAN_MAX) {
-            tile_scan_kernel<<<1, SCAN_THREADS, 0, ctx->stream>>>(kg, delta, reach, count, td.keys, stats, start, sc);
+            tile_scan_kernel<<<1, SCAN_THREADS, 0, ctx->stream>>>(kg, delta, reach, gather_most, count, td.keys, stats, start, sc);
             IBM_LAUNCH_CHECK(ctx);
         } else {
             IBM_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(scan_tmp, scan_bytes, count, start, td.keys + 1, ctx->stream));
             tile_max_kernel<<<std::min(blocks_for(td.keys, 256), 1024), 256, 0, ctx->stream>>>(count, td.keys, stats);
             IBM_LAUNCH_CHECK(ctx);
-            tile_scale_kernel<<<1, 64, 0, ctx->stream>>>(kg, delta, reach, stats, sc);
+            tile_scale_kernel<<<1, 64, 0, ctx->stream>>>(kg, delta, reach, gather_most, stats, sc);
             IBM_LAUNCH_CHECK(ctx);
         }
         if (total > 0) {
@@ -1867,11 +2054,20 @@ ibm_status spread_tiles(ibm_ctx* ctx, const kgrids& kg, const bin_desc& bd, int 
         prof_scope prof(ctx, timed ? "spread_tile" : nullptr, 48.0 * sets.total);
         const int blocks = (int) nbricks * 3, chunk = (blocks + 7) / 8;
         tile_spread_kernel<<<(unsigned) (8 * chunk), TILE_THREADS, 0, ctx->stream>>>(sets, kg, bd, td, delta, start, perm, sc,
-                                                                                     tiles, flags, blocks, chunk);
+                                                                                     tiles, flags, blocks, chunk, may_gather);
         IBM_LAUNCH_CHECK(ctx);
     }
     {
         prof_scope prof(ctx, timed ? "spread_merge" : nullptr, 8.0 * grid_points);
+        if (may_gather) {
+            int bricks[3] = {0, 0, 0};
+            for (int c = 0; c < 3; ++c)
+                for (int j = 0; j < 3; ++j) bricks[j] = std::max(bricks[j], (kg.points[c][j] + BX - 1) / BX);
+            const int n = bricks[0] * bricks[1] * bricks[2], chunk = (n + 7) / 8;
+            tile_gather_kernel<<<(unsigned) (8 * chunk), GATHER_THREADS, 0, ctx->stream>>>(
+                sets, kg, bd, td, delta, start, perm, sc, fe[0], fe[1], fe[2], bricks[0], bricks[1], n, chunk);
+            IBM_LAUNCH_CHECK(ctx);
+        }
         bool whole = true;
         for (int c = 0; c < 3; ++c)
             for (int j = 0; j < 3; ++j) whole = whole && (kg.a[c][j].solid || kg.a[c][j].cells % TB == 0);
@@ -1882,10 +2078,10 @@ ibm_status spread_tiles(ibm_ctx* ctx, const kgrids& kg, const bin_desc& bd, int 
             const dim3 grid(8 * chunk, (unsigned) (3 * nb));
             if (whole)
                 tile_merge_kernel<true><<<grid, MERGE_THREADS, 0, ctx->stream>>>(kg, bd, td, b0, chunk, tiles, flags, sc,
-                                                                                 fe[0], fe[1], fe[2]);
+                                                                                 fe[0], fe[1], fe[2], may_gather);
             else
                 tile_merge_kernel<false><<<grid, MERGE_THREADS, 0, ctx->stream>>>(kg, bd, td, b0, chunk, tiles, flags, sc,
-                                                                                  fe[0], fe[1], fe[2]);
+                                                                                  fe[0], fe[1], fe[2], may_gather);
             IBM_LAUNCH_CHECK(ctx);
         }
     }
