@@ -40,6 +40,7 @@ constexpr int ZT = 8;              // kx columns per z-transform block
 constexpr int MAX_FFT_POINTS = 512;
 constexpr int MAX_WALL_POINTS = 800;
 constexpr int LINE_THREADS = 256, LINE_MODES = 8, LINE_CHUNKS = LINE_THREADS / LINE_MODES;
+constexpr int SHORT_ROWS = 8, SHORT_MODES = 64;      // lines of up to SHORT_ROWS rows: fewer chunks, more modes a block
 constexpr size_t MAX_DYNAMIC_LDS = 160 * 1024;
 
 // Row stride of the half-spectrum in coefficients: nh rounded up to 8 (rows
@@ -470,43 +471,45 @@ __device__ inline void tri_row(const wall_axis& y, double sigma, double tau, dou
     diag = id * (sigma + tau * mu) + ty * d;
 }
 
-// Sum over a workgroup's LINE_CHUNKS chunks of the lanes with t = 0.
+// Sum over a workgroup's chunks of the lanes with t = 0.
+template <int MODES>
 __device__ inline double2 line_sum(double2 v, double2* part)
 {
     __syncthreads();
-    if (threadIdx.x % LINE_MODES == 0) part[threadIdx.x / LINE_MODES] = v;
+    if (threadIdx.x % MODES == 0) part[threadIdx.x / MODES] = v;
     __syncthreads();
     double2 m = make_double2(0.0, 0.0);
-    for (int i = 0; i < LINE_CHUNKS; ++i) {
+    for (int i = 0; i < LINE_THREADS / MODES; ++i) {
         m.x += part[i].x;
         m.y += part[i].y;
     }
     return m;
 }
 
-// Every Fourier mode's tridiagonal system along y: block (tile of LINE_MODES
-// kx, kz), one thread per mode and chunk of M consecutive rows, which it keeps
+// Every Fourier mode's tridiagonal system along y: block (tile of MODES kx,
+// kz), one thread per mode and chunk of M consecutive rows, which it keeps
 // in registers (rows past ny are identity rows).  A forward elimination leaves
 // row r as X_r = d_r - c_r X_{r+1} - a_r X_{-1}, with X_{-1} the last row of
 // the chunk before, and a backward one gives the first row by the chunk's and
 // the previous chunk's last; put into the previous chunk's last row that is
-// one equation per chunk, solved by cyclic reduction over the LINE_CHUNKS of
-// them, and a back substitution ends it.  The singular mode's last equation is
+// one equation per chunk, solved by cyclic reduction over them, and a back substitution ends it.  The singular mode's last equation is
 // replaced by x = 0 after its right-hand side loses its mean, and its solution
 // loses its mean.  Bound by memory (16 bytes per row read and written, whole
 // 128-byte lines): cyclic reduction over all rows in LDS took two divisions
 // per row and step, eight in all, this one and a fraction.  65 x 256 x 128
-// coefficients: 48 us / 17.
-template <int M>
+// coefficients: 48 us / 17.  Few rows leave most chunks without any: a solve of
+// 256 x 2 x 256 points 37 us with 8 modes a block, 30 with 64.
+template <int M, int MODES = LINE_MODES>
 __global__ void __launch_bounds__(LINE_THREADS) line_kernel(int nh, wall_axis y, double sigma, double tau, int singular,
                                                             const double* __restrict__ lam_x,
                                                             const double* __restrict__ lam_z, double2* __restrict__ s)
 {
     __shared__ double2 D[2][LINE_THREADS];
     __shared__ double2 AC[2][LINE_THREADS];
-    __shared__ double2 part[LINE_CHUNKS];
-    const int ny = y.n, t = threadIdx.x % LINE_MODES, q = threadIdx.x / LINE_MODES;
-    const int kx = blockIdx.x * LINE_MODES + t, kz = blockIdx.y, j0 = q * M;
+    constexpr int CHUNKS = LINE_THREADS / MODES;
+    __shared__ double2 part[CHUNKS];
+    const int ny = y.n, t = threadIdx.x % MODES, q = threadIdx.x / MODES;
+    const int kx = blockIdx.x * MODES + t, kz = blockIdx.y, j0 = q * M;
     const int ld = spec_ld(nh);
     const bool pin_block = singular && blockIdx.x == 0 && kz == 0;     // holds the singular mode (t = 0)
     const bool pinned = pin_block && t == 0;
@@ -520,7 +523,7 @@ __global__ void __launch_bounds__(LINE_THREADS) line_kernel(int nh, wall_axis y,
         double2 own = make_double2(0.0, 0.0);
 #pragma unroll
         for (int r = 0; r < M; ++r) own = make_double2(own.x + d[r].x, own.y + d[r].y);
-        const double2 sum = line_sum(own, part);
+        const double2 sum = line_sum<MODES>(own, part);
         if (pinned) {
 #pragma unroll
             for (int r = 0; r < M; ++r)
@@ -565,8 +568,8 @@ __global__ void __launch_bounds__(LINE_THREADS) line_kernel(int nh, wall_axis y,
     __syncthreads();
     double ra = a[M - 1], rc = 0.0;
     double2 rd = d[M - 1];
-    if (q + 1 < LINE_CHUNKS) {
-        const double2 np = D[0][id + LINE_MODES], nfg = AC[0][id + LINE_MODES];
+    if (q + 1 < CHUNKS) {
+        const double2 np = D[0][id + MODES], nfg = AC[0][id + MODES];
         const double inv = 1.0 / (1.0 - c[M - 1] * nfg.x);
         ra *= inv;
         rc = -c[M - 1] * nfg.y * inv;
@@ -576,18 +579,18 @@ __global__ void __launch_bounds__(LINE_THREADS) line_kernel(int nh, wall_axis y,
     // cyclic reduction of X_q + ra X_{q-1} + rc X_{q+1} = rd
     int buf = 1;
 #pragma unroll
-    for (int sft = 1; sft < LINE_CHUNKS; sft <<= 1) {
+    for (int sft = 1; sft < CHUNKS; sft <<= 1) {
         D[buf][id] = rd;
         AC[buf][id] = make_double2(ra, rc);
         __syncthreads();
         double2 dm = make_double2(0.0, 0.0), dn = dm, am = dm, an = dm;
         if (q >= sft) {
-            dm = D[buf][id - sft * LINE_MODES];
-            am = AC[buf][id - sft * LINE_MODES];
+            dm = D[buf][id - sft * MODES];
+            am = AC[buf][id - sft * MODES];
         }
-        if (q + sft < LINE_CHUNKS) {
-            dn = D[buf][id + sft * LINE_MODES];
-            an = AC[buf][id + sft * LINE_MODES];
+        if (q + sft < CHUNKS) {
+            dn = D[buf][id + sft * MODES];
+            an = AC[buf][id + sft * MODES];
         }
         const double inv = 1.0 / (1.0 - ra * am.y - rc * an.x);
         rd = make_double2((rd.x - ra * dm.x - rc * dn.x) * inv, (rd.y - ra * dm.y - rc * dn.y) * inv);
@@ -597,7 +600,7 @@ __global__ void __launch_bounds__(LINE_THREADS) line_kernel(int nh, wall_axis y,
     }
     D[buf][id] = rd;
     __syncthreads();
-    const double2 before = q > 0 ? D[buf][id - LINE_MODES] : make_double2(0.0, 0.0);
+    const double2 before = q > 0 ? D[buf][id - MODES] : make_double2(0.0, 0.0);
     d[M - 1] = rd;
 #pragma unroll
     for (int r = M - 2; r >= 0; --r)
@@ -607,7 +610,7 @@ __global__ void __launch_bounds__(LINE_THREADS) line_kernel(int nh, wall_axis y,
 #pragma unroll
         for (int r = 0; r < M; ++r)
             if (j0 + r < ny) own = make_double2(own.x + d[r].x, own.y + d[r].y);
-        const double2 sum = line_sum(own, part);
+        const double2 sum = line_sum<MODES>(own, part);
         if (pinned) {
 #pragma unroll
             for (int r = 0; r < M; ++r) d[r] = make_double2(d[r].x - sum.x / ny, d[r].y - sum.y / ny);
@@ -763,11 +766,11 @@ ibm_status fft_solve(ibm_ctx* ctx, ibm_fft* p, double sigma, double tau, const d
         IBM_LAUNCH_CHECK(ctx);
     }
     const int singular = sigma == 0.0 && p->neumann;
-    const dim3 tgrid((p->nh + LINE_MODES - 1) / LINE_MODES, p->nz);
-    auto lines = [&](auto kernel) {
-        kernel<<<tgrid, LINE_THREADS, 0, ctx->stream>>>(p->nh, p->y, sigma, tau, singular, p->lam_x, p->lam_z, p->spec);
+    auto lines = [&](auto kernel, int modes = LINE_MODES) {
+        kernel<<<dim3((p->nh + modes - 1) / modes, p->nz), LINE_THREADS, 0, ctx->stream>>>(p->nh, p->y, sigma, tau, singular, p->lam_x, p->lam_z, p->spec);
     };
-    if (p->ny <= 2 * LINE_CHUNKS) lines(line_kernel<2>);
+    if (p->ny <= SHORT_ROWS) lines(line_kernel<2, SHORT_MODES>, SHORT_MODES);
+    else if (p->ny <= 2 * LINE_CHUNKS) lines(line_kernel<2>);
     else if (p->ny <= 4 * LINE_CHUNKS) lines(line_kernel<4>);
     else if (p->ny <= 8 * LINE_CHUNKS) lines(line_kernel<8>);
     else if (p->ny <= 16 * LINE_CHUNKS) lines(line_kernel<16>);
