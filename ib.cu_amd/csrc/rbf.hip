@@ -606,16 +606,21 @@ void launch_f64(int wn, const gemm_groups& G, int blocks, hipStream_t stream)
 // operators from 330 x 300 to 8832 x 2210, 3 to 1200 columns), and the large
 // ones run in rounds of 256: the smaller estimate is taken.  The multiply
 // sequence of an output is the same either way.
-constexpr int SMALL_TILE = 64;
+// FP32 contractions of a single chunk of 64 elements are bound by storing their
+// outputs, where the large tiles' longer runs are faster once there are many
+// (six operators 8832 x 40: 600 columns, 2070 tiles, 67 / 78; 1200 130 / 163).
+constexpr int SMALL_TILE = 64, SHORT_LARGE_TILES = 1536;
 bool small_tiles(int mode, const gemm_groups& G)
 {
-    if (mode == MODE_F32) return true;
     long large = 0, small = 0;
+    int kp = 0;
     for (int q = 0; q < G.count; ++q) {
         const gemm_group& g = G.g[q];
+        kp = std::max(kp, g.Kp);
         large += (long) ((g.M + TILE - 1) / TILE) * ((g.N + TILE - 1) / TILE);
         small += (long) ((g.M + SMALL_TILE - 1) / SMALL_TILE) * ((g.N + SMALL_TILE - 1) / SMALL_TILE);
     }
+    if (mode == MODE_F32) return kp > KPAD || large < SHORT_LARGE_TILES;
     return 0.38 * small < 256.0 * ((large + 255) / 256);
 }
 
@@ -899,7 +904,8 @@ ibm_status rbf_eval_range(ibm_ctx* ctx, hipStream_t stream, int count, ibm_rbf* 
     if (mode == MODE_F64) {
         launch_f64(wn, G, blocks, stream);
     } else if (mode == MODE_F32) {
-        rbf_gemm_kernel<MODE_F32, 2, ROWB, 2, SMALL_TILE><<<blocks, NTHREADS, 0, stream>>>(G);
+        if (edge == SMALL_TILE) rbf_gemm_kernel<MODE_F32, 2, ROWB, 2, SMALL_TILE><<<blocks, NTHREADS, 0, stream>>>(G);
+        else rbf_gemm_kernel<MODE_F32, 2><<<blocks, NTHREADS, 0, stream>>>(G);
     } else {
         if (edge == SMALL_TILE) rbf_gemm_kernel<MODE_BF16X3, 2, ROWB, 2, SMALL_TILE><<<blocks, NTHREADS, 0, stream>>>(G);
         else rbf_gemm_kernel<MODE_BF16X3, 2><<<blocks, NTHREADS, 0, stream>>>(G);
